@@ -146,21 +146,35 @@ QMX_DEV void block_sum(double (&v)[NV], double* red) {
 
 // Publish this block's NV partial values and detect the last block of state b.
 // Returns true (uniformly) in the block that arrives last; that block then
-// sees every block's partials.
+// reads every block's partials with load_partial.
+// The partials are stored at agent scope (written through to the point where
+// the XCDs' L2 caches agree), wave 0 waits until its stores are acknowledged,
+// and only then counts the block.  No __threadfence: a device-scope release
+// makes every wave that runs it write back its XCD's whole L2, and those
+// write-backs queue up; with one per wave of 8192 blocks the norm of 32 states
+// of 2^20 complex64 amplitudes took 905 us, against 126 us like this
+// (the overlap of 32 complex64 states with their references: 566 against 292).
 template <int NV>
 QMX_DEV bool publish_partial(const double* red, double* part, int* counter, int nblk,
                              int* s_flag) {
-  if (threadIdx.x < NV) part[(size_t)blockIdx.x * NV + threadIdx.x] = red[threadIdx.x];
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int prev = atomicAdd(counter, 1);
-    *s_flag = (prev == nblk - 1) ? 1 : 0;
+  static_assert(NV <= 64, "the partials are stored by wave 0");
+  if (threadIdx.x < 64) {
+    if (threadIdx.x < NV)
+      __hip_atomic_store(&part[(size_t)blockIdx.x * NV + threadIdx.x], red[threadIdx.x], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (threadIdx.x == 0) {
+      const int prev = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *s_flag = (prev == nblk - 1) ? 1 : 0;
+    }
   }
   __syncthreads();
-  bool last = *s_flag != 0;
-  if (last) __threadfence();
-  return last;
+  return *s_flag != 0;
+}
+
+// a partial value published by another block (past this XCD's caches)
+QMX_DEV double load_partial(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Sum the NV partial values of nblk blocks (pb[q * NV + j]) with the whole
@@ -175,13 +189,13 @@ QMX_DEV void reduce_partials(const double* pb, int nblk, double* scratch, double
   if (g0 < groups) {
     int q = g0;
     for (; q + 3 * groups < nblk; q += 4 * groups) {
-      double a0 = pb[(size_t)q * NV + j];
-      double a1 = pb[(size_t)(q + groups) * NV + j];
-      double a2 = pb[(size_t)(q + 2 * groups) * NV + j];
-      double a3 = pb[(size_t)(q + 3 * groups) * NV + j];
+      double a0 = load_partial(pb + (size_t)q * NV + j);
+      double a1 = load_partial(pb + (size_t)(q + groups) * NV + j);
+      double a2 = load_partial(pb + (size_t)(q + 2 * groups) * NV + j);
+      double a3 = load_partial(pb + (size_t)(q + 3 * groups) * NV + j);
       acc += ((a0 + a1) + (a2 + a3));
     }
-    for (; q < nblk; q += groups) acc += pb[(size_t)q * NV + j];
+    for (; q < nblk; q += groups) acc += load_partial(pb + (size_t)q * NV + j);
   }
   scratch[threadIdx.x] = acc;
   __syncthreads();
