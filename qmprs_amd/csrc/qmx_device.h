@@ -2,9 +2,9 @@
 //
 // Complex numbers are double2 (re, im) in registers and LDS; dense states are
 // stored either as float2 (complex64) or double2 (complex128) in HBM.
-// All small linear algebra here (4x4 Hermitian eigensolver, 4x4 polar factor,
-// Householder completion) runs serially in one lane in FP64: the matrices are
-// tiny and the results feed every later step, so accuracy wins over width.
+// All small linear algebra here is FP64: the matrices are tiny and the results
+// feed every later step.  The 4x4 Hermitian eigensolver and the Householder
+// completion run serially in one lane, the 4x4 polar factor on one wave.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -201,195 +201,354 @@ QMX_DEV int canonical_basis4(int k, const double2* v, double2* w, double tol) {
 }
 
 // ------------------------------------------------------- polar (d <= 4) ----
-// In-place inverse of a 4 x 4 complex matrix m by Gauss-Jordan elimination
-// with partial (row) pivoting: row swaps are recorded and undone as column
-// swaps at the end.  False when a pivot is zero or the result is not finite.
-// Compile-time indices only (swaps are selects).
-QMX_DEV bool inv4_inplace(double2* m) {
-  int perm[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    int p = k;
-    double best = cabs2(m[k * 4 + k]);
-#pragma unroll
-    for (int i = k + 1; i < 4; ++i) {
-      const double v = cabs2(m[i * 4 + k]);
-      if (v > best) {
-        best = v;
-        p = i;
-      }
-    }
-    if (!(best > 0.0)) return false;
-    perm[k] = p;
-#pragma unroll
-    for (int i = k + 1; i < 4; ++i) {
-      if (p == i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const double2 t = m[k * 4 + j];
-          m[k * 4 + j] = m[i * 4 + j];
-          m[i * 4 + j] = t;
-        }
-      }
-    }
-    const double ib = 1.0 / best;
-    const double2 ip = make_double2(m[k * 4 + k].x * ib, -m[k * 4 + k].y * ib);   // 1 / pivot
-    m[k * 4 + k] = make_double2(1.0, 0.0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) m[k * 4 + j] = cmul(m[k * 4 + j], ip);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (i != k) {
-        const double2 f = m[i * 4 + k];
-        m[i * 4 + k] = cz();
-#pragma unroll
-        for (int j = 0; j < 4; ++j) m[i * 4 + j] = csub(m[i * 4 + j], cmul(f, m[k * 4 + j]));
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 3; k >= 0; --k) {
-#pragma unroll
-    for (int c = k + 1; c < 4; ++c) {
-      if (perm[k] == c) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const double2 t = m[i * 4 + k];
-          m[i * 4 + k] = m[i * 4 + c];
-          m[i * 4 + c] = t;
-        }
-      }
-    }
-  }
-  double s = 0.0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) s += cabs2(m[i]);
-  return s < 1e300;   // false for inf / nan
+// ---- the polar factor on one wave ---------------------------------------------
+// A 4 x 4 matrix lives in 16 lanes, lane l = 4 i + j holding entry (i, j); the
+// wave's four rows of 16 lanes all hold the same matrix, so every branch below
+// is uniform over the wave.  Neighbours are read with DPP moves (row_ror by
+// multiples of 4 walks the matrix rows, quad_perm the columns), which cost
+// their issue slots only; a ds_bpermute would add an LDS round trip to a chain
+// that is bound by its latency.
+template <int CTRL>
+QMX_DEV double dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
 }
+template <int CTRL>
+QMX_DEV double2 dpp2(double2 v) { return make_double2(dpp<CTRL>(v.x), dpp<CTRL>(v.y)); }
+constexpr int kDppRow1 = 0x12c, kDppRow2 = 0x128, kDppRow3 = 0x124;   // matrix row (i + 1, 2, 3) % 4
+constexpr int kDppCol1 = 0x39, kDppCol2 = 0x4e, kDppCol3 = 0x93;      // matrix column (j + 1, 2, 3) % 4
+constexpr int kDppSwap = 0xb1;                                         // column j ^ 1
 
-// Unitary polar factor of a nonsingular 4 x 4 matrix by the scaled Newton
-// iteration (N. J. Higham, "Computing the polar decomposition -- with
-// applications", SIAM J. Sci. Stat. Comput. 7 (1986)), in place on u (which
-// holds the matrix on entry):
-//   X_0 = u,  X_{k+1} = (z X_k + X_k^{-H} / z) / 2,
-//   z = (||X_k^{-1}||_F / ||X_k||_F)^{1/2}  (z = 1 once ||X_{k+1} - X_k||_F < 1e-2),
-// which converges quadratically; it stops when ||X_{k+1} - X_k||_F <= 1e-8
-// (the last iterate is then accurate to rounding).  Returns false, with u
-// unspecified, when the matrix is ill-conditioned (||X_0||_F ||X_0^{-1}||_F >
-// 1e6), an inverse fails, or 40 iterations do not converge.
-QMX_DEV bool polar4_newton(double2* u) {
-  double2 xi[16];
-  bool scale = true;
-  for (int it = 0; it < 40; ++it) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) xi[i] = u[i];
-    if (!inv4_inplace(xi)) return false;
-    double nx = 0.0, ni = 0.0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      nx += cabs2(u[i]);
-      ni += cabs2(xi[i]);
-    }
-    if (it == 0 && nx * ni > 1e12) return false;
-    const double z = scale ? sqrt(sqrt(ni / nx)) : 1.0;
-    const double zi = 1.0 / z;
-    double dl = 0.0;
-    // X_{k+1}[i][j] = (z X[i][j] + conj(X^{-1}[j][i]) / z) / 2
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double2 a = u[i * 4 + j], b = xi[j * 4 + i];
-        const double2 v = make_double2(0.5 * (z * a.x + zi * b.x), 0.5 * (z * a.y - zi * b.y));
-        dl += cabs2(csub(v, a));
-        u[i * 4 + j] = v;
-      }
-    if (dl < 1e-4) scale = false;
-    if (dl <= 1e-16) return true;
-  }
-  return false;
-}
-
-// ---- the same Newton iteration on 16 lanes -----------------------------------
-// Lanes 0..15 of one wave (all active, the rest of the wave idle) hold one
-// entry each: lane l = 4 i + j holds X[i][j].  Cross-lane reads are __shfl
-// within the 16 lanes; sums are xor butterflies, in which both partners add
-// the same two values at every level, so every lane holds the bitwise same
-// sum and every branch below is uniform over the 16 lanes.
-QMX_DEV double2 shfl16(double2 v, int src) {
-  return make_double2(__shfl(v.x, src, 16), __shfl(v.y, src, 16));
-}
+// sum over the 16 lanes (both partners add the same two values at every
+// level, so every lane holds the bitwise same sum)
 QMX_DEV double sum16(double v) {
-#pragma unroll
-  for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 16);
+  v += dpp<kDppRow2>(v);
+  v += dpp<kDppRow1>(v);
+  v += dpp<kDppCol2>(v);
+  v += dpp<kDppSwap>(v);
   return v;
 }
+// sum over the 4 rows of a column
+QMX_DEV double sumcol(double v) {
+  v += dpp<kDppRow2>(v);
+  v += dpp<kDppRow1>(v);
+  return v;
+}
+QMX_DEV double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+QMX_DEV double2 lane_value2(double2 v, int lane) { return make_double2(lane_value(v.x, lane), lane_value(v.y, lane)); }
 
-// In-place inverse by Gauss-Jordan elimination with row pivoting (largest
-// |entry| in the pivot column, first on ties), the operations of
-// inv4_inplace entry by entry.  Returns false (on every lane) for a zero
-// pivot or a non-finite result.
-QMX_DEV bool inv4_lanes(double2& m, int l) {
-  const int i = l >> 2, j = l & 3;
-  int perm[4];
+// Cofactor of entry (i, j): rows and columns taken cyclically after i and j
+// (a cyclic shift of three is an even permutation), sign (-1)^(i + j).
+QMX_DEV double2 cofactor4(double2 m, int l) {
+  const double2 a0 = dpp2<kDppRow1>(m), b0 = dpp2<kDppRow2>(m), c0 = dpp2<kDppRow3>(m);
+  const double2 a1 = dpp2<kDppCol1>(a0), a2 = dpp2<kDppCol2>(a0), a3 = dpp2<kDppCol3>(a0);
+  const double2 b1 = dpp2<kDppCol1>(b0), b2 = dpp2<kDppCol2>(b0), b3 = dpp2<kDppCol3>(b0);
+  const double2 c1 = dpp2<kDppCol1>(c0), c2 = dpp2<kDppCol2>(c0), c3 = dpp2<kDppCol3>(c0);
+  auto minor = [](double2 p, double2 q, double2 r, double2 s) { return csub(cmul(p, s), cmul(q, r)); };
+  double2 c = cmul(a1, minor(b2, b3, c2, c3));
+  c = csub(c, cmul(a2, minor(b1, b3, c1, c3)));
+  c = cfma(a3, minor(b1, b2, c1, c2), c);
+  const double s = ((l ^ (l >> 2)) & 1) ? -1.0 : 1.0;
+  return cscale(c, s);
+}
+
+// 1 / x to rounding: the hardware estimate and two Newton steps
+QMX_DEV double rcp_newton(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+
+// 1 / sqrt(x) to rounding, x in the normal range away from its ends
+QMX_DEV double rsqrt_newton(double x) {
+  double r = __builtin_amdgcn_rsq(x);
+  const double h = 0.5 * x;
+  r = fma(r, fma(-h * r, r, 0.5), r);
+  return fma(r, fma(-h * r, r, 0.5), r);
+}
+
+// conj(X^{-1}[j][i]) at lane (i, j), by Gauss-Jordan exchange steps with row
+// pivoting (largest |entry| of the column among the rows not used yet, first
+// on ties).  Rows stay in place: after step k row p_k stands for unknown k and
+// column k for equation p_k, so X^{-1}[a][b] = M[p_a][l] with p_l = b.
+// False (on every lane) for a zero pivot or a non-finite result.
+QMX_DEV bool inv4_wave(double2 m, int l, double2& out) {
+  const int i = (l >> 2) & 3, j = l & 3;
+  int pj = 0, qi = 0;       // p_j and the l with p_l = i
+  unsigned used = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const double c = cabs2(m);
-    int p = k;
-    double best = __shfl(c, k * 4 + k, 16);
+    double2 f;
+    f = k == 0 ? dpp2<0x00>(m) : (k == 1 ? dpp2<0x55>(m) : (k == 2 ? dpp2<0xaa>(m) : dpp2<0xff>(m)));   // X[i][k]
+    const double c = cabs2(f);
+    int p = -1;
+    double best = 0.0;
 #pragma unroll
-    for (int r = k + 1; r < 4; ++r) {
-      const double v = __shfl(c, r * 4 + k, 16);
-      if (v > best) {
+    for (int r = 0; r < 4; ++r) {
+      const double v = lane_value(c, 4 * r);
+      if (!((used >> r) & 1u) && v > best) {
         best = v;
         p = r;
       }
     }
-    if (!(best > 0.0)) return false;
-    perm[k] = p;
-    if (p != k) m = shfl16(m, i == k ? p * 4 + j : (i == p ? k * 4 + j : l));
-    const double2 piv = shfl16(m, k * 4 + k);
-    const double ib = 1.0 / best;
+    if (p < 0) return false;
+    p = __builtin_amdgcn_readfirstlane(p);
+    used |= 1u << p;
+    if (j == k) pj = p;
+    if (i == p) qi = k;
+    const double2 rk = make_double2(__shfl(m.x, 4 * p + j, 16), __shfl(m.y, 4 * p + j, 16));   // X[p][j]
+    const double2 piv = lane_value2(m, 4 * p + k);
+    const double ib = rcp_newton(best);
     const double2 ip = make_double2(piv.x * ib, -piv.y * ib);   // 1 / pivot
-    const double2 rk = shfl16(m, k * 4 + j);                      // row k, column j
-    const double2 f = shfl16(m, i * 4 + k);                       // row i, column k
     const double2 rkj = cmul(j == k ? make_double2(1.0, 0.0) : rk, ip);
-    m = (i == k) ? rkj : csub(j == k ? cz() : m, cmul(f, rkj));
+    m = (i == p) ? rkj : csub(j == k ? cz() : m, cmul(f, rkj));
   }
-#pragma unroll
-  for (int k = 3; k >= 0; --k) {
-    const int p = perm[k];
-    if (p != k) m = shfl16(m, j == k ? i * 4 + p : (j == p ? i * 4 + k : l));
-  }
+  const int src = 4 * pj + qi;
+  out = make_double2(__shfl(m.x, src, 16), -__shfl(m.y, src, 16));
   return sum16(cabs2(m)) < 1e300;   // false for inf / nan
 }
 
-// polar4_newton on 16 lanes (lane l holds X[l / 4][l % 4] on entry and the
-// unitary factor on a true return).
-QMX_DEV bool polar4_newton_lanes(double2& x, int l) {
-  const int i = l >> 2, j = l & 3;
-  bool scale = true;
+// Unitary polar factor of a nonsingular 4 x 4 matrix by the scaled Newton
+// iteration (N. J. Higham, "Computing the polar decomposition -- with
+// applications", SIAM J. Sci. Stat. Comput. 7 (1986)); x is this lane's entry,
+// the factor's on a true return:
+//   X_{k+1} = (z X_k + X_k^{-H} / z) / 2,  z = (||X_k^{-1}||_F / ||X_k||_F)^{1/2},
+// which converges quadratically.  With P = |X|_F^2 |X^{-1}|_F^2, 16 for a
+// multiple of a unitary, the singular values s of z X satisfy
+// sum (s - 1/s)^2 = 2 sqrt(P) - 8: a step with P <= 16 + 3.2e-7 leaves them
+// within 1e-8 of 1, and one more step, with z = 1, within rounding.  False, with x unspecified,
+// for an ill-conditioned matrix (P > 1e12 at the start), a failed inverse, or
+// no convergence in 40 steps.  The inverse comes from cofactors, 1 / det times
+// one 3 x 3 minor per lane with no serial pivots, once |det| says that no
+// cancellation can matter: normalised by (|X|_F / 2)^4 it is 1 for a multiple
+// of a unitary, and below kPolarDetMin the step takes the pivoted inverse.
+// On the sweeps' environments (condition numbers 5 to 90 at the median) 0.2 to
+// 1.0 of the 5 to 6 steps are pivoted.  z only has to be close to the optimal
+// scaling and comes from FP32 estimates; 1 / z is its inverse to rounding.
+// Bound by the latency of its dependent FP64 chain: 6700 cycles for a
+// Gaussian 4 x 4 matrix, 10500 at condition number 100 to 1000 (one pivoted
+// step), where one 16-lane pivoted inverse per step through ds_bpermute took
+// 24100 and 26600.
+constexpr double kPolarDetMin = 0.05;
+
+QMX_DEV bool polar4_newton_wave(double2& x, int l) {
+  bool last = false;
   for (int it = 0; it < 40; ++it) {
-    double2 xi = x;
-    if (!inv4_lanes(xi, l)) return false;
-    const double nx = sum16(cabs2(x)), ni = sum16(cabs2(xi));
-    if (it == 0 && nx * ni > 1e12) return false;
-    const double z = scale ? sqrt(sqrt(ni / nx)) : 1.0;
-    const double zi = 1.0 / z;
-    // X_{k+1}[i][j] = (z X[i][j] + conj(X^{-1}[j][i]) / z) / 2
-    const double2 b = shfl16(xi, j * 4 + i);
-    const double2 v = make_double2(0.5 * (z * x.x + zi * b.x), 0.5 * (z * x.y - zi * b.y));
-    const double dl = sum16(cabs2(csub(v, x)));
-    x = v;
-    if (dl < 1e-4) scale = false;
-    if (dl <= 1e-16) return true;
+    const double2 c = cofactor4(x, l);
+    const double nx = sum16(cabs2(x)), nc = sum16(cabs2(c));
+    double2 d = cmul(x, c);
+    d.x += dpp<kDppCol2>(d.x);
+    d.y += dpp<kDppCol2>(d.y);
+    d.x += dpp<kDppSwap>(d.x);
+    d.y += dpp<kDppSwap>(d.y);
+    d = lane_value2(d, 0);                      // det X
+    const double ad = cabs2(d);
+    const double q = 0.0625 * nx * nx;          // (|X|_F / 2)^4
+    double2 b;                                  // conj(X^{-1}[j][i])
+    double ni;                                  // |X^{-1}|_F^2
+    if (ad >= kPolarDetMin * kPolarDetMin * q * q) {
+      // conj(C / det) = conj(C) det / |det|^2
+      const double r = rcp_newton(ad);
+      ni = nc * r;
+      b = cscale(cmulc(c, d), r);
+    } else {
+      if (!inv4_wave(x, l, b)) return false;
+      ni = sum16(cabs2(b));
+      if (it == 0 && !(nx * ni <= 1e12)) return false;
+    }
+    const double p = nx * ni;
+    double z = 0.5, zi = 0.5;
+    if (!last) {
+      const float s = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf((float)ni * __builtin_amdgcn_rcpf((float)nx)));
+      z = (double)s;
+      zi = (double)__builtin_amdgcn_rcpf(s);
+      zi = fma(fma(-z, zi, 1.0), zi, zi);
+      zi = 0.5 * fma(fma(-z, zi, 1.0), zi, zi);
+      z *= 0.5;
+    }
+    x = make_double2(fma(z, x.x, zi * b.x), fma(z, x.y, zi * b.y));
+    if (last) return true;
+    last = p <= 16.0 + 3.2e-7;
   }
   return false;
 }
 
+// Unitary polar factor of a 2 x 2 matrix (a b; c d): with e = det / |det|,
+// M + e adj(M)^H has both singular values s_1 + s_2, whose square is
+// |M|_F^2 + 2 |det|; so the factor is that sum over its norm.  False for a
+// matrix singular to 1e-13.  |M|_F is near 1.
+QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc) {
+  const double fro = (cabs2(a) + cabs2(b)) + (cabs2(c) + cabs2(d));
+  const double2 det = csub(cmul(a, d), cmul(b, c));
+  const double d2 = cabs2(det);
+  if (!(d2 > 1e-26 * fro * fro)) return false;
+  const double id = rsqrt_newton(d2);
+  const double2 e = cscale(det, id);
+  const double s2 = fma(2.0 * d2, id, fro);
+  const double r = rsqrt_newton(s2);
+  *nuc = s2 * r;
+  // adj(M)^H = (conj d, -conj c; -conj b, conj a)
+  const double2 a2 = cadd(a, cmulc(d, e)), b2 = csub(b, cmulc(c, e));
+  const double2 c2 = csub(c, cmulc(b, e)), e2 = cadd(d, cmulc(a, e));
+  a = cscale(a2, r); b = cscale(b2, r); c = cscale(c2, r); d = cscale(e2, r);
+  return true;
+}
+
+// The environments of the gates next to a site still in |0>: two columns of E
+// are zero (to 1e-14 of its norm; the Jacobi path drops singular values below
+// 1e-13 of the largest).  With Q R = the two columns left (Gram-Schmidt, two
+// passes), their part of the factor is Q polar(R); the zero columns z_1 < z_2,
+// whose right singular vectors are e_{z_1}, e_{z_2}, take the rule's left
+// completion, the first unit vectors with a residual above 1/2 (which one
+// pass of Gram-Schmidt then gives to rounding): 5300 cycles, against 30600 by
+// the Jacobi path.  x: this lane's entry of E,
+// es 2^-h: all 16, fro: |x|^2, near 1.  False if E is not of this kind.
+QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, double fro, double* nuc) {
+  const double cn = sumcol(cabs2(x));
+  unsigned zero = 0;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (lane_value(cn, j) <= 1e-28 * fro) zero |= 1u << j;
+  zero = __builtin_amdgcn_readfirstlane(zero);
+  if (__popc(zero) != 2) return false;
+  const unsigned live = ~zero & 15u;
+  const int c0 = __ffs(live) - 1, c1 = 31 - __clz(live), z0 = __ffs(zero) - 1, z1 = 31 - __clz(zero);
+  // every lane holds the whole 4 x 2 problem
+  double2 q0[4], q1[4], q2[4], q3[4];
+  double n0 = 0.0, n1 = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const double2 u = es[i * 4 + c0], v = es[i * 4 + c1];
+    q0[i] = make_double2(ldexp(u.x, h), ldexp(u.y, h));
+    q1[i] = make_double2(ldexp(v.x, h), ldexp(v.y, h));
+    n0 += cabs2(q0[i]);
+  }
+  const double i0 = rsqrt_newton(n0);
+  double2 p00 = make_double2(n0 * i0, 0.0), p01 = cz(), p10 = cz();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q0[i] = cscale(q0[i], i0);
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    double2 d = cz();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d = cfmac(q0[i], q1[i], d);
+    p01 = cadd(p01, d);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q1[i] = csub(q1[i], cmul(q0[i], d));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) n1 += cabs2(q1[i]);
+  if (!(n1 > 1e-26 * fro)) return false;
+  const double i1 = rsqrt_newton(n1);
+  double2 p11 = make_double2(n1 * i1, 0.0);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) q1[i] = cscale(q1[i], i1);
+  if (!polar2(p00, p01, p10, p11, nuc)) return false;
+  // squared residuals of e_0 .. e_3 against the vectors so far
+  double res[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) res[e] = 1.0 - cabs2(q0[e]) - cabs2(q1[e]);
+  int e2 = -1, e3 = -1;
+#pragma unroll
+  for (int e = 3; e >= 0; --e)
+    if (res[e] > 0.25) e2 = e;
+  if (e2 < 0) return false;
+  auto pick = [](const double2 (&v)[4], int k) { return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3])); };
+  {
+    const double2 h0 = pick(q0, e2), h1 = pick(q1, e2);
+    double nr = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double2 t = cadd(cmulc(h0, q0[i]), cmulc(h1, q1[i]));
+      q2[i] = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
+      nr += cabs2(q2[i]);
+    }
+    const double ir = rsqrt_newton(nr);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q2[i] = cscale(q2[i], ir);
+  }
+#pragma unroll
+  for (int e = 3; e >= 0; --e)
+    if (e > e2 && res[e] - cabs2(q2[e]) > 0.25) e3 = e;
+  if (e3 < 0) return false;
+  {
+    const double2 h0 = pick(q0, e3), h1 = pick(q1, e3), h2 = pick(q2, e3);
+    double nr = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double2 t = cadd(cadd(cmulc(h0, q0[i]), cmulc(h1, q1[i])), cmulc(h2, q2[i]));
+      q3[i] = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
+      nr += cabs2(q3[i]);
+    }
+    const double ir = rsqrt_newton(nr);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q3[i] = cscale(q3[i], ir);
+  }
+  const int i = (l >> 2) & 3, j = l & 3;
+  const double2 a = pick(q0, i), b = pick(q1, i);
+  if (j == z0) x = pick(q2, i);
+  else if (j == z1) x = pick(q3, i);
+  else if (j == c0) x = cadd(cmul(a, p00), cmul(b, p10));
+  else x = cadd(cmul(a, p01), cmul(b, p11));
+  return true;
+}
+
+// Polar factor of the d x d matrix in es (LDS, stride 4) on one wave; lane l
+// returns entry l & 15 in x (zero outside the d x d block) and the sum of the
+// singular values.  False: the matrix is left to polar4_jacobi.
+QMX_DEV bool polar4_wave(int d, const double2* es, double2& x, int lane, double* nuc) {
+  const int l = lane & 15, i = l >> 2, j = l & 3;
+  const bool in = i < d && j < d;
+  const double2 e = in ? es[l] : cz();
+  double fro = sum16(cabs2(e));
+  if (!(fro > 1e-280) || !(fro < 1e280)) return false;
+  // exact scaling by a power of two to |x|^2 in [1/2, 2)
+  const int h = -(__builtin_amdgcn_frexp_exp(fro) >> 1);
+  x = make_double2(ldexp(e.x, h), ldexp(e.y, h));
+  fro = ldexp(fro, 2 * h);
+  bool ok;
+  double s = 0.0;
+  if (d == 2) {
+    double2 a = lane_value2(x, 0), b = lane_value2(x, 1), c = lane_value2(x, 4), f = lane_value2(x, 5);
+    const double n0 = cabs2(a) + cabs2(c), n1 = cabs2(b) + cabs2(f);
+    if (n1 <= 1e-28 * n0) {
+      // the site is still in |0>: one column, completed as in polar4_jacobi
+      const double r = rsqrt_newton(n0);
+      s = n0 * r;
+      a = cscale(a, r);
+      c = cscale(c, r);
+      const bool first = cabs2(c) > 0.25;   // the residual of e_0 has norm |c|
+      const double2 g = first ? a : c;
+      const double2 t0 = cmulc(g, a), t1 = cmulc(g, c);
+      b = make_double2((first ? 1.0 : 0.0) - t0.x, -t0.y);
+      f = make_double2((first ? 0.0 : 1.0) - t1.x, -t1.y);
+      const double q = rsqrt_newton(cabs2(b) + cabs2(f));
+      b = cscale(b, q);
+      f = cscale(f, q);
+      ok = true;
+    } else {
+      ok = polar2(a, b, c, f, &s);
+    }
+    x = i == 0 ? (j == 0 ? a : b) : (j == 0 ? c : f);
+    if (!in) x = cz();
+  } else if (polar4_two_columns(x, l, es, h, fro, &s)) {
+    ok = true;
+  } else {
+    const double2 y = x;
+    ok = polar4_newton_wave(x, l);
+    if (ok) s = sum16(x.x * y.x + x.y * y.y);   // Re tr(U^H E)
+  }
+  *nuc = ldexp(s, -h);
+  return ok;
+}
+
 // Unitary polar factor U V^H of the d x d (d = 2 or 4) matrix e (row-major,
-// stride 4).  Well-conditioned inputs (see polar4_newton) take the Newton
-// iteration; the others (and any input it rejects) a one-sided (Hestenes) Jacobi SVD on a 4 x 4 working matrix (a
+// stride 4) in one lane, for the inputs that polar4_wave leaves to it: a
+// one-sided (Hestenes) Jacobi SVD on a 4 x 4 working matrix (a
 // 2 x 2 problem is embedded as diag(E, |E| I), whose padded columns are
 // orthogonal to E's and never rotate).  Rotations: cyclic pairs p < q, when
 // |a_p^H a_q| > 1e-16 |a_p| |a_q|.  Pairs (u_j, v_j) with sigma_j >
@@ -530,66 +689,50 @@ QMX_DEV void polar4_jacobi(int d, const double2* e, double2* out, double* nuc) {
     }
 }
 
-QMX_DEV void polar4(int d, const double2* e, double2* out, double* nuc) {
-  // the Newton iterate, in out: e, or diag(E, |E|_F I) for a 2 x 2 problem
-  double fro = 0.0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int r = i / 4, c = i % 4;
-    out[i] = (r < d && c < d) ? e[i] : cz();
-    fro += cabs2(out[i]);
-  }
-  if (d == 2) {
-    const double s = fro > 0.0 ? sqrt(fro) : 1.0;
-    out[10] = make_double2(s, 0.0);
-    out[15] = make_double2(s, 0.0);
-  }
-  // e is read again below (from LDS where the kernels keep it) instead of
-  // being held in registers through the iteration
-  asm volatile("" ::: "memory");
-  if (fro > 0.0 && polar4_newton(out)) {
-    asm volatile("" ::: "memory");
-    double tr = 0.0;   // Re tr(U^H E) = sum of the singular values
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int r = i / 4, c = i % 4;
-      if (r < d && c < d) {
-        tr += out[i].x * e[i].x + out[i].y * e[i].y;
-      } else {
-        out[i] = cz();
-      }
-    }
-    *nuc = tr;
-    return;
-  }
-  asm volatile("" ::: "memory");
-  polar4_jacobi(d, e, out, nuc);
-}
-
-// Over-relaxed local update (no reference counterpart).  g holds the plain
-// update conj(polar(E)) of a gate whose value before the update was g_old;
-// with omega_m1 = omega - 1 its d x d block becomes
+// The update of one gate on one wave: g_new = conj(polar(E)), d x d block of
+// the 4 x 4 es, and zero outside it.  With omega_m1 = omega - 1 != 0 the
+// over-relaxed update (no reference counterpart): g becomes
 //   polar(g + omega_m1 (g - g_old)),
 // a step past the local optimum along the direction of the update, projected
-// back onto the unitaries (omega = 1 leaves g as it is).  Returns the
-// overlap after the update, |sum_{o,i} g[o][i] E[o][i]| over the block.
-QMX_DEV double relax_update(int d, double omega_m1, const double2* g_old, double2* g, const double2* e,
-                            double2* m) {
-  // m (16 entries of scratch, LDS in the kernels: the polar reads it from
-  // there rather than holding a second copy in registers)
+// back onto the unitaries.  es, g_old, rm (scratch) and g_new hold 16 entries
+// each in LDS and are used by this wave alone until the caller's barrier.
+// Returns the overlap after the update, the sum of E's singular values or
+// |sum_{o,i} g[o][i] E[o][i]| (on every lane).
+QMX_DEV double update_gate_wave(int d, double omega_m1, const double2* g_old, const double2* es, double2* rm,
+                                double2* g_new, int lane) {
+  const int l = lane & 15;
+  const bool in = (l >> 2) < d && (l & 3) < d;
+  const int rounds = omega_m1 != 0.0 ? 2 : 1;
+  const double2* m = es;
+  double nuc = 0.0;
+  double2 g = cz();
+  for (int r = 0; r < rounds; ++r) {
+    __builtin_amdgcn_wave_barrier();
+    if (!polar4_wave(d, m, g, lane, &nuc)) {
+      // zero or ill-conditioned matrices, and whatever else it declined
+      if (lane == 0) {
+        double2 w[16];
+        polar4_jacobi(d, m, w, &nuc);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const bool in = (k / 4) < d && (k % 4) < d;
-    m[k] = in ? cadd(g[k], cscale(csub(g[k], g_old[k]), omega_m1)) : cz();
+        for (int k = 0; k < 16; ++k) g_new[k] = w[k];
+      }
+      __builtin_amdgcn_wave_barrier();
+      nuc = lane_value(nuc, 0);
+      g = g_new[l];
+    }
+    if (r == 0) g = cconj(g);
+    if (r + 1 < rounds) {
+      if (lane < 16) rm[l] = in ? cadd(g, cscale(csub(g, g_old[l]), omega_m1)) : cz();
+      m = rm;
+    }
   }
-  double unused = 0.0;
-  polar4(d, m, g, &unused);
-  asm volatile("" ::: "memory");
-  double2 ov = cz();
-#pragma unroll
-  for (int k = 0; k < 16; ++k)
-    if ((k / 4) < d && (k % 4) < d) ov = cfma(g[k], e[k], ov);
-  return cabs_(ov);
+  if (lane < 16) g_new[l] = g;
+  if (rounds > 1) {
+    const double2 p = in ? cmul(g, es[l]) : cz();
+    const double re = sum16(p.x), im = sum16(p.y);
+    nuc = sqrt(re * re + im * im);
+  }
+  return nuc;
 }
 
 // --------------------------------------------- Householder null space -----

@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void apply_pass_kernel(PassArgs<S> a) {
 //   phi <- G_k^dagger phi          (remove the old gate)
 //   E_k[o, i] += conj(T'[o]) phi[i]  (FP64 partial sums)
 // The last block of each state reduces the partials in a fixed order, takes
-// the polar factor of E_k (one-sided Jacobi, FP64) and stores
+// the polar factor of E_k (update_gate_wave, FP64) and stores
 // G'_k = conj(U V^H) in place of G_k; overlap[b] receives tr(S) = <T|C'|0>.
 template <typename S>
 __global__ __launch_bounds__(256) void sweep_step_kernel(SweepArgs<S> a) {
@@ -539,22 +539,19 @@ __global__ __launch_bounds__(256) void sweep_step_kernel(SweepArgs<S> a) {
   double* pb = a.part + (size_t)b * gridDim.x * 32;
   if (publish_partial<32>(red, pb, a.counter + b, gridDim.x, &s_flag)) {
     reduce_partials<32>(pb, gridDim.x, scratch, tot);
-    if (threadIdx.x == 0) {
-      // E and the relaxed update's scratch in LDS: the polar solves read them
-      // from there
-      double2 u[16];
-      for (int j = 0; j < 16; ++j) s_em[j] = make_double2(tot[2 * j], tot[2 * j + 1]);
-      int d = wc == 2 ? 4 : 2;
-      double nuc = 0.0;
-      polar4(d, s_em, u, &nuc);
-      for (int j = 0; j < 16; ++j) {
-        int o = j / 4, i = j % 4;
-        u[j] = (o < d && i < d) ? cconj(u[j]) : cz();
+    if (threadIdx.x < 64) {
+      const int lane = threadIdx.x, l = lane & 15;
+      if (lane < 16) {
+        s_em[l] = make_double2(tot[2 * l], tot[2 * l + 1]);
+        gp[l] = a.gates[gic * 16 + l];
       }
-      if (a.omega_m1 != 0.0) nuc = relax_update(d, a.omega_m1, a.gates + gic * 16, u, s_em, s_rm);
-      for (int j = 0; j < 16; ++j) a.gates[gic * 16 + j] = u[j];
-      if (a.overlap) a.overlap[(size_t)b * a.overlap_stride] = nuc;
-      a.counter[b] = 0;
+      const double nuc = update_gate_wave(wc == 2 ? 4 : 2, a.omega_m1, gp, s_em, s_rm, gc, lane);
+      __builtin_amdgcn_wave_barrier();
+      if (lane < 16) a.gates[gic * 16 + l] = gc[l];
+      if (lane == 0) {
+        if (a.overlap) a.overlap[(size_t)b * a.overlap_stride] = nuc;
+        a.counter[b] = 0;
+      }
     }
   }
 }

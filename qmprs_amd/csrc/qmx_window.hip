@@ -823,7 +823,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   fwd_mfma_body(a);
 }
 
-// Replay the window on the 16-dim space of U (one block per state).
+// Replay the window on the 16-dim space of U (one block per state).  A chain
+// of dependent small steps, bound by their latency: wave 0 takes each gate's
+// environment and polar factor without a barrier inside, the other waves apply
+// the next gate to the state side of Q at the same time (the two sides
+// commute), and two barriers per gate are left.  16.6 us per window of one
+// N=10 complex128 state (3.3 gates), against 48.3 us with a barrier around each
+// of the gate's steps and the 16-lane pivoted polar.
 // It runs beside the other half-batch's window pass, whose waves fill the
 // SIMDs; its own waves take the highest issue priority so that this short,
 // latency-bound chain is not slowed down by them.
@@ -837,8 +843,6 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
   __shared__ double2 es[16];
   __shared__ double2 rm[16];
   __shared__ double part_sum[512];
-  __shared__ double s_nuc;
-  __shared__ int s_ok;
   const int b = a.list ? a.list[blockIdx.x] : blockIdx.x;
   const int n = a.n;
   if (a.skip && a.skip[b]) return;
@@ -883,108 +887,73 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
     part_sum[e] = s;
   }
   __syncthreads();
-  const int x = threadIdx.x >> 4, y = threadIdx.x & 15;
   q[threadIdx.x] = make_double2(part_sum[2 * threadIdx.x], part_sum[2 * threadIdx.x + 1]);
   __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int j = 0; j < nc; ++j) {
     const int w = gw[j], hb = gh[j], lb = gl[j];
-    // E[o][i] = sum_z Q[(o,z)][(i,z)] over the U bits outside gate j (16 lanes)
-    if (threadIdx.x < 16) {
-      const int o = threadIdx.x >> 2, i = threadIdx.x & 3;
-      const int d = w == 2 ? 4 : 2;
+    const int d = w == 2 ? 4 : 2;
+    const bool more = j + 1 < nc;
+    if (wave == 0) {
+      // E[o][i] = sum_z Q[(o,z)][(i,z)] over the U bits outside gate j, one
+      // entry per lane (the four rows of 16 lanes alike)
+      const int o = (lane >> 2) & 3, i = lane & 3;
+      const int gmask = w == 2 ? (1 << hb) | (1 << lb) : 1 << hb;
+      const int xo = w == 2 ? ((o >> 1) << hb) | ((o & 1) << lb) : (o & 1) << hb;
+      const int yi = w == 2 ? ((i >> 1) << hb) | ((i & 1) << lb) : (i & 1) << hb;
       double2 acc = cz();
       if (o < d && i < d) {
-        for (int xx = 0; xx < 16; ++xx) {
-          int go = w == 2 ? (((xx >> hb) & 1) << 1) | ((xx >> lb) & 1) : ((xx >> hb) & 1);
-          if (go != o) continue;
-          int yy;
-          if (w == 2) yy = (xx & ~((1 << hb) | (1 << lb))) | (((i >> 1) & 1) << hb) | ((i & 1) << lb);
-          else yy = (xx & ~(1 << hb)) | ((i & 1) << hb);
-          acc = cadd(acc, q[xx * 16 + yy]);
+        int z = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if (k >= 16 / d) break;
+          acc = cadd(acc, q[(z | xo) * 16 + (z | yi)]);
+          z = ((z | gmask) + 1) & ~gmask & 15;   // the next pattern of the other bits
         }
       }
-      es[threadIdx.x] = acc;
+      if (lane < 16) es[lane] = acc;
+      const double nuc = update_gate_wave(d, a.omega_m1, gm[j], es, rm, gnew, lane);
+      __builtin_amdgcn_wave_barrier();
+      if (lane < 16) {
+        int layer, site;
+        step_gate(n, a.s0 + j, layer, site);
+        const size_t gi = ((size_t)b * a.lmax + layer) * n + site;
+        a.gates[gi * 16 + lane] = gnew[lane];
+      }
+      if (lane == 0 && a.s0 + j == kb - 1 && a.overlap) a.overlap[(size_t)b * a.overlap_stride] = nuc;
+    } else if (more) {
+      // the other waves apply the next gate on the state side meanwhile:
+      // Q[x][y] <- sum_{y'} Q[x][y'] conj(G_{j+1}[y'_g][y_g])
+      const int w2 = gw[j + 1], hb2 = gh[j + 1], lb2 = gl[j + 1];
+      const int m2 = w2 == 2 ? (1 << hb2) | (1 << lb2) : 1 << hb2;
+      for (int e = threadIdx.x - 64; e < 256; e += 192) {
+        const int x = e >> 4, y = e & 15;
+        const int yg = w2 == 2 ? (((y >> hb2) & 1) << 1) | ((y >> lb2) & 1) : ((y >> hb2) & 1);
+        double2 s = cz();
+#pragma unroll
+        for (int pg = 0; pg < 4; ++pg) {
+          if (pg >= 2 && w2 != 2) break;
+          const int yp = (y & ~m2) | (w2 == 2 ? ((pg >> 1) << hb2) | ((pg & 1) << lb2) : pg << hb2);
+          s = cfmac(gm[j + 1][pg * 4 + yg], q[x * 16 + yp], s);
+        }
+        qn[e] = s;
+      }
     }
+    if (!more) break;   // Q is not read after the window's last gate
     __syncthreads();
-    const int d = w == 2 ? 4 : 2;
-    const bool last_gate = a.s0 + j == kb - 1 && a.overlap;
-    if (threadIdx.x < 16) {
-      // polar(E) by the scaled Newton iteration on 16 lanes (one entry
-      // each); the iterate is E, or diag(E, |E|_F I) for a 2 x 2 problem
-      const int l = threadIdx.x, r = l >> 2, c = l & 3;
-      const bool in = r < d && c < d;
-      double2 xv = in ? es[l] : cz();
-      const double fro = sum16(cabs2(xv));
-      if (d == 2 && (l == 10 || l == 15)) xv = make_double2(fro > 0.0 ? sqrt(fro) : 1.0, 0.0);
-      const bool ok = fro > 0.0 && polar4_newton_lanes(xv, l);
-      if (ok) {
-        const double2 uv = in ? xv : cz();
-        // Re tr(U^H E) = sum of the singular values
-        const double tr = sum16(in ? uv.x * es[l].x + uv.y * es[l].y : 0.0);
-        gnew[l] = cconj(uv);
-        if (l == 0) {
-          s_nuc = tr;
-          if (last_gate && a.omega_m1 == 0.0) a.overlap[(size_t)b * a.overlap_stride] = tr;
-        }
-      }
-      if (l == 0) s_ok = ok ? 1 : 0;
-    }
-    __syncthreads();
-    if (!s_ok || a.omega_m1 != 0.0) {
-      // ill-conditioned E (Jacobi SVD, one lane), and the over-relaxed step
-      if (threadIdx.x == 0) {
-        double2 u[16];
-        double nuc = s_nuc;
-        if (!s_ok) {
-          polar4_jacobi(d, es, u, &nuc);
-#pragma unroll
-          for (int k = 0; k < 16; ++k) u[k] = cconj(u[k]);
-        } else {
-#pragma unroll
-          for (int k = 0; k < 16; ++k) u[k] = gnew[k];
-        }
-        if (a.omega_m1 != 0.0) nuc = relax_update(d, a.omega_m1, gm[j], u, es, rm);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) gnew[k] = u[k];
-        if (last_gate) a.overlap[(size_t)b * a.overlap_stride] = nuc;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x < 16) {
-      int layer, site;
-      step_gate(n, a.s0 + j, layer, site);
-      size_t gi = ((size_t)b * a.lmax + layer) * n + site;
-      a.gates[gi * 16 + threadIdx.x] = gnew[threadIdx.x];
-    }
     // target side: Q[x][y] <- sum_{x'} G'[x'_g][x_g] Q[x'][y]
     {
-      double2 s = cz();
+      const int x = threadIdx.x >> 4, y = threadIdx.x & 15;
+      const int gmask = w == 2 ? (1 << hb) | (1 << lb) : 1 << hb;
       const int xg = w == 2 ? (((x >> hb) & 1) << 1) | ((x >> lb) & 1) : ((x >> hb) & 1);
-      const int d = w == 2 ? 4 : 2;
-      for (int pg = 0; pg < d; ++pg) {
-        int xp = x;
-        if (w == 2) xp = (xp & ~((1 << hb) | (1 << lb))) | (((pg >> 1) & 1) << hb) | ((pg & 1) << lb);
-        else xp = (xp & ~(1 << hb)) | ((pg & 1) << hb);
-        s = cfma(gnew[pg * 4 + xg], q[xp * 16 + y], s);
-      }
-      qn[threadIdx.x] = s;
-    }
-    __syncthreads();
-    // state side: Q[x][y] <- sum_{y'} Q[x][y'] conj(G_{j+1}[y'_g][y_g])
-    if (j + 1 < nc) {
-      const int w2 = gw[j + 1], hb2 = gh[j + 1], lb2 = gl[j + 1];
-      const int yg = w2 == 2 ? (((y >> hb2) & 1) << 1) | ((y >> lb2) & 1) : ((y >> hb2) & 1);
-      const int d2 = w2 == 2 ? 4 : 2;
       double2 s = cz();
-      for (int pg = 0; pg < d2; ++pg) {
-        int yp = y;
-        if (w2 == 2) yp = (yp & ~((1 << hb2) | (1 << lb2))) | (((pg >> 1) & 1) << hb2) | ((pg & 1) << lb2);
-        else yp = (yp & ~(1 << hb2)) | ((pg & 1) << hb2);
-        s = cfmac(gm[j + 1][pg * 4 + yg], qn[x * 16 + yp], s);
+#pragma unroll
+      for (int pg = 0; pg < 4; ++pg) {
+        if (pg >= 2 && w != 2) break;
+        const int xp = (x & ~gmask) | (w == 2 ? ((pg >> 1) << hb) | ((pg & 1) << lb) : pg << hb);
+        s = cfma(gnew[pg * 4 + xg], qn[xp * 16 + y], s);
       }
       q[threadIdx.x] = s;
-    } else {
-      q[threadIdx.x] = qn[threadIdx.x];
     }
     __syncthreads();
   }
