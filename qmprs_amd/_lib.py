@@ -7,6 +7,7 @@ the library or the GPU is missing every entry point raises.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from pathlib import Path
@@ -221,12 +222,33 @@ QMX_OPT_SWEEP_RELAXATION = 6
 QMX_OPT_JACOBI_SWEEP_CAP = 7
 QMX_OPT_FAIL_UNITARITY = 8
 QMX_OPT_FWD_MFMA = 9
+QMX_OPT_TWO_SIDED_JACOBI = 10
 FWD_MFMA_DEFAULT = 1  # the library's default for QMX_OPT_FWD_MFMA
 
 
 def set_option(option: int, value: int) -> None:
     h = handle()
     check(load().qmx_set_option(h, option, int(value)), h)
+    _set_options()[option] = int(value)
+
+
+def _set_options() -> dict:
+    """The options set on this thread's handle of the current device."""
+    per = getattr(_local, "options", None)
+    if per is None:
+        per = _local.options = {}
+    return per.setdefault(torch.cuda.current_device(), {})
+
+
+@contextlib.contextmanager
+def two_sided_jacobi():
+    """QMX_OPT_TWO_SIDED_JACOBI = 1 on this thread's handle inside the block."""
+    before = _set_options().get(QMX_OPT_TWO_SIDED_JACOBI, 0)
+    set_option(QMX_OPT_TWO_SIDED_JACOBI, 1)
+    try:
+        yield
+    finally:
+        set_option(QMX_OPT_TWO_SIDED_JACOBI, before)
 
 
 def forward_plan(num_qubits: int, num_layers: int):

@@ -40,6 +40,7 @@ struct qmx_handle {
   int relax_milli = 1000;               // QMX_OPT_SWEEP_RELAXATION (omega * 1000)
   int jacobi_sweep_cap = 0;             // QMX_OPT_JACOBI_SWEEP_CAP (0: the solvers' own limits)
   bool fail_unitarity = false;          // QMX_OPT_FAIL_UNITARITY (failure injection)
+  bool two_sided = false;               // QMX_OPT_TWO_SIDED_JACOBI
   hipStream_t aux[2] = {nullptr, nullptr};   // the two half-batch jobs
   hipEvent_t pass_ev[2] = {nullptr, nullptr};
   hipEvent_t join_ev[2] = {nullptr, nullptr};
@@ -204,7 +205,8 @@ struct ChiLayout {
   int* kk;
   int* ncur;
   int* error;
-  double* jlog;      // LDS Jacobi rotation log (nmax <= 128)
+  int* jrank;        // one-sided Jacobi: Cholesky factors' column counts (nmax <= 128)
+  double* jlog;      // two-sided LDS Jacobi: rotation log (nmax <= 128)
   int* jstate;
   char* jblock;      // block Jacobi state (nmax > 512)
   int i_first, nmax, nchunks_max, nblk_norm;
@@ -233,6 +235,7 @@ ChiLayout chi_layout(Carver& c, int n, int batch, int chi, bool need_psi) {
     L.v = c.take<double2>(nm2 * batch);
     L.w = c.take<double2>(nm2 * batch * (i_first + 1));
     L.part = c.take<double2>(nm2 * batch * L.nchunks_max);
+    if (osj_fits(L.nmax)) L.jrank = c.take<int>(batch);
     if (jacobi_lds_fits(L.nmax)) {
       L.jlog = c.take<double>(jacobi_lds_log_doubles(L.nmax) * batch);
       L.jstate = c.take<int>(2 * static_cast<size_t>(batch));
@@ -257,7 +260,7 @@ struct LayerLayout {
   int* error;
 };
 constexpr int kChain2MaxBlocks = 256;
-constexpr int kJacobiSweeps = 30;   // sweep launches of the LDS Jacobi per bond (16-17 run at 2r = 128)
+constexpr int kJacobiSweeps = 30;   // sweeps for 2r <= 128 (at 2r = 128 one-sided 8 to 10 run, two-sided 16 to 17)
 // sweeps of the block Jacobi (2r > 512): 1 to 34 per bond (16 on average)
 // on the Gram matrices of an N=26 random-MPS state of bond 1024 at chi = 512
 constexpr int kJacobiBlockSweeps = 80;
@@ -564,8 +567,13 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
       if (launch_jacobi_block(L.a, L.v, nm2, L.ncur, nmax, batch, L.jblock, conv.data(), cap(kJacobiBlockSweeps),
                               L.error, st) != 0)
         return fail(h, QMX_ERR_HIP, "block Jacobi");
-    } else if (L.jlog && jacobi_lds_setup(nmax) == hipSuccess) {
+    } else if (h->two_sided && L.jlog && jacobi_lds_setup(nmax) == hipSuccess) {
       launch_jacobi_lds(L.a, L.v, nm2, L.ncur, nmax, batch, L.jlog, L.jstate, cap(kJacobiSweeps), L.error, st);
+    } else if (!h->two_sided && L.jrank) {
+      // (the spectra of bonds that are not truncated are wanted too if any are)
+      if (launch_osj(L.a, L.v, nm2, L.ncur, nmax, batch, spectra ? 0 : chi, L.jrank, cap(kJacobiSweeps), L.error,
+                     st) != 0)
+        return fail(h, QMX_ERR_HIP, "one-sided Jacobi");
     } else {
       launch_jacobi(L.a, L.v, nm2, L.ncur, nmax, batch, cap(kJacobiGlobalSweeps), L.error, st);
     }
@@ -1191,6 +1199,7 @@ void qmx_copy_options(const qmx_handle* from, qmx_handle* to) {
   to->fwd_mfma = from->fwd_mfma;
   to->jacobi_sweep_cap = from->jacobi_sweep_cap;
   to->fail_unitarity = from->fail_unitarity;
+  to->two_sided = from->two_sided;
 }
 
 // =================================================================== C-ABI ==
@@ -1284,6 +1293,11 @@ int qmx_set_option(qmx_handle* h, int option, int value) {
   if (option == QMX_OPT_FAIL_UNITARITY) {
     if (value != 0 && value != 1) return fail(h, QMX_ERR_INVALID, "fail unitarity: 0 or 1");
     h->fail_unitarity = value != 0;
+    return QMX_OK;
+  }
+  if (option == QMX_OPT_TWO_SIDED_JACOBI) {
+    if (value != 0 && value != 1) return fail(h, QMX_ERR_INVALID, "two-sided Jacobi: 0 or 1");
+    h->two_sided = value != 0;
     return QMX_OK;
   }
   if (option == QMX_OPT_SPLIT_SWEEPS) {

@@ -293,12 +293,18 @@ void launch_gram_reduce(const double2* part, int nchunks, const int* ncols_dev, 
 size_t jacobi_block_bytes(int ncols_max, int batch);
 int launch_jacobi_block(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int batch,
                         void* ws, int* conv_host_buf, int max_sweeps, int* error, hipStream_t st);
-// LDS-resident Jacobi for matrices up to 128 x 128 (qmx_linalg.hip)
+// LDS-resident two-sided Jacobi for matrices up to 128 x 128 (qmx_linalg.hip)
 size_t jacobi_lds_log_doubles(int ncols_max);
 bool jacobi_lds_fits(int ncols_max);
 hipError_t jacobi_lds_setup(int ncols_max);
 void launch_jacobi_lds(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max,
                        int batch, double* log, int* state, int max_sweeps, int* error, hipStream_t st);
+// one-sided Jacobi on the pivoted Cholesky factor, up to 128 x 128
+// (qmx_linalg.hip); rank: batch ints of scratch.  Matrices of at most keep_all
+// columns are not truncated and get the identity.  -1 on a HIP failure
+bool osj_fits(int ncols_max);
+int launch_osj(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int batch, int keep_all,
+               int* rank, int max_sweeps, int* error, hipStream_t st);
 void launch_jacobi(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max,
                    int batch, int max_sweeps, int* error, hipStream_t);
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,

@@ -3,7 +3,7 @@
 // Step i of the right-to-left truncated projection chain works on
 // Y_i = X_{i+1} viewed as a (2^i x n_i) row-major complex128 matrix:
 //   rho_i = Y_i^H Y_i             gram + gram_reduce   (n_i x n_i, ld = nmax)
-//   rho_i = V diag(lam) V^H       jacobi               (one block per state)
+//   rho_i = V diag(lam) V^H       one-sided / two-sided / block Jacobi by size
 //   W_i   = V[:, top k_i]         select               (rsum2 cutoff, max bond chi)
 //   X_i   = Y_i W_i               gemm
 // and the state is contracted back with Z_{i+1} = Z_i W_i^H (gemm, conj_b).
@@ -189,6 +189,7 @@ __global__ __launch_bounds__(512) void jacobi_kernel(double2* a_all, double2* v_
 }
 
 // ------------------------------------------------ LDS-resident Jacobi -------
+// QMX_OPT_TWO_SIDED_JACOBI (the one-sided solver below is the default).
 // For n <= kJacobiLdsMax the upper triangle of A (n (n + 1) / 2 complex128,
 // 132 KiB at n = 128) lives in LDS for a whole sweep: one block per state,
 // the same parallel (circle) ordering and rotations as jacobi_kernel.  Each
@@ -419,6 +420,338 @@ __global__ void jacobi_lds_init_kernel(double2* v_all, size_t stride, const int*
 __global__ void jacobi_lds_check_kernel(const int* state, int batch, int* error) {
   const int b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b < batch && !state[b] && error) atomicOr(error, kErrEigNoConv);
+}
+
+// ------------------------------------ one-sided Jacobi on L -----------------
+// Eigensolver for up to 128 columns: one-sided Jacobi on the pivoted Cholesky
+// factor of the Gram matrix.
+//
+//   A = L L^H       pivoted Cholesky (largest remaining diagonal first), cut at
+//                   eps * trace: L has as many columns as A has rank
+//   L J = U S       one-sided Jacobi on L's columns (K. Veselic, V. Hari, "A
+//                   note on a one-sided Jacobi algorithm", Numer. Math. 56
+//                   (1989)): plane rotations from the right until every two
+//                   columns are orthogonal to kOsjTol of their norms
+// The columns of U = (L J) S^{-1} are A's eigenvectors and the squared column
+// norms its eigenvalues; nothing has to be accumulated beside the columns
+// themselves.  The factor of a pivoted Cholesky is graded, which is what makes
+// the rotations converge (8 to 10 sweeps on the chain's matrices, the last of
+// them only checking), and the columns that a rank-deficient Gram matrix does
+// not have (fewer rows than columns left of the chain's centre) are never
+// touched.  Columns dropped at eps * trace get eigenvalue 0 and a zero vector.
+constexpr double kEps = 2.220446049250313e-16;
+// columns p, q are orthogonal when |p^H q| <= kOsjTol |p| |q|: the rounding of
+// a 128-term product is about sqrt(128) eps
+constexpr double kOsjTol = 2e-15;
+
+// The totals over the wave of four per-lane values: row k (lanes 16 k ..
+// 16 k + 15) holds the total of v_k on every lane.  Two half-swaps merge the
+// four registers, then four DPP steps add inside the rows.
+QMX_DEV double swap_add32(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+QMX_DEV double swap_add16(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+QMX_DEV double rows_total(double v0, double v1, double v2, double v3) {
+  return sum16(swap_add16(swap_add32(v0, v2), swap_add32(v1, v3)));
+}
+
+// NR entries of one column: rows lane, lane + 64, ...
+template <int NR> struct Col { double2 v[NR]; };
+
+template <int NR> QMX_DEV double col_norm(const Col<NR>& a) {
+  double s = 0.0;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) s += cabs2(a.v[r]);
+  return s;
+}
+template <int NR> QMX_DEV double2 col_dot(const Col<NR>& a, const Col<NR>& b) {
+  double2 s = cz();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) s = cfmac(a.v[r], b.v[r], s);
+  return s;
+}
+
+// Rotates the four disjoint pairs (p_k, q_k) to orthogonality.  al, be: squared
+// norms of p_k and q_k in row k of the wave, updated.  With g = p^H q and
+// d = |q|^2 - |p|^2 the smaller root of t^2 + t d / |g| - 1 = 0 gives
+//   t e^{i arg g} = te = 2 g sign(d) / (|d| + sqrt(d^2 + 4 |g|^2)),
+//   p' = c (p - conj(te) q),  q' = c (q + te p),  c = 1 / sqrt(1 + |te|^2),
+//   |p'|^2 = |p|^2 - t |g|,  |q'|^2 = |q|^2 + t |g|.
+// The four pairs' parameters are computed once, one pair per row, and read back
+// as scalars.  Returns whether any pair was rotated (uniform over the wave).
+template <int NR>
+QMX_DEV bool rotate4(Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>& p2, Col<NR>& q2, Col<NR>& p3,
+                     Col<NR>& q3, double& al, double& be) {
+  const double2 g0 = col_dot(p0, q0), g1 = col_dot(p1, q1), g2 = col_dot(p2, q2), g3 = col_dot(p3, q3);
+  const double2 g = make_double2(rows_total(g0.x, g1.x, g2.x, g3.x), rows_total(g0.y, g1.y, g2.y, g3.y));
+  const double ag2 = cabs2(g);
+  const bool rot = ag2 > kOsjTol * kOsjTol * al * be && ag2 > 0.0;
+  if (!__any(rot)) return false;
+  const double d = be - al;
+  const double q = fma(4.0, ag2, d * d);
+  double f = 2.0 * rcp_newton(fma(q, rsqrt_newton(q), fabs(d)));
+  f = rot ? (d >= 0.0 ? f : -f) : 0.0;
+  const double2 te = rot ? cscale(g, f) : cz();
+  const double c = rsqrt_newton(1.0 + cabs2(te));
+  const double tg = rot ? ag2 * f : 0.0;
+  al -= tg;
+  be += tg;
+  auto apply = [&](Col<NR>& p, Col<NR>& q, int k) {
+    const double tx = lane_value(te.x, 16 * k), ty = lane_value(te.y, 16 * k), cc = lane_value(c, 16 * k);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const double2 u = p.v[r], w = q.v[r];
+      p.v[r] = make_double2(cc * fma(-tx, w.x, fma(-ty, w.y, u.x)), cc * fma(-tx, w.y, fma(ty, w.x, u.y)));
+      q.v[r] = make_double2(cc * fma(tx, u.x, fma(-ty, u.y, w.x)), cc * fma(tx, u.y, fma(ty, u.x, w.y)));
+    }
+  };
+  apply(p0, q0, 0);
+  apply(p1, q1, 1);
+  apply(p2, q2, 2);
+  apply(p3, q3, 3);
+  return true;
+}
+
+// ------------------------------------------------ up to 128 columns ---------
+// One block per state, the matrix in registers: wave w holds two blocks of 4
+// columns, lane l their rows l (and l + 64).  The blocks are paired by the
+// circle method: nb - 1 rounds of 4 sets of 4 disjoint pairs per sweep, after
+// which every wave passes its blocks on through LDS; at the start of a sweep
+// the pairs inside the blocks are rotated and the norms recomputed.
+// Bound by FP64 issue (per set and wave about 250 instructions, half of them
+// the 12 NR + 4 NR per pair that the rotations and products need) with 3 to 4
+// waves per SIMD, one CU per state.  The truncation chain of 32 states (N=20,
+// chi = 64: ten matrices of 128 columns and rank 96 to 8) spends 13.2 ms here
+// and 1.3 ms in the Cholesky factors; the two-sided Jacobi it replaces, which
+// kept A's triangle in LDS and logged its rotations for a second kernel that
+// accumulated V, spent 62.7 + 16.1 ms (14 sweeps per matrix).
+constexpr int kOsjMax = 128;
+
+// Pivoted Cholesky factor of one state's Gram matrix (n <= 128): thread (row,
+// g) holds columns 16 g .. 16 g + 15 of its row in registers, and every step
+// subtracts the outer product of the new column.  Column k of L goes to
+// a + k ld (A's own storage), L's column count to rank[b]; -1 for a matrix that
+// is zero, not finite, or not truncated at all (n <= keep_all), which stays as
+// it is.  Bound by the two barriers and the pivot search per step.
+__global__ __launch_bounds__(1024) void chol_kernel(double2* a_all, size_t stride, const int* ncols_dev, int ld,
+                                                    int keep_all, int* rank_out) {
+  __shared__ double2 lcol[kOsjMax];
+  __shared__ int s_p;
+  __shared__ double s_d;
+  const int b = blockIdx.x;
+  const int n = ncols_dev[b];
+  double2* a = a_all + (size_t)b * stride;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row = tid & (kOsjMax - 1), g = wave >> 1;
+  if (n <= keep_all) {
+    if (tid == 0) rank_out[b] = -1;
+    return;
+  }
+  // a column of the Hermitian matrix is its conjugated row: contiguous loads
+  double2 x[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const int col = 16 * g + c;
+    x[c] = col < n && row < n ? cconj(a[(size_t)col * ld + row]) : cz();
+  }
+  // wave 0: the remaining diagonal of columns lane, lane + 64
+  double d0 = lane < n ? a[(size_t)lane * ld + lane].x : 0.0;
+  double d1 = lane + 64 < n ? a[(size_t)(lane + 64) * ld + lane + 64].x : 0.0;
+  const double tr = wave_sum(d0 + d1);
+  if (!(tr > 0.0) || !(tr < 1e300)) {
+    if (tid == 0) rank_out[b] = -1;
+    return;
+  }
+  if (lane >= n) d0 = -1.0;
+  if (lane + 64 >= n) d1 = -1.0;
+  __syncthreads();   // A is in registers: its storage takes L
+  unsigned done = 0;
+  bool used = false;
+  int rank = 0;
+  for (; rank < n; ++rank) {
+    if (wave == 0) {
+      // largest remaining diagonal entry, lowest index on ties
+      double best = d1 > d0 ? d1 : d0;
+      int p = d1 > d0 ? lane + 64 : lane;
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) {
+        const double o = __shfl_xor(best, m, 64);
+        const int op = __shfl_xor(p, m, 64);
+        if (o > best || (o == best && op < p)) {
+          best = o;
+          p = op;
+        }
+      }
+      if (lane == 0) {
+        s_p = best > kEps * tr ? p : -1;
+        s_d = best;
+      }
+    }
+    __syncthreads();
+    const int p = __builtin_amdgcn_readfirstlane(s_p);
+    if (p < 0) break;
+    if (g == (p >> 4)) {
+      double2 t = cz();
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        if (c == (p & 15)) t = x[c];
+      const double d = s_d, inv = rsqrt_newton(d);
+      t = used ? cz() : (row == p ? make_double2(d * inv, 0.0) : cscale(t, inv));
+      lcol[row] = t;
+      if (row < n) a[(size_t)rank * ld + row] = t;
+      done |= 1u << (p & 15);
+    }
+    __syncthreads();
+    const double2 l = lcol[row];
+    if (row == p) used = true;
+#pragma unroll
+    for (int c = 0; c < 16; ++c)
+      if (!((done >> c) & 1u)) {
+        const double2 lc = lcol[16 * g + c];   // x -= l conj(l_c)
+        x[c].x = fma(-l.x, lc.x, fma(-l.y, lc.y, x[c].x));
+        x[c].y = fma(-l.y, lc.x, fma(l.x, lc.y, x[c].y));
+      }
+    if (wave == 0) {
+      d0 = lane == p ? -1.0 : d0 - cabs2(lcol[lane]);
+      d1 = lane + 64 == p ? -1.0 : d1 - cabs2(lcol[lane + 64]);
+    }
+  }
+  if (tid == 0) rank_out[b] = rank;
+}
+
+template <int NR>
+__global__ __launch_bounds__(NR == 2 ? 1024 : 512) void osj_kernel(double2* a_all, double2* v_all, size_t stride,
+                                                                   const int* ncols_dev, int ld,
+                                                                   const int* rank_in, int max_sweeps, int* error) {
+  constexpr int kRows = 64 * NR;
+  extern __shared__ double2 xbuf[];                   // W + 1 slots of 4 columns
+  __shared__ double nbuf[17][4];
+  const int b = blockIdx.x;
+  const int n = ncols_dev[b], rank = rank_in[b];
+  double2* a = a_all + (size_t)b * stride;
+  double2* v = v_all + (size_t)b * stride;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (rank < 0) {   // any unitary basis will do; the diagonal stays as it is
+    for (int e = tid; e < n * n; e += blockDim.x) {
+      const int i = e / n, j = e % n;
+      v[(size_t)i * ld + j] = make_double2(i == j ? 1.0 : 0.0, 0.0);
+    }
+    return;
+  }
+  Col<NR> x[8];
+  const int nb = ((rank + 3) / 4 + 1) & ~1;   // blocks of 4, an even number
+  const int m = nb / 2;                       // waves with columns
+  const int tb = 4 * wave, bb = 4 * (nb - 1 - wave);   // first columns of this wave's blocks
+  const bool live = wave < m;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      const int k = c < 4 ? tb + c : bb + c - 4, row = lane + 64 * r;
+      x[c].v[r] = live && k < rank && row < n ? a[(size_t)k * ld + row] : cz();
+    }
+  __syncthreads();   // L is in registers: A's storage takes the eigenvalues
+  // ---- one-sided Jacobi sweeps: x[0..3] the top block, x[4..7] the bottom one
+  auto slot = [&](int s) { return xbuf + (size_t)s * 4 * kRows; };
+  auto put = [&](int s, int c0, double nrm) {
+    double2* t = slot(s);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) t[c * kRows + lane + 64 * r] = c0 ? x[4 + c].v[r] : x[c].v[r];
+    if ((lane & 15) == 0) nbuf[s][lane >> 4] = nrm;
+  };
+  auto get = [&](int s, int c0, double& nrm) {
+    const double2* t = slot(s);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int r = 0; r < NR; ++r) {
+        const double2 w = t[c * kRows + lane + 64 * r];
+        if (c0) x[4 + c].v[r] = w;
+        else x[c].v[r] = w;
+      }
+    nrm = nbuf[s][lane >> 4];
+  };
+  bool converged = false;
+  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    bool rot = false;
+    double nt = 0.0, nq = 0.0;   // squared norms: row k of the wave, column k of the top / bottom block
+    if (live) {
+      auto inside = [&](Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>& p2, Col<NR>& q2, Col<NR>& p3,
+                        Col<NR>& q3) {
+        double al = rows_total(col_norm(p0), col_norm(p1), col_norm(p2), col_norm(p3));
+        double be = rows_total(col_norm(q0), col_norm(q1), col_norm(q2), col_norm(q3));
+        rot |= rotate4(p0, q0, p1, q1, p2, q2, p3, q3, al, be);
+      };
+      inside(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
+      inside(x[0], x[2], x[1], x[3], x[4], x[6], x[5], x[7]);
+      inside(x[0], x[3], x[1], x[2], x[4], x[7], x[5], x[6]);
+      nt = rows_total(col_norm(x[0]), col_norm(x[1]), col_norm(x[2]), col_norm(x[3]));
+      nq = rows_total(col_norm(x[4]), col_norm(x[5]), col_norm(x[6]), col_norm(x[7]));
+    }
+    for (int round = 0; round < nb - 1; ++round) {
+      if (live) {
+        // set s: pairs (top k, bottom (k + s) % 4); the bottom norms move up one row per set
+        auto next = [&]() { nq = __shfl(nq, (lane + 16) & 63, 64); };
+        rot |= rotate4(x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7], nt, nq);
+        next();
+        rot |= rotate4(x[0], x[5], x[1], x[6], x[2], x[7], x[3], x[4], nt, nq);
+        next();
+        rot |= rotate4(x[0], x[6], x[1], x[7], x[2], x[4], x[3], x[5], nt, nq);
+        next();
+        rot |= rotate4(x[0], x[7], x[1], x[4], x[2], x[5], x[3], x[6], nt, nq);
+        next();
+      }
+      if (m == 1) continue;   // two blocks: the only pair
+      // circle: top 0 stays, top w goes to top w + 1, the last top to the last
+      // bottom, bottom w to bottom w - 1, bottom 0 to top 1.  Tops first, then
+      // bottoms; the last top waits in its slot, so the last bottom uses slot m.
+      if (live && wave > 0) put(wave, 0, nt);
+      __syncthreads();
+      if (live && wave > 1) get(wave - 1, 0, nt);
+      __syncthreads();
+      if (live) put(wave == m - 1 ? m : wave, 1, nq);
+      __syncthreads();
+      if (live) {
+        if (wave == 1) get(0, 0, nt);
+        get(wave == m - 1 ? m - 1 : (wave + 1 == m - 1 ? m : wave + 1), 1, nq);
+      }
+      __syncthreads();
+    }
+    if (!__syncthreads_or(rot ? 1 : 0)) {
+      converged = true;
+      break;
+    }
+  }
+  if (!converged && tid == 0 && error) atomicOr(error, kErrEigNoConv);
+  // eigenvalues to A's diagonal, eigenvectors to V; the dropped columns are zero
+  const double nt = rows_total(col_norm(x[0]), col_norm(x[1]), col_norm(x[2]), col_norm(x[3]));
+  const double nq = rows_total(col_norm(x[4]), col_norm(x[5]), col_norm(x[6]), col_norm(x[7]));
+  if (live) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int k = c < 4 ? tb + c : bb + c - 4;
+      const double nn = lane_value(c < 4 ? nt : nq, 16 * (c & 3));
+      const double inv = nn > 0.0 ? rsqrt_newton(nn) : 0.0;
+      if (k < n) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r)
+          if (lane + 64 * r < n) v[(size_t)(lane + 64 * r) * ld + k] = cscale(x[c].v[r], inv);
+        if (lane == 0) a[(size_t)k * ld + k] = make_double2(nn, 0.0);
+      }
+    }
+  }
+  for (int k = 4 * nb + wave; k < n; k += blockDim.x >> 6) {
+    for (int row = lane; row < n; row += 64) v[(size_t)row * ld + k] = cz();
+    if (lane == 0) a[(size_t)k * ld + k] = cz();
+  }
 }
 
 // ------------------------------------------------ circle ordering --------
@@ -702,6 +1035,12 @@ __global__ __launch_bounds__(512) void select_kernel(const double2* a_all, const
   const double2* a = a_all + (size_t)b * stride;
   const double2* v = v_all + (size_t)b * stride;
   double2* w = w_all + (size_t)b * stride;
+  // (entries that are not numbers have no rank: perm stays in range for them)
+  for (int j = threadIdx.x; j < n; j += blockDim.x) {
+    lam[j] = 0.0;
+    perm[j] = j;
+  }
+  __syncthreads();
   for (int j = threadIdx.x; j < n; j += blockDim.x) {
     double lj = a[(size_t)j * ld + j].x;
     int rank = 0;
@@ -921,6 +1260,31 @@ hipError_t jacobi_lds_setup(int ncols_max) {
   const size_t tri_bytes = sizeof(double2) * (size_t)kJacobiLdsMax * (kJacobiLdsMax + 1) / 2;
   return hipFuncSetAttribute(reinterpret_cast<const void*>(jacobi_lds_sweep_kernel),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_bytes);
+}
+
+bool osj_fits(int ncols_max) { return ncols_max >= 1 && ncols_max <= kOsjMax; }
+
+int launch_osj(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int batch, int keep_all,
+               int* rank, int max_sweeps, int* error, hipStream_t st) {
+  const int waves = (ncols_max + 7) / 8;
+  // the dynamic-LDS limit is set to the largest need (16 waves), whatever this
+  // call needs, so that launches from several host threads never lower it
+  const size_t most = (size_t)17 * 4 * 128 * sizeof(double2);
+  if (ncols_max > 64 && hipFuncSetAttribute(reinterpret_cast<const void*>(osj_kernel<2>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)most) != hipSuccess)
+    return -1;
+  hipLaunchKernelGGL(chol_kernel, dim3(batch), dim3(1024), 0, st, a, stride, ncols_dev, ncols_max, keep_all, rank);
+  if (ncols_max <= 64) {
+    // at most 9 slots of 4 KiB: below the default limit
+    const size_t shm = (size_t)(waves + 1) * 4 * 64 * sizeof(double2);
+    hipLaunchKernelGGL(osj_kernel<1>, dim3(batch), dim3(64 * waves), shm, st, a, v, stride, ncols_dev, ncols_max,
+                       rank, max_sweeps, error);
+  } else {
+    const size_t shm = (size_t)(waves + 1) * 4 * 128 * sizeof(double2);
+    hipLaunchKernelGGL(osj_kernel<2>, dim3(batch), dim3(64 * waves), shm, st, a, v, stride, ncols_dev, ncols_max,
+                       rank, max_sweeps, error);
+  }
+  return 0;
 }
 
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,

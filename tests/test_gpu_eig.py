@@ -1,0 +1,93 @@
+"""The chi-truncation's one-sided Jacobi at the edges of its sizes and ranks.
+
+Column counts n = 2 chi around 8 (one wave), 64 and 128 (its limits), with
+Gram matrices of full rank, of fewer rows than columns, and with clusters of
+equal eigenvalues.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import qmprs_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _engine():
+    from qmprs_amd import engine
+    return engine
+
+
+@pytest.mark.parametrize("n,chi", [(6, 1), (7, 2), (8, 3), (8, 4), (9, 5), (11, 31), (11, 32), (12, 33), (13, 63),
+                                   (14, 64)])
+@pytest.mark.parametrize("kind", ["uniform", "mps"])
+def test_truncation_edges(gpu, n, chi, kind):
+    """Targets to 1e-10 and spectra to 1e-12 of the largest eigenvalue (the
+    suite's bars for the truncation): a batch of three states, of which the
+    oracle truncates each by itself."""
+    eng = _engine()
+    svs = [O.random_uniform_state(n, s) if kind == "uniform" else O.random_mps_state(n, max(2, chi + chi // 2), s)
+           for s in (1, 2, 3)]
+    _, target, spec = eng.chi_truncate(eng.as_device_states(np.stack(svs)), chi, spectra=True)
+    _, plain, _ = eng.chi_truncate(eng.as_device_states(np.stack(svs)), chi)
+    for k, sv in enumerate(svs):
+        ref, ref_spec = O.chi_truncate(O.ket(sv), n, chi)
+        for got in (target, plain):
+            err = np.linalg.norm(got[k].cpu().numpy() - ref) / np.linalg.norm(ref)
+            print(f"n={n} chi={chi} {kind} state {k} rel.err {err:.2e}")
+            assert err < 1e-10
+        for i, lam in enumerate(ref_spec):
+            if lam is not None:
+                kk = min(len(lam), chi)
+                assert np.max(np.abs(spec[k, i, :kk].cpu().numpy() - lam[:kk])) < 1e-12 * lam[0]
+
+
+@pytest.mark.parametrize("pairs,chi", [(4, 16), (5, 32), (6, 64)])
+def test_equal_eigenvalues(gpu, pairs, chi):
+    """Bell pairs across the centre plus noise below the cutoff: 2^pairs equal
+    eigenvalues at the middle bond, all kept, so the truncation returns the
+    state (the cutoff of 1e-10 drops at most that weight at each of the bonds;
+    the noise has 1e-16)."""
+    eng = _engine()
+    n = 2 * pairs
+    psi = np.zeros((2 ** pairs, 2 ** pairs), dtype=np.complex128)
+    psi[np.arange(2 ** pairs), np.arange(2 ** pairs)] = 2.0 ** (-pairs / 2)
+    rng = np.random.default_rng(pairs)
+    noise = rng.standard_normal(psi.shape) + 1j * rng.standard_normal(psi.shape)
+    psi = O.ket((psi + 1e-8 * noise / np.linalg.norm(noise)).reshape(-1))
+    wide = np.kron(psi, np.array([1.0, 1.0]) / np.sqrt(2.0))   # one more site: bonds above chi columns
+    for sv, m in ((psi, n), (wide, n + 1)):
+        _, target, _ = eng.chi_truncate(eng.as_device_states(sv), chi)
+        assert np.linalg.norm(target[0].cpu().numpy() - sv) < 1e-7, m
+
+
+def test_state_that_is_not_a_number_stays_alone(gpu):
+    eng = _engine()
+    sv = np.stack([O.random_uniform_state(9, s) for s in (4, 5, 6)])
+    _, ref, _ = eng.chi_truncate(eng.as_device_states(sv), 8)
+    bad = sv.copy()
+    bad[1, 3] = np.nan
+    _, got, _ = eng.chi_truncate(eng.as_device_states(bad), 8)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[2], ref[2])
+    assert not bool(torch.isfinite(torch.view_as_real(got[1])).all())
+
+
+def test_two_sided_option(gpu):
+    """QMX_OPT_TWO_SIDED_JACOBI changes the truncation by rounding only (1e-10,
+    the suite's bar); MPS truncates with it and leaves the option as it was."""
+    from qmprs_amd import _lib
+    from qmprs_amd.primitives import MPS
+    eng = _engine()
+    sv = O.random_mps_state(13, 48, 9)
+    dev = eng.as_device_states(sv)
+    _, one, _ = eng.chi_truncate(dev, 32)
+    with _lib.two_sided_jacobi():
+        _, two, _ = eng.chi_truncate(dev, 32)
+    mps = MPS(sv, bond_dimension=32)
+    assert torch.equal(mps.state, two)
+    _, again, _ = eng.chi_truncate(dev, 32)
+    assert torch.equal(one, again)
+    assert float(torch.linalg.vector_norm(one - two) / torch.linalg.vector_norm(two)) < 1e-10
+    with pytest.raises(ValueError):
+        _lib.set_option(_lib.QMX_OPT_TWO_SIDED_JACOBI, 2)
