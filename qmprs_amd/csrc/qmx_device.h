@@ -214,10 +214,8 @@ QMX_DEV double dpp(double v) {
   const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
-template <int CTRL>
-QMX_DEV double2 dpp2(double2 v) { return make_double2(dpp<CTRL>(v.x), dpp<CTRL>(v.y)); }
-constexpr int kDppRow1 = 0x12c, kDppRow2 = 0x128, kDppRow3 = 0x124;   // matrix row (i + 1, 2, 3) % 4
-constexpr int kDppCol1 = 0x39, kDppCol2 = 0x4e, kDppCol3 = 0x93;      // matrix column (j + 1, 2, 3) % 4
+constexpr int kDppRow1 = 0x12c, kDppRow2 = 0x128, kDppRow3 = 0x124;   // lane + 4, 8, 12 of the 16
+constexpr int kDppCol2 = 0x4e;                                         // matrix column (j + 2) % 4
 constexpr int kDppSwap = 0xb1;                                         // column j ^ 1
 
 // sum over the 16 lanes (both partners add the same two values at every
@@ -229,31 +227,9 @@ QMX_DEV double sum16(double v) {
   v += dpp<kDppSwap>(v);
   return v;
 }
-// sum over the 4 rows of a column
-QMX_DEV double sumcol(double v) {
-  v += dpp<kDppRow2>(v);
-  v += dpp<kDppRow1>(v);
-  return v;
-}
 QMX_DEV double lane_value(double v, int lane) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-QMX_DEV double2 lane_value2(double2 v, int lane) { return make_double2(lane_value(v.x, lane), lane_value(v.y, lane)); }
-
-// Cofactor of entry (i, j): rows and columns taken cyclically after i and j
-// (a cyclic shift of three is an even permutation), sign (-1)^(i + j).
-QMX_DEV double2 cofactor4(double2 m, int l) {
-  const double2 a0 = dpp2<kDppRow1>(m), b0 = dpp2<kDppRow2>(m), c0 = dpp2<kDppRow3>(m);
-  const double2 a1 = dpp2<kDppCol1>(a0), a2 = dpp2<kDppCol2>(a0), a3 = dpp2<kDppCol3>(a0);
-  const double2 b1 = dpp2<kDppCol1>(b0), b2 = dpp2<kDppCol2>(b0), b3 = dpp2<kDppCol3>(b0);
-  const double2 c1 = dpp2<kDppCol1>(c0), c2 = dpp2<kDppCol2>(c0), c3 = dpp2<kDppCol3>(c0);
-  auto minor = [](double2 p, double2 q, double2 r, double2 s) { return csub(cmul(p, s), cmul(q, r)); };
-  double2 c = cmul(a1, minor(b2, b3, c2, c3));
-  c = csub(c, cmul(a2, minor(b1, b3, c1, c3)));
-  c = cfma(a3, minor(b1, b2, c1, c2), c);
-  const double s = ((l ^ (l >> 2)) & 1) ? -1.0 : 1.0;
-  return cscale(c, s);
 }
 
 // 1 / x to rounding: the hardware estimate and two Newton steps
@@ -271,108 +247,76 @@ QMX_DEV double rsqrt_newton(double x) {
   return fma(r, fma(-h * r, r, 0.5), r);
 }
 
-// conj(X^{-1}[j][i]) at lane (i, j), by Gauss-Jordan exchange steps with row
-// pivoting (largest |entry| of the column among the rows not used yet, first
-// on ties).  Rows stay in place: after step k row p_k stands for unknown k and
-// column k for equation p_k, so X^{-1}[a][b] = M[p_a][l] with p_l = b.
-// False (on every lane) for a zero pivot or a non-finite result.
-QMX_DEV bool inv4_wave(double2 m, int l, double2& out) {
-  const int i = (l >> 2) & 3, j = l & 3;
-  int pj = 0, qi = 0;       // p_j and the l with p_l = i
-  unsigned used = 0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    double2 f;
-    f = k == 0 ? dpp2<0x00>(m) : (k == 1 ? dpp2<0x55>(m) : (k == 2 ? dpp2<0xaa>(m) : dpp2<0xff>(m)));   // X[i][k]
-    const double c = cabs2(f);
-    int p = -1;
-    double best = 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const double v = lane_value(c, 4 * r);
-      if (!((used >> r) & 1u) && v > best) {
-        best = v;
-        p = r;
-      }
-    }
-    if (p < 0) return false;
-    p = __builtin_amdgcn_readfirstlane(p);
-    used |= 1u << p;
-    if (j == k) pj = p;
-    if (i == p) qi = k;
-    const double2 rk = make_double2(__shfl(m.x, 4 * p + j, 16), __shfl(m.y, 4 * p + j, 16));   // X[p][j]
-    const double2 piv = lane_value2(m, 4 * p + k);
-    const double ib = rcp_newton(best);
-    const double2 ip = make_double2(piv.x * ib, -piv.y * ib);   // 1 / pivot
-    const double2 rkj = cmul(j == k ? make_double2(1.0, 0.0) : rk, ip);
-    m = (i == p) ? rkj : csub(j == k ? cz() : m, cmul(f, rkj));
-  }
-  const int src = 4 * pj + qi;
-  out = make_double2(__shfl(m.x, src, 16), -__shfl(m.y, src, 16));
-  return sum16(cabs2(m)) < 1e300;   // false for inf / nan
+// ---- 4 x 4 complex products on the matrix cores --------------------------------
+// v_mfma_f64_4x4x4_4b: four 4 x 4 products at once, operands A[i][k] in lane
+// i + 4 blk + 16 k, B[k][j] in lane j + 4 blk + 16 k, result D[i][j] in lane
+// j + 4 blk + 16 i (checked on gfx950).  A complex matrix M is held in the
+// result's layout, real parts in the even blocks and imaginary parts in the odd
+// ones (v, the two pairs of blocks alike), with the other part beside it (o).
+// As an A operand this layout reads as the transpose.
+struct Mat4 {
+  double v, o;
+};
+QMX_DEV Mat4 mat4(double v) { return {v, dpp<kDppRow3>(v)}; }   // row_ror:4: the block before
+// M^T B, or M^H B with CONJ
+template <bool CONJ>
+QMX_DEV double mat4_tmul(Mat4 m, Mat4 b, bool even) {
+  const double re = even ? m.v : m.o;
+  const double im = CONJ ? (even ? m.o : -m.v) : (even ? -m.o : m.v);
+  const double d = __builtin_amdgcn_mfma_f64_4x4x4f64(re, b.v, 0.0, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(im, b.o, d, 0, 0, 0);
 }
 
-// Unitary polar factor of a nonsingular 4 x 4 matrix by the scaled Newton
-// iteration (N. J. Higham, "Computing the polar decomposition -- with
-// applications", SIAM J. Sci. Stat. Comput. 7 (1986)); x is this lane's entry,
-// the factor's on a true return:
-//   X_{k+1} = (z X_k + X_k^{-H} / z) / 2,  z = (||X_k^{-1}||_F / ||X_k||_F)^{1/2},
-// which converges quadratically.  With P = |X|_F^2 |X^{-1}|_F^2, 16 for a
-// multiple of a unitary, the singular values s of z X satisfy
-// sum (s - 1/s)^2 = 2 sqrt(P) - 8: a step with P <= 16 + 3.2e-7 leaves them
-// within 1e-8 of 1, and one more step, with z = 1, within rounding.  False, with x unspecified,
-// for an ill-conditioned matrix (P > 1e12 at the start), a failed inverse, or
-// no convergence in 40 steps.  The inverse comes from cofactors, 1 / det times
-// one 3 x 3 minor per lane with no serial pivots, once |det| says that no
-// cancellation can matter: normalised by (|X|_F / 2)^4 it is 1 for a multiple
-// of a unitary, and below kPolarDetMin the step takes the pivoted inverse.
-// On the sweeps' environments (condition numbers 5 to 90 at the median) 0.2 to
-// 1.0 of the 5 to 6 steps are pivoted.  z only has to be close to the optimal
-// scaling and comes from FP32 estimates; 1 / z is its inverse to rounding.
-// Bound by the latency of its dependent FP64 chain: 6700 cycles for a
-// Gaussian 4 x 4 matrix, 10500 at condition number 100 to 1000 (one pivoted
-// step), where one 16-lane pivoted inverse per step through ds_bpermute took
-// 24100 and 26600.
-constexpr double kPolarDetMin = 0.05;
-
-QMX_DEV bool polar4_newton_wave(double2& x, int l) {
-  bool last = false;
-  for (int it = 0; it < 40; ++it) {
-    const double2 c = cofactor4(x, l);
-    const double nx = sum16(cabs2(x)), nc = sum16(cabs2(c));
-    double2 d = cmul(x, c);
-    d.x += dpp<kDppCol2>(d.x);
-    d.y += dpp<kDppCol2>(d.y);
-    d.x += dpp<kDppSwap>(d.x);
-    d.y += dpp<kDppSwap>(d.y);
-    d = lane_value2(d, 0);                      // det X
-    const double ad = cabs2(d);
-    const double q = 0.0625 * nx * nx;          // (|X|_F / 2)^4
-    double2 b;                                  // conj(X^{-1}[j][i])
-    double ni;                                  // |X^{-1}|_F^2
-    if (ad >= kPolarDetMin * kPolarDetMin * q * q) {
-      // conj(C / det) = conj(C) det / |det|^2
-      const double r = rcp_newton(ad);
-      ni = nc * r;
-      b = cscale(cmulc(c, d), r);
-    } else {
-      if (!inv4_wave(x, l, b)) return false;
-      ni = sum16(cabs2(b));
-      if (it == 0 && !(nx * ni <= 1e12)) return false;
+// Unitary polar factor of es 2^h (|.|_F^2 = fro, near 1) by the scaled
+// Newton-Schulz iteration
+//   X <- X (a - b X^H X),  a = 3 s / 2,  b = s^3 / 2,
+// two products per step, on one wave.  It maps a singular value x <= 1 to
+// f(s x) <= 1, f(y) = y (3 - y^2) / 2, and with s^2 = 3 / (1 + l + l^2) the
+// interval [l, 1] to [f(s l), 1], the best a cubic can do (J. Chen, E. Chow, "A
+// stable scaling of Newton-Schulz for improving the sign function computation
+// of a Hermitian matrix", 2014).  Six steps are scaled for l = 0.05, then s = 1,
+// which gains a factor of 1.5 per step on a value that is still small and ends
+// quadratically: once |X^H X - 1| <= 3e-9 in every entry the next step is exact
+// to rounding.  On the sweeps' environments (condition numbers 5 to 90 at the
+// median, 1e3 to 1e4 at the 90th percentile) that takes 8 to 14 steps on
+// average.  The transpose of X is carried along as the left operand.
+// Bound by the latency of the two products, about 300 cycles per step: 3700
+// cycles for a Gaussian 4 x 4 matrix, 4900 at condition number 1000.  The scaled
+// Newton iteration took 24000 and 27000 with its pivoted inverse by ds_bpermute,
+// 6700 and 10500 with an inverse from cofactors by DPP moves.  Error against
+// 80-bit arithmetic: within 1.6 times that of the Newton iteration (both a few
+// 1e-16 times the condition number over 5).
+// u: this lane's part of the factor in the split layout.  False after 34
+// unscaled steps (a condition number above about 1e6).
+QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane, Mat4& u) {
+  const int i = lane >> 4, j = lane & 3;
+  const bool even = !(lane & 4);
+  const double r = rsqrt_newton(fro);
+  const double2 e = es[4 * i + j], t = es[4 * j + i];
+  Mat4 x = mat4(ldexp(even ? e.x : e.y, h) * r), xt = mat4(ldexp(even ? t.x : t.y, h) * r);
+  const double one = even && i == j ? 1.0 : 0.0;
+  auto step = [&](double a, double b, double y) {
+    const Mat4 p = mat4(fma(-b, y, a * one));
+    const double xn = mat4_tmul<false>(xt, p, even);
+    const double tn = mat4_tmul<false>(p, xt, even);
+    x = mat4(xn);
+    xt = mat4(tn);
+  };
+  auto gram = [&]() { return mat4_tmul<true>(x, x, even); };
+  step(2.5324497354750872, 2.406128014703171, gram());   // l = 0.05
+  step(2.430892812235437, 2.128107957418897, gram());    // 0.1263
+  step(2.200129819325986, 1.5777607537549168, gram());   // 0.3028
+  step(1.832672820412407, 0.9119080391587333, gram());   // 0.6224
+  step(1.5614350757473685, 0.5639856062462636, gram());  // 0.9208
+  step(1.5019149323066294, 0.5019173779907503, gram());  // 0.9974
+  for (int it = 0; it < 34; ++it) {
+    const double y = gram();
+    const bool last = __all(fabs(y - one) <= 3e-9);
+    step(1.5, 0.5, y);
+    if (last) {
+      u = x;
+      return true;
     }
-    const double p = nx * ni;
-    double z = 0.5, zi = 0.5;
-    if (!last) {
-      const float s = __builtin_amdgcn_sqrtf(__builtin_amdgcn_sqrtf((float)ni * __builtin_amdgcn_rcpf((float)nx)));
-      z = (double)s;
-      zi = (double)__builtin_amdgcn_rcpf(s);
-      zi = fma(fma(-z, zi, 1.0), zi, zi);
-      zi = 0.5 * fma(fma(-z, zi, 1.0), zi, zi);
-      z *= 0.5;
-    }
-    x = make_double2(fma(z, x.x, zi * b.x), fma(z, x.y, zi * b.y));
-    if (last) return true;
-    last = p <= 16.0 + 3.2e-7;
   }
   return false;
 }
@@ -405,16 +349,9 @@ QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc)
 // whose right singular vectors are e_{z_1}, e_{z_2}, take the rule's left
 // completion, the first unit vectors with a residual above 1/2 (which one
 // pass of Gram-Schmidt then gives to rounding): 5300 cycles, against 30600 by
-// the Jacobi path.  x: this lane's entry of E,
-// es 2^-h: all 16, fro: |x|^2, near 1.  False if E is not of this kind.
-QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, double fro, double* nuc) {
-  const double cn = sumcol(cabs2(x));
-  unsigned zero = 0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (lane_value(cn, j) <= 1e-28 * fro) zero |= 1u << j;
-  zero = __builtin_amdgcn_readfirstlane(zero);
-  if (__popc(zero) != 2) return false;
+// the Jacobi path.  zero: the columns that are (bits), es 2^h: the matrix, fro:
+// its squared norm, near 1; lane l < 16 of x gets entry l.
+QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, unsigned zero, double fro, double* nuc) {
   const unsigned live = ~zero & 15u;
   const int c0 = __ffs(live) - 1, c1 = 31 - __clz(live), z0 = __ffs(zero) - 1, z1 = 31 - __clz(zero);
   // every lane holds the whole 4 x 2 problem
@@ -497,23 +434,25 @@ QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, dou
   return true;
 }
 
-// Polar factor of the d x d matrix in es (LDS, stride 4) on one wave; lane l
-// returns entry l & 15 in x (zero outside the d x d block) and the sum of the
-// singular values.  False: the matrix is left to polar4_jacobi.
-QMX_DEV bool polar4_wave(int d, const double2* es, double2& x, int lane, double* nuc) {
+// Polar factor of the d x d matrix in es (LDS, stride 4, zero outside the
+// block) on one wave, to out (LDS; imaginary parts times sgn).  *nuc: the sum of
+// the singular values, if wanted.  False: the matrix is left to polar4_jacobi.
+QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int lane, bool want, double* nuc) {
   const int l = lane & 15, i = l >> 2, j = l & 3;
-  const bool in = i < d && j < d;
-  const double2 e = in ? es[l] : cz();
-  double fro = sum16(cabs2(e));
+  const double2 e = es[l];
+  const double n2 = cabs2(e);
+  double fro = sum16(n2);
   if (!(fro > 1e-280) || !(fro < 1e280)) return false;
-  // exact scaling by a power of two to |x|^2 in [1/2, 2)
+  // exact scaling by a power of two to a squared norm in [1/2, 2)
   const int h = -(__builtin_amdgcn_frexp_exp(fro) >> 1);
-  x = make_double2(ldexp(e.x, h), ldexp(e.y, h));
-  fro = ldexp(fro, 2 * h);
-  bool ok;
+  double2 x;
   double s = 0.0;
   if (d == 2) {
-    double2 a = lane_value2(x, 0), b = lane_value2(x, 1), c = lane_value2(x, 4), f = lane_value2(x, 5);
+    auto at = [&](int k) {
+      const double2 v = es[k];
+      return make_double2(ldexp(v.x, h), ldexp(v.y, h));
+    };
+    double2 a = at(0), b = at(1), c = at(4), f = at(5);
     const double n0 = cabs2(a) + cabs2(c), n1 = cabs2(b) + cabs2(f);
     if (n1 <= 1e-28 * n0) {
       // the site is still in |0>: one column, completed as in polar4_jacobi
@@ -529,21 +468,37 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2& x, int lane, double*
       const double q = rsqrt_newton(cabs2(b) + cabs2(f));
       b = cscale(b, q);
       f = cscale(f, q);
-      ok = true;
-    } else {
-      ok = polar2(a, b, c, f, &s);
+    } else if (!polar2(a, b, c, f, &s)) {
+      return false;
     }
     x = i == 0 ? (j == 0 ? a : b) : (j == 0 ? c : f);
-    if (!in) x = cz();
-  } else if (polar4_two_columns(x, l, es, h, fro, &s)) {
-    ok = true;
-  } else {
-    const double2 y = x;
-    ok = polar4_newton_wave(x, l);
-    if (ok) s = sum16(x.x * y.x + x.y * y.y);   // Re tr(U^H E)
+    if (i > 1 || j > 1) x = cz();
+    if (lane < 16) out[l] = make_double2(x.x, sgn * x.y);
+    *nuc = ldexp(s, -h);
+    return true;
   }
-  *nuc = ldexp(s, -h);
-  return ok;
+  // columns with an entry above 1e-14 of the norm
+  const unsigned long long big = __ballot(n2 > 1e-28 * fro);
+  unsigned zero = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (!(big & (0x1111ull << k))) zero |= 1u << k;
+  fro = ldexp(fro, 2 * h);
+  if (__popc(zero) == 2) {
+    if (!polar4_two_columns(x, l, es, h, zero, fro, &s)) return false;
+    if (lane < 16) out[l] = make_double2(x.x, sgn * x.y);
+    *nuc = ldexp(s, -h);
+    return true;
+  }
+  Mat4 u;
+  if (!polar4_newton_schulz(es, h, fro, lane, u)) return false;
+  if (!(lane & 12)) out[4 * (lane >> 4) + (lane & 3)] = make_double2(u.v, sgn * u.o);
+  if (want) {   // Re tr(U^H E)
+    __builtin_amdgcn_wave_barrier();
+    const double2 g = out[l];
+    *nuc = sum16(g.x * e.x + sgn * g.y * e.y);
+  }
+  return true;
 }
 
 // Unitary polar factor U V^H of the d x d (d = 2 or 4) matrix e (row-major,
@@ -697,38 +652,36 @@ QMX_DEV void polar4_jacobi(int d, const double2* e, double2* out, double* nuc) {
 // back onto the unitaries.  es, g_old, rm (scratch) and g_new hold 16 entries
 // each in LDS and are used by this wave alone until the caller's barrier.
 // Returns the overlap after the update, the sum of E's singular values or
-// |sum_{o,i} g[o][i] E[o][i]| (on every lane).
+// |sum_{o,i} g[o][i] E[o][i]| (on every lane), if wanted.
 QMX_DEV double update_gate_wave(int d, double omega_m1, const double2* g_old, const double2* es, double2* rm,
-                                double2* g_new, int lane) {
+                                double2* g_new, int lane, bool want) {
   const int l = lane & 15;
-  const bool in = (l >> 2) < d && (l & 3) < d;
   const int rounds = omega_m1 != 0.0 ? 2 : 1;
   const double2* m = es;
   double nuc = 0.0;
-  double2 g = cz();
   for (int r = 0; r < rounds; ++r) {
+    const double sgn = r == 0 ? -1.0 : 1.0;
     __builtin_amdgcn_wave_barrier();
-    if (!polar4_wave(d, m, g, lane, &nuc)) {
+    if (!polar4_wave(d, m, g_new, sgn, lane, want, &nuc)) {
       // zero or ill-conditioned matrices, and whatever else it declined
       if (lane == 0) {
         double2 w[16];
         polar4_jacobi(d, m, w, &nuc);
 #pragma unroll
-        for (int k = 0; k < 16; ++k) g_new[k] = w[k];
+        for (int k = 0; k < 16; ++k) g_new[k] = make_double2(w[k].x, sgn * w[k].y);
       }
-      __builtin_amdgcn_wave_barrier();
       nuc = lane_value(nuc, 0);
-      g = g_new[l];
     }
-    if (r == 0) g = cconj(g);
+    __builtin_amdgcn_wave_barrier();
     if (r + 1 < rounds) {
+      const bool in = (l >> 2) < d && (l & 3) < d;
+      const double2 g = g_new[l];
       if (lane < 16) rm[l] = in ? cadd(g, cscale(csub(g, g_old[l]), omega_m1)) : cz();
       m = rm;
     }
   }
-  if (lane < 16) g_new[l] = g;
-  if (rounds > 1) {
-    const double2 p = in ? cmul(g, es[l]) : cz();
+  if (rounds > 1 && want) {
+    const double2 p = cmul(g_new[l], es[l]);
     const double re = sum16(p.x), im = sum16(p.y);
     nuc = sqrt(re * re + im * im);
   }

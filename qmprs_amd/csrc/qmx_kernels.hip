@@ -545,8 +545,7 @@ __global__ __launch_bounds__(256) void sweep_step_kernel(SweepArgs<S> a) {
         s_em[l] = make_double2(tot[2 * l], tot[2 * l + 1]);
         gp[l] = a.gates[gic * 16 + l];
       }
-      const double nuc = update_gate_wave(wc == 2 ? 4 : 2, a.omega_m1, gp, s_em, s_rm, gc, lane);
-      __builtin_amdgcn_wave_barrier();
+      const double nuc = update_gate_wave(wc == 2 ? 4 : 2, a.omega_m1, gp, s_em, s_rm, gc, lane, a.overlap != nullptr);
       if (lane < 16) a.gates[gic * 16 + l] = gc[l];
       if (lane == 0) {
         if (a.overlap) a.overlap[(size_t)b * a.overlap_stride] = nuc;

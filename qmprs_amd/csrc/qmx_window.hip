@@ -827,7 +827,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // of dependent small steps, bound by their latency: wave 0 takes each gate's
 // environment and polar factor without a barrier inside, the other waves apply
 // the next gate to the state side of Q at the same time (the two sides
-// commute), and two barriers per gate are left.  16.6 us per window of one
+// commute), and two barriers per gate are left.  13.2 us per window of one
 // N=10 complex128 state (3.3 gates), against 48.3 us with a barrier around each
 // of the gate's steps and the 16-lane pivoted polar.
 // It runs beside the other half-batch's window pass, whose waves fill the
@@ -912,15 +912,15 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
         }
       }
       if (lane < 16) es[lane] = acc;
-      const double nuc = update_gate_wave(d, a.omega_m1, gm[j], es, rm, gnew, lane);
-      __builtin_amdgcn_wave_barrier();
+      const bool last = a.s0 + j == kb - 1 && a.overlap;
+      const double nuc = update_gate_wave(d, a.omega_m1, gm[j], es, rm, gnew, lane, last);
       if (lane < 16) {
         int layer, site;
         step_gate(n, a.s0 + j, layer, site);
         const size_t gi = ((size_t)b * a.lmax + layer) * n + site;
         a.gates[gi * 16 + lane] = gnew[lane];
       }
-      if (lane == 0 && a.s0 + j == kb - 1 && a.overlap) a.overlap[(size_t)b * a.overlap_stride] = nuc;
+      if (lane == 0 && last) a.overlap[(size_t)b * a.overlap_stride] = nuc;
     } else if (more) {
       // the other waves apply the next gate on the state side meanwhile:
       // Q[x][y] <- sum_{y'} Q[x][y'] conj(G_{j+1}[y'_g][y_g])
