@@ -50,10 +50,12 @@ int qmx_destroy(qmx_handle* h);
 const char* qmx_last_error(const qmx_handle* h);
 
 /* Tuning options (no reference counterpart).
- * QMX_OPT_SWEEP_MODE: QMX_SWEEP_AUTO (windowed passes for N >= 10, else one
- * pass per gate), QMX_SWEEP_STEP (one pass per gate) or QMX_SWEEP_WINDOW
- * (windowed passes; below N = 10, where a tile holds too few rest indices for
- * the pass kernel's four waves, it also runs one pass per gate). */
+ * QMX_OPT_SWEEP_MODE: QMX_SWEEP_AUTO (small states, up to N = 12 in complex128
+ * and 13 in complex64, each in one block that keeps the state on chip for all
+ * sweeps; windowed passes above, else one pass per gate), QMX_SWEEP_STEP (one
+ * pass per gate) or QMX_SWEEP_WINDOW (windowed passes; below N = 10, where a
+ * tile holds too few rest indices for the pass kernel's four waves, it runs
+ * one pass per gate). */
 #define QMX_OPT_SWEEP_MODE 1
 #define QMX_SWEEP_AUTO 0
 #define QMX_SWEEP_STEP 1
@@ -214,7 +216,8 @@ int qmx_extract_layers(qmx_handle* h, int num_qubits, int batch, int num_layers,
  *   overlap     device or NULL, B x num_sweeps doubles: <T|C'|0> at the end of
  *               each sweep (sum of singular values of the last environment)
  *   goal        device or NULL, B doubles: a state stops sweeping once
- *               |<psi_ref|C|0>| >= goal[b] (requires psi_ref; synchronises
+ *               |<psi_ref|C|0>| >= goal[b] (requires psi_ref; but for the
+ *               one-block sweeps of small states it synchronises
  *               once per sweep); sweeps_done (device or NULL, B ints) then
  *               receives the number of sweeps each state ran.
  *   circuit_out device or NULL, B x 2^N of storage_dtype: final C|0..0> */

@@ -285,7 +285,8 @@ def set_sweep_relaxation(omega: float) -> None:
 
 
 def set_sweep_mode(mode: str) -> None:
-    """'auto' (windowed passes for N >= 10), 'step' (one pass per gate) or
-    'window' (windowed passes; below N = 10 it also runs one pass per gate)."""
+    """'auto' (small states in one block each, else windowed passes), 'step'
+    (one pass per gate) or 'window' (windowed passes; below N = 10 it also
+    runs one pass per gate)."""
     h = handle()
     check(load().qmx_set_option(h, QMX_OPT_SWEEP_MODE, SWEEP_MODES[mode]), h)

@@ -1063,6 +1063,52 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
                    double2* fidelity, double* overlap, const double* goal, int* sweeps_done,
                    S* circuit_out, Carver& c, hipStream_t st, int snap_first = -1,
                    double2* snapshots = nullptr) {
+  // Small states are swept by one block each, in one launch: their sweeps are
+  // chains of polar factors, and a launch per window or gate costs more than
+  // its work (complex128, 4 layers, 4 sweeps: N=5 0.40 ms against 1.46 gate by
+  // gate; N=11 1.16 against 1.55 in windows, for 16 states 1.19 against 2.93).
+  // At the largest N a block has a CU for itself and is bound by its one CU's
+  // work, so a lone state (1.88 ms against 1.70 in windows at N=12) and batches
+  // that run in more than two rounds over the CUs (600 complex64 states of
+  // N=13: 10.2 against 8.8) stay in windows.  Snapshots with a goal keep the
+  // windows too: whether one is written depends on the whole batch there.  And
+  // so does a goal on a capturing stream: the windows' host check ends such a
+  // capture with an error at every size.
+  const int lds_most = lds_sweep_qubits(sizeof(S));
+  const bool one_block = n < lds_most || (n == lds_most && batch > 1 && batch <= 2 * h->cus);
+  bool goal_capture = false;
+  if (goal && one_block) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    QMX_HIP(h, hipStreamIsCapturing(st, &cs));
+    goal_capture = cs != hipStreamCaptureStatusNone;
+  }
+  if (h->sweep_mode == QMX_SWEEP_AUTO && one_block && !(goal && snapshots) && !goal_capture) {
+    PhaseTimer swt(h, st, QMX_PHASE_SWEEP);
+    LdsSweepArgs<S> a{};
+    a.n = n;
+    a.lmax = lmax;
+    a.nsweeps = nsweeps;
+    a.target = target;
+    a.gates = gates;
+    a.widths = widths;
+    a.layers = layers_used;
+    a.psi_ref = psi_ref;
+    a.fidelity = fidelity;
+    a.overlap = overlap;
+    a.goal = goal;
+    a.sweeps_done = sweeps_done;
+    a.circuit_out = circuit_out;
+    a.omega_m1 = (h->relax_milli - 1000) * 1e-3;
+    if (snapshots && snap_first >= 0) {
+      a.snap_first = snap_first;
+      a.snaps = snapshots;
+      a.snap_stride = (size_t)batch * lmax * n * 16;
+    }
+    if (fidelity) launch_fill_int(reinterpret_cast<int*>(fidelity), 0, batch * (nsweeps + 1) * 4, st);
+    QMX_HIP(h, launch_lds_sweep<S>(a, batch, st));
+    swt.stop(1);
+    return QMX_OK;
+  }
   const bool split = h->split_sweeps && batch >= 2 && sweep_windowed(h, n);
   const size_t len = state_len(n);
   auto job = [&](int b0, int nb, hipStream_t js) {

@@ -232,6 +232,24 @@ QMX_DEV double lane_value(double v, int lane) {
                           __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
+// Half-wave (quarter-wave) exchange and add: lanes below 32 (even rows of 16)
+// get a's sum over the two halves (the row and the next), the others b's.
+QMX_DEV double swap_add32(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+QMX_DEV double swap_add16(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+// the sum over the wave's four rows of 16 lanes, on every lane
+QMX_DEV double rows_sum(double v) {
+  v = swap_add32(v, v);
+  return swap_add16(v, v);
+}
+
 // 1 / x to rounding: the hardware estimate and two Newton steps
 QMX_DEV double rcp_newton(double x) {
   double r = __builtin_amdgcn_rcp(x);
@@ -348,89 +366,95 @@ QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc)
 // passes), their part of the factor is Q polar(R); the zero columns z_1 < z_2,
 // whose right singular vectors are e_{z_1}, e_{z_2}, take the rule's left
 // completion, the first unit vectors with a residual above 1/2 (which one
-// pass of Gram-Schmidt then gives to rounding): 5300 cycles, against 30600 by
-// the Jacobi path.  zero: the columns that are (bits), es 2^h: the matrix, fro:
-// its squared norm, near 1; lane l < 16 of x gets entry l.
+// pass of Gram-Schmidt then gives to rounding).  Lane 4 i + j of 16 works on
+// row i and on column j of (live, live, zero, zero).  zero: the zero columns
+// (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry (i, j) of
+// the factor.  False where the Jacobi path decides (30600 cycles); 2700
+// cycles, against 5300 to 7500 with the whole problem in every lane.
+template <int J> QMX_DEV double quad_bcast(double v) { return dpp<J * 0x55>(v); }
+template <int J> QMX_DEV double2 quad_bcast2(double2 v) { return make_double2(quad_bcast<J>(v.x), quad_bcast<J>(v.y)); }
+// sum over the 4 rows i
+QMX_DEV double col_total(double v) {
+  v += dpp<kDppRow2>(v);
+  return v + dpp<kDppRow1>(v);
+}
 QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, unsigned zero, double fro, double* nuc) {
   const unsigned live = ~zero & 15u;
   const int c0 = __ffs(live) - 1, c1 = 31 - __clz(live), z0 = __ffs(zero) - 1, z1 = 31 - __clz(zero);
-  // every lane holds the whole 4 x 2 problem
-  double2 q0[4], q1[4], q2[4], q3[4];
-  double n0 = 0.0, n1 = 0.0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const double2 u = es[i * 4 + c0], v = es[i * 4 + c1];
-    q0[i] = make_double2(ldexp(u.x, h), ldexp(u.y, h));
-    q1[i] = make_double2(ldexp(v.x, h), ldexp(v.y, h));
-    n0 += cabs2(q0[i]);
-  }
+  const int i = l >> 2, j = l & 3;
+  const double2 e = es[4 * i + (j & 1 ? c1 : c0)];
+  double2 y = make_double2(ldexp(e.x, h), ldexp(e.y, h));   // columns j = 0, 1 (and again at 2, 3)
+  const double n0 = quad_bcast<0>(col_total(cabs2(y)));
   const double i0 = rsqrt_newton(n0);
+  const double2 q0 = cscale(quad_bcast2<0>(y), i0);         // row i of q_0
   double2 p00 = make_double2(n0 * i0, 0.0), p01 = cz(), p10 = cz();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) q0[i] = cscale(q0[i], i0);
-#pragma unroll
   for (int pass = 0; pass < 2; ++pass) {
-    double2 d = cz();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) d = cfmac(q0[i], q1[i], d);
-    p01 = cadd(p01, d);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q1[i] = csub(q1[i], cmul(q0[i], d));
+    const double2 t = cmulc(q0, y);
+    const double2 d = make_double2(col_total(t.x), col_total(t.y));
+    p01 = cadd(p01, quad_bcast2<1>(d));
+    y = csub(y, cmul(q0, d));
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) n1 += cabs2(q1[i]);
+  const double n1 = quad_bcast<1>(col_total(cabs2(y)));
   if (!(n1 > 1e-26 * fro)) return false;
   const double i1 = rsqrt_newton(n1);
+  const double2 q1 = cscale(quad_bcast2<1>(y), i1);
   double2 p11 = make_double2(n1 * i1, 0.0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) q1[i] = cscale(q1[i], i1);
   if (!polar2(p00, p01, p10, p11, nuc)) return false;
-  // squared residuals of e_0 .. e_3 against the vectors so far
-  double res[4];
+  // squared residual of e_i against q_0, q_1; the first above 1/4
+  const double res = 1.0 - cabs2(q0) - cabs2(q1);
+  const unsigned m2 = (unsigned)__ballot(res > 0.25) & 0x1111u;
+  if (!m2) return false;
+  const int e2 = __builtin_amdgcn_readfirstlane((__ffs(m2) - 1) >> 2);
+  auto row = [&](double2 v, int k) { return make_double2(lane_value(v.x, 4 * k), lane_value(v.y, 4 * k)); };
+  double2 t = cadd(cmulc(row(q0, e2), q0), cmulc(row(q1, e2), q1));
+  double2 q2 = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
+  q2 = cscale(q2, rsqrt_newton(col_total(cabs2(q2))));
+  const unsigned m3 = (unsigned)__ballot(i > e2 && res - cabs2(q2) > 0.25) & 0x1111u;
+  if (!m3) return false;
+  const int e3 = __builtin_amdgcn_readfirstlane((__ffs(m3) - 1) >> 2);
+  t = cadd(cadd(cmulc(row(q0, e3), q0), cmulc(row(q1, e3), q1)), cmulc(row(q2, e3), q2));
+  double2 q3 = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
+  q3 = cscale(q3, rsqrt_newton(col_total(cabs2(q3))));
+  // out column z_1: q_2, z_2: q_3, the live ones: Q polar(R)
+  const double2 a = j == c0 ? p00 : p01, b = j == c0 ? p10 : p11;
+  x = cadd(cmul(q0, a), cmul(q1, b));
+  if (j == z0) x = q2;
+  if (j == z1) x = q3;
+  return true;
+}
+
+// The same with three zero columns, the environment of the gate whose both
+// sites are in |0>: the live column over its norm, and three completions.
+QMX_DEV bool polar4_one_column(double2& x, int l, const double2* es, int h, unsigned zero, double* nuc) {
+  const int c0 = __ffs(~zero & 15u) - 1;
+  const int i = l >> 2, j = l & 3;
+  const double2 e = es[4 * i + c0];
+  const double2 y = make_double2(ldexp(e.x, h), ldexp(e.y, h));
+  const double n0 = col_total(cabs2(y)), i0 = rsqrt_newton(n0);
+  *nuc = n0 * i0;
+  double2 q[4];
+  q[0] = cscale(y, i0);
+  x = q[0];
+  double res = 1.0 - cabs2(q[0]);   // squared residual of e_i
+  int from = 0, slot = 0;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) res[e] = 1.0 - cabs2(q0[e]) - cabs2(q1[e]);
-  int e2 = -1, e3 = -1;
+  for (int k = 1; k < 4; ++k) {
+    const unsigned m = (unsigned)__ballot(i >= from && res > 0.25) & 0x1111u;
+    if (!m) return false;
+    const int ek = __builtin_amdgcn_readfirstlane((__ffs(m) - 1) >> 2);
+    double2 t = cz();
 #pragma unroll
-  for (int e = 3; e >= 0; --e)
-    if (res[e] > 0.25) e2 = e;
-  if (e2 < 0) return false;
-  auto pick = [](const double2 (&v)[4], int k) { return k == 0 ? v[0] : (k == 1 ? v[1] : (k == 2 ? v[2] : v[3])); };
-  {
-    const double2 h0 = pick(q0, e2), h1 = pick(q1, e2);
-    double nr = 0.0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const double2 t = cadd(cmulc(h0, q0[i]), cmulc(h1, q1[i]));
-      q2[i] = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
-      nr += cabs2(q2[i]);
-    }
-    const double ir = rsqrt_newton(nr);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q2[i] = cscale(q2[i], ir);
+    for (int b = 0; b < k; ++b)
+      t = cadd(t, cmulc(make_double2(lane_value(q[b].x, 4 * ek), lane_value(q[b].y, 4 * ek)), q[b]));
+    const double2 w = make_double2((i == ek ? 1.0 : 0.0) - t.x, -t.y);
+    q[k] = cscale(w, rsqrt_newton(col_total(cabs2(w))));
+    res -= cabs2(q[k]);
+    from = ek + 1;
+    if (slot == c0) ++slot;
+    if (j == slot) x = q[k];
+    ++slot;
   }
-#pragma unroll
-  for (int e = 3; e >= 0; --e)
-    if (e > e2 && res[e] - cabs2(q2[e]) > 0.25) e3 = e;
-  if (e3 < 0) return false;
-  {
-    const double2 h0 = pick(q0, e3), h1 = pick(q1, e3), h2 = pick(q2, e3);
-    double nr = 0.0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const double2 t = cadd(cadd(cmulc(h0, q0[i]), cmulc(h1, q1[i])), cmulc(h2, q2[i]));
-      q3[i] = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
-      nr += cabs2(q3[i]);
-    }
-    const double ir = rsqrt_newton(nr);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q3[i] = cscale(q3[i], ir);
-  }
-  const int i = (l >> 2) & 3, j = l & 3;
-  const double2 a = pick(q0, i), b = pick(q1, i);
-  if (j == z0) x = pick(q2, i);
-  else if (j == z1) x = pick(q3, i);
-  else if (j == c0) x = cadd(cmul(a, p00), cmul(b, p10));
-  else x = cadd(cmul(a, p01), cmul(b, p11));
   return true;
 }
 
@@ -484,8 +508,10 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int
   for (int k = 0; k < 4; ++k)
     if (!(big & (0x1111ull << k))) zero |= 1u << k;
   fro = ldexp(fro, 2 * h);
-  if (__popc(zero) == 2) {
-    if (!polar4_two_columns(x, l, es, h, zero, fro, &s)) return false;
+  if (__popc(zero) >= 2) {
+    if (!(__popc(zero) == 2 ? polar4_two_columns(x, l, es, h, zero, fro, &s)
+                            : polar4_one_column(x, l, es, h, zero, &s)))
+      return false;
     if (lane < 16) out[l] = make_double2(x.x, sgn * x.y);
     *nuc = ldexp(s, -h);
     return true;

@@ -121,6 +121,32 @@ struct WinPassArgs {
   int store;           // write T' and phi back (0 for a sweep's last window: neither is read again)
 };
 
+// All sweeps of small states in one launch (qmx_window.hip): one block per
+// state, T' and phi in LDS.
+template <typename S>
+struct LdsSweepArgs {
+  int n, lmax, nsweeps;
+  const S* target;
+  double2* gates;
+  const int* widths;
+  const int* layers;
+  const double2* psi_ref;   // may be nullptr
+  double2* fidelity;        // fidelity[b (nsweeps + 1) + s], may be nullptr
+  double* overlap;          // overlap[b nsweeps + s], may be nullptr
+  const double* goal;       // stop once |fidelity| >= goal[b]; nullptr: all sweeps
+  int* sweeps_done;         // may be nullptr
+  S* circuit_out;           // may be nullptr
+  double omega_m1;
+  double2* snaps;           // gates after snap_first and snap_first + 1 sweeps, may be nullptr
+  size_t snap_stride;
+  int snap_first;
+};
+// largest N whose T' and phi fit one block's LDS beside its partial sums
+// (2 x 64 KiB of 160): 2^12 complex128 or 2^13 complex64 amplitudes
+constexpr int lds_sweep_qubits(size_t amp_bytes) { return amp_bytes == 8 ? 13 : 12; }
+template <typename S>
+hipError_t launch_lds_sweep(const LdsSweepArgs<S>& a, int batch, hipStream_t st);
+
 // Forward circuit pass (qmx_window.hip): up to kMaxStages stages of gates,
 // each stage acting inside its own 4-bit group set, exchanged through LDS.
 // Stage k applies the gates at forward positions fpos[gstart[k] .. gstart[k+1]).

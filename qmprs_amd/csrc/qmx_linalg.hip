@@ -447,16 +447,6 @@ constexpr double kOsjTol = 2e-15;
 // The totals over the wave of four per-lane values: row k (lanes 16 k ..
 // 16 k + 15) holds the total of v_k on every lane.  Two half-swaps merge the
 // four registers, then four DPP steps add inside the rows.
-QMX_DEV double swap_add32(double a, double b) {
-  const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-  const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
-}
-QMX_DEV double swap_add16(double a, double b) {
-  const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-  const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-  return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
-}
 QMX_DEV double rows_total(double v0, double v1, double v2, double v3) {
   return sum16(swap_add16(swap_add32(v0, v2), swap_add32(v1, v3)));
 }

@@ -959,6 +959,406 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
   }
 }
 
+// ---- all sweeps of a small state in one block -------------------------------
+// T' and phi (up to 2^12 complex128 or 2^13 complex64 amplitudes) stay in LDS
+// from the first sweep to the last.  The sweep is a serial chain of polar
+// factors, so everything else is taken off that chain: in phase p of a sweep
+// wave 0, the lead, turns the cross matrix of step p - 1 into its environment
+// and new gate G'_{p-1}, while waves 1 to 4 prepare step p without it,
+//   T'  <- G'_{p-2}^dagger T',   phi <- G_p^dagger phi,
+//   R_p[x][y] = sum_r conj(T'[x, r]) phi[y, r]
+// over the set V of the bits of steps p - 1 and p (three of them, the steps
+// descend one site at a time), an 8 x 8 matrix.  G'_{p-1}, which R_p still lacks, acts inside V, so the
+// next phase's environment is
+//   E_p[o][i] = sum_z sum_x' G'_{p-1}[x'_g][x_g] R_p[x'][y],  x = (o, z), y = (i, z).
+// Each worker owns a quarter of the indices r outside U = V and step p - 2's
+// bits in a phase, so updates and products need no barrier between them, and
+// one barrier per step is left.  Gate p + 2 is fetched two phases ahead.
+// After the gate of site i of the first circuit layer is removed, the sites
+// behind i are in |0>: phi is set to exactly zero where they are not.
+// The lead's chain bounds it up to 2^10 complex128 amplitudes (8.4k cycles a
+// step at N = 6, environment 1.9k and polar factor 6k, and 8.8k at N = 10), the
+// workers' updates and products above (18k at N = 12).  One state, 4 layers, 4
+// sweeps: 0.40 ms against 1.46 gate by gate at N = 5, 0.83 against 1.32 in
+// windows at N = 10; 16 states of N = 12 1.9 ms against 3.2.
+constexpr int kLdsWorkers = 4;
+constexpr int kLdsThreads = 64 * (1 + kLdsWorkers);
+constexpr int kLdsChunk = 32;   // gates per stage of the circuit rebuild (the partials' space)
+
+// Place of amplitude l in LDS: its banks, 8 double2 or 16 float2 wide, take the
+// XOR of l's 3-bit or 4-bit digits, so that the three neighbouring bits which
+// the lanes of a product run over never share a bank.  (Linear over XOR.)
+template <typename S> QMX_DEV int lds_at(int l) {
+  if constexpr (sizeof(S) == 16) return l ^ (((l >> 3) ^ (l >> 6) ^ (l >> 9) ^ (l >> 12)) & 7);
+  else return l ^ (((l >> 4) ^ (l >> 8) ^ (l >> 12)) & 15);
+}
+// x with a zero bit inserted at position p
+QMX_DEV int zero_at(int x, int p) { return x + (x & ~((1 << p) - 1)); }
+// the low bits of z at the set bits of mask (at most three of them)
+QMX_DEV int spread3(int z, uint32_t mask) {
+  const uint32_t f0 = mask & (~mask + 1u), r1 = mask ^ f0, f1 = r1 & (~r1 + 1u), f2 = r1 ^ f1;
+  return (z & 1 ? f0 : 0) | (z & 2 ? f1 : 0) | (z & 4 ? f2 : 0);
+}
+
+// y = G^dagger x on amplitude quads (w = 2: bits h, h - 1) or pairs (w = 1: bit
+// h) of an LDS state: this lane's patterns are base ^ su(u), u < nu (swizzled
+// indices with the gate's bits zero; every index map here is linear over bit
+// fields and the swizzle over XOR), if `on`.
+template <typename S, typename F>
+QMX_DEV void lds_gate(S* s, int w, int h, const double2* g, int nu, bool on, int base, F su) {
+  using T = CT<typename StoreC<S>::C>;
+  using c2 = typename T::c2;
+  const int sh = lds_at<S>(1 << h);
+  if (!on) return;
+  if (w == 2) {
+    const int sl = lds_at<S>(1 << (h - 1));
+    c2 gc[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) gc[k] = T::mk(g[k]);
+    auto load = [&](int i0, c2 (&x)[4]) {
+      x[0] = T::mk(to_c(s[i0]));
+      x[1] = T::mk(to_c(s[i0 ^ sl]));
+      x[2] = T::mk(to_c(s[i0 ^ sh]));
+      x[3] = T::mk(to_c(s[i0 ^ sl ^ sh]));
+    };
+    auto apply = [&](int i0, const c2 (&x)[4]) {
+      c2 y[4];
+#pragma unroll
+      for (int o = 0; o < 4; ++o) {
+        c2 acc = T::mulc(gc[o], x[0]);
+        acc = T::fmac(gc[4 + o], x[1], acc);
+        acc = T::fmac(gc[8 + o], x[2], acc);
+        y[o] = T::fmac(gc[12 + o], x[3], acc);
+      }
+      s[i0] = from_c<S>(make_double2(y[0].x, y[0].y));
+      s[i0 ^ sl] = from_c<S>(make_double2(y[1].x, y[1].y));
+      s[i0 ^ sh] = from_c<S>(make_double2(y[2].x, y[2].y));
+      s[i0 ^ sl ^ sh] = from_c<S>(make_double2(y[3].x, y[3].y));
+    };
+    // two patterns at a time: one's loads are in flight under the other's work
+    int u = 0;
+    for (; u + 1 < nu; u += 2) {
+      const int ia = base ^ su(u), ib = base ^ su(u + 1);
+      c2 xa[4], xb[4];
+      load(ia, xa);
+      load(ib, xb);
+      apply(ia, xa);
+      apply(ib, xb);
+    }
+    if (u < nu) {
+      const int ia = base ^ su(u);
+      c2 xa[4];
+      load(ia, xa);
+      apply(ia, xa);
+    }
+  } else {
+    const c2 g00 = T::mk(g[0]), g01 = T::mk(g[1]), g10 = T::mk(g[4]), g11 = T::mk(g[5]);
+    for (int u = 0; u < nu; ++u) {
+      const int i0 = base ^ su(u), i1 = i0 ^ sh;
+      const c2 x0 = T::mk(to_c(s[i0])), x1 = T::mk(to_c(s[i1]));
+      const c2 y0 = T::fmac(g10, x1, T::mulc(g00, x0)), y1 = T::fmac(g11, x1, T::mulc(g01, x0));
+      s[i0] = from_c<S>(make_double2(y0.x, y0.y));
+      s[i1] = from_c<S>(make_double2(y1.x, y1.y));
+    }
+  }
+}
+
+template <typename S>
+__global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> a) {
+  extern __shared__ char wsm[];
+  __shared__ double2 gold[4][16];            // old gates of steps p - 1 .. p + 1
+  __shared__ double2 gnew[3][16];            // new gates of steps p - 3 .. p - 1
+  __shared__ double2 es[16], rm[16];
+  __shared__ int wold[4];                    // widths of gold (and of the new gates)
+  __shared__ int wch[kLdsChunk];
+  __shared__ uint32_t uset[16], vset[16];
+  __shared__ double red[2 * (1 + kLdsWorkers)];
+  const int b = blockIdx.x, n = a.n;
+  const size_t len = (size_t)1 << n;
+  S* sT = reinterpret_cast<S*>(wsm);
+  S* sP = sT + len;
+  double2* part = reinterpret_cast<double2*>(sP + len);   // 2 phases x kLdsWorkers x 64; gate stages
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lb = min(max(a.layers[b], 0), a.lmax), K = lb * n;
+  double2* gates = a.gates + (size_t)b * a.lmax * n * 16;
+  const int* widths = a.widths + (size_t)b * a.lmax * n;
+  const double2* ref = a.psi_ref && a.fidelity ? a.psi_ref + (size_t)b * len : nullptr;
+  const int mu = n < 4 ? n : 4, mv = n < 3 ? n : 3;   // bits of U and V
+  // C|0..0> into sP, gates in forward order (their adjoints into the stage:
+  // lds_gate conjugates back)
+  auto rebuild = [&]() {
+    for (int l = tid; l < (int)len; l += kLdsThreads) sP[lds_at<S>(l)] = from_c<S>(make_double2(l == 0 ? 1.0 : 0.0, 0.0));
+    for (int f0 = 0; f0 < K; f0 += kLdsChunk) {
+      const int nf = min(kLdsChunk, K - f0);
+      __syncthreads();
+      for (int e = tid; e < nf * 16; e += kLdsThreads) {
+        const int f = f0 + (e >> 4);
+        const size_t gi = (size_t)(lb - 1 - f / n) * n + f % n;
+        part[e] = cconj(gates[gi * 16 + (e & 3) * 4 + ((e >> 2) & 3)]);
+        if ((e & 15) == 0) wch[e >> 4] = wsane(n, f % n, widths[gi]);
+      }
+      __syncthreads();
+      int h = n - 1 - f0 % n;
+      for (int g = 0; g < nf; ++g) {
+        // one wave per SIMD: wave 0 would be the fifth
+        if (wave) {
+          const int w = __builtin_amdgcn_readfirstlane(wch[g]);
+          const int cnt = (int)(len >> w), t0 = tid - 64;
+          auto at = [&](int t) { return lds_at<S>(w == 2 ? zero_at(zero_at(t, h - 1), h) : zero_at(t, h)); };
+          lds_gate<S>(sP, w, h, part + g * 16, (cnt + kLdsThreads - 65) / (kLdsThreads - 64), t0 < cnt, at(t0),
+                      [&](int u) { return at(u * (kLdsThreads - 64)); });
+        }
+        h = h ? h - 1 : n - 1;
+        __syncthreads();
+      }
+    }
+    __syncthreads();
+  };
+  // <psi_ref|C|0..0> of sP, on every thread (fixed order)
+  auto overlap_ref = [&]() {
+    double re = 0.0, im = 0.0;
+    for (int l = tid; l < (int)len; l += kLdsThreads) {
+      const double2 r = ref[l], p = to_c(sP[lds_at<S>(l)]);
+      re = fma(r.x, p.x, fma(r.y, p.y, re));
+      im = fma(r.x, p.y, fma(-r.y, p.x, im));
+    }
+    re = rows_sum(sum16(re));
+    im = rows_sum(sum16(im));
+    if (lane == 0) {
+      red[2 * wave] = re;
+      red[2 * wave + 1] = im;
+    }
+    __syncthreads();
+    double2 t = cz();
+#pragma unroll
+    for (int w = 0; w <= kLdsWorkers; ++w) t = cadd(t, make_double2(red[2 * w], red[2 * w + 1]));
+    __syncthreads();
+    return t;
+  };
+  auto snapshot = [&](int done) {
+    if (!a.snaps || done < a.snap_first || done > a.snap_first + 1) return;
+    double2* dst = a.snaps + (size_t)(done - a.snap_first) * a.snap_stride + (size_t)b * a.lmax * n * 16;
+    for (int e = tid; e < a.lmax * n * 16; e += kLdsThreads) dst[e] = gates[e];
+  };
+  // Step p acts on bit r = p % n (site n - 1 - r) and, with two qubits, on
+  // bit r - 1.  By residue: U, the worst-case bits of steps p, p - 1 and p - 2,
+  // and V, those of p and p - 1 (before the sweep's start any bits will do),
+  // padded with the lowest free ones (V inside U).
+  if (tid < n) {
+    uint32_t u = 0, v = 0;
+    for (int k = 0; k < 3; ++k) {
+      const int r = (tid + 2 * n - k) % n;
+      u |= 1u << r | (r > 0 ? 1u << (r - 1) : 0u);
+      if (k == 1) v = u;
+    }
+    for (int bit = 0; bit < n && __popc(u) < mu; ++bit) u |= 1u << bit;
+    for (int bit = 0; bit < n && __popc(v) < mv; ++bit) v |= u & (1u << bit);
+    uset[tid] = u;
+    vset[tid] = v;
+  }
+  auto prev = [&](int r) { return r == 0 ? n - 1 : r - 1; };
+  auto rank_in = [](uint32_t u, int bit) { return __popc(u & ((1u << bit) - 1u)); };
+  auto gate_at = [&](int r, int layer) { return (size_t)layer * n + (n - 1 - r); };
+  snapshot(0);
+  const bool use_goal = a.goal && ref;
+  int done = 0;
+  double2 fid = cz();
+  int s = 0;
+  for (; s < a.nsweeps; ++s) {
+    rebuild();
+    if (ref) {
+      fid = overlap_ref();
+      if (tid == 0) a.fidelity[(size_t)b * (a.nsweeps + 1) + s] = fid;
+    }
+    if (use_goal && sqrt(fid.x * fid.x + fid.y * fid.y) >= a.goal[b]) break;
+    ++done;
+    const S* tsrc = a.target + (size_t)b * len;
+    for (int l = tid; l < (int)len; l += kLdsThreads) sT[lds_at<S>(l)] = tsrc[l];
+    // old gates: step 0 now, step p + 1 written in phase p, where step p + 2 is
+    // fetched into a worker's registers
+    if (tid < 16 && K > 0) {
+      gold[0][tid] = gates[gate_at(0, 0) * 16 + tid];
+      if (tid == 0) wold[0] = wsane(n, n - 1, widths[gate_at(0, 0)]);
+    }
+    const bool fetcher = wave == 1 && lane < 16;
+    double2 gnext = cz();
+    int wnext = 0;
+    int fr = 1, fl = 0;   // residue and layer of the step to fetch next (n >= 2)
+    if (fetcher && K > 1) {
+      gnext = gates[gate_at(fr, fl) * 16 + lane];
+      wnext = wsane(n, n - 1 - fr, widths[gate_at(fr, fl)]);
+    }
+    int rp = 0, layer_prev = 0;   // p % n; the layer of step p - 1
+    __syncthreads();
+    for (int p = 0; p <= K && K > 0; ++p) {
+      if (wave == 0) {
+        if (p > 0) {
+          // ---- lead: the environment and the new gate of step k = p - 1
+          __builtin_amdgcn_s_setprio(3);
+          const int k = p - 1, hbit = prev(rp);
+          const uint32_t v = __builtin_amdgcn_readfirstlane(vset[hbit]);
+          const int w = __builtin_amdgcn_readfirstlane(wold[k & 3]), d = w == 2 ? 4 : 2;
+          const int hb = rank_in(v, hbit), gl = w == 2 ? hb - 1 : hb;   // the gate's lowest bit in V
+          // the pending gate of step k - 1
+          const int kp = k - 1, hpbit = prev(hbit);
+          const int wp = kp >= 0 ? __builtin_amdgcn_readfirstlane(wold[kp & 3]) : 0;
+          const int pl = rank_in(v, hpbit) - (wp == 2 ? 1 : 0), np = wp == 2 ? 4 : (wp == 1 ? 2 : 1);
+          const int pmask = (np - 1) << pl;
+          const double2* gp = gnew[(kp + 3) % 3];
+          const int o = (lane >> 2) & 3, i = lane & 3, row = lane >> 4;
+          const uint32_t fm = ((1u << mv) - 1u) & ~((uint32_t)(d - 1) << gl);   // V's bits beside the gate's
+          const int nz = (1 << mv) / d;
+          // terms (z, x'_g), one in four per row of lanes
+          double2 acc = cz();
+          for (int t = row; t < nz * np; t += 4) {
+            const int pg = t & (np - 1), z = spread3(t / np, fm);
+            const int x = (z | (o & (d - 1)) << gl), y = (z | (i & (d - 1)) << gl);
+            const int at = (wp ? (x & ~pmask) | pg << pl : x) * 8 + y;
+            const double2* q = part + (k & 1) * kLdsWorkers * 64 + at;
+            const double2 e = cadd(cadd(q[0], q[64]), cadd(q[128], q[192]));
+            acc = wp ? cfma(gp[pg * 4 + ((x >> pl) & (np - 1))], e, acc) : cadd(acc, e);
+          }
+          acc = make_double2(rows_sum(acc.x), rows_sum(acc.y));
+          if (lane < 16) es[lane] = o < d && i < d ? acc : cz();
+          const bool last = k == K - 1 && a.overlap;
+          const double nuc = update_gate_wave(d, a.omega_m1, gold[k & 3], es, rm, gnew[k % 3], lane, last);
+          if (lane < 16) gates[gate_at(hbit, layer_prev) * 16 + lane] = gnew[k % 3][lane];
+          if (lane == 0 && last) a.overlap[(size_t)b * a.nsweeps + s] = nuc;
+          __builtin_amdgcn_s_setprio(0);
+        }
+      } else if (p < K) {
+        // ---- workers: step p without G'_{p-1}
+        const int wid = wave - 1;
+        if (fetcher && p + 1 < K) {
+          gold[(p + 1) & 3][lane] = gnext;
+          if (lane == 0) wold[(p + 1) & 3] = wnext;
+          if (++fr == n) {
+            fr = 0;
+            ++fl;
+          }
+          if (p + 2 < K) {
+            gnext = gates[gate_at(fr, fl) * 16 + lane];
+            wnext = wsane(n, n - 1 - fr, widths[gate_at(fr, fl)]);
+          }
+        }
+        const uint32_t u = __builtin_amdgcn_readfirstlane(uset[rp]), v = __builtin_amdgcn_readfirstlane(vset[rp]);
+        int ub[4];
+        {
+          uint32_t t = u;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            ub[k] = t ? __ffs(t) - 1 : 31;
+            t &= t - 1u;
+          }
+        }
+        auto roff = [&](int r) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (k < mu) r = zero_at(r, ub[k]);
+          return r;
+        };
+        // this worker's indices r outside U: r0 .. r0 + nr - 1 (G a power of
+        // two, r0 a multiple of it)
+        const int rest = 1 << (n - mu);
+        const int G = rest >= kLdsWorkers ? rest / kLdsWorkers : 1, glog = __ffs(G) - 1;
+        const int r0 = wid * G, nr = r0 < rest ? G : 0;
+        const int sr0 = lds_at<S>(roff(r0));
+        auto update = [&](S* s, int w, int h, const double2* g) {
+          const uint32_t om = u & ~(w == 2 ? 3u << (h - 1) : 1u << h);   // U's bits beside the gate's
+          const int cnt = nr << (mu - w);
+          auto at = [&](int t) { return lds_at<S>(roff(t & (G - 1)) | spread3(t >> glog, om)); };
+          lds_gate<S>(s, w, h, g, (cnt + 63) >> 6, lane < cnt, sr0 ^ at(lane), [&](int k) { return at(64 * k); });
+        };
+        const int kt = p - 2, h = rp;
+        auto width_of = [&](int k) { return __builtin_amdgcn_readfirstlane(wold[k & 3]); };
+        if (kt >= 0) update(sT, width_of(kt), prev(prev(rp)), gnew[kt % 3]);
+        update(sP, width_of(p), h, gold[p & 3]);
+        __builtin_amdgcn_wave_barrier();
+        if (p >= K - n && h > 0) {
+          // the sites behind step p's are in |0> once this gate of the first
+          // circuit layer is gone
+          const uint32_t om = u & ~(1u << (h - 1));
+          for (int t = lane; t < nr << (mu - 1); t += 64)
+            sP[sr0 ^ lds_at<S>(roff(t & (G - 1)) | spread3(t >> glog, om) | 1 << (h - 1))] = from_c<S>(cz());
+          __builtin_amdgcn_wave_barrier();
+        }
+        // R over V by vector FMA (the 4 x 4 x 4 matrix instruction measured 80
+        // cycles here, four times the vector unit's for the same products): lane
+        // bits 0-2 take eight indices (r and U's bit outside V), bits 3-4 two x
+        // of T' and bit 5 four y of phi
+        const uint32_t far = u & ~v;                   // one bit, none for n < 4
+        const int cnt = far ? 2 * nr : nr, kk = lane & 7, x0 = 2 * ((lane >> 3) & 3), y0 = 4 * (lane >> 5);
+        auto at = [&](int t) { return lds_at<S>(roff(t & (G - 1)) | ((t >> glog) & 1 ? (int)far : 0)); };
+        // (lanes beyond V read valid places too: spread3 drops the bits that V lacks)
+        const int base = sr0 ^ at(kk), bt = base ^ lds_at<S>(spread3(x0, v)), bp = base ^ lds_at<S>(spread3(y0, v));
+        const int v0 = lds_at<S>(spread3(1, v)), v1 = lds_at<S>(spread3(2, v));
+        double2 acc[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = cz();
+        for (int k0 = 0; k0 < cnt; k0 += 8) {
+          const int off = at(k0);
+          double2 tv[2], pv[4];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) tv[j] = to_c(sT[bt ^ off ^ (j ? v0 : 0)]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) pv[j] = to_c(sP[bp ^ off ^ (j & 1 ? v0 : 0) ^ (j & 2 ? v1 : 0)]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] = cfmac(tv[e >> 2], pv[e & 3], acc[e]);
+        }
+        if (kk >= cnt)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) acc[e] = cz();
+        // sum over the eight lanes; each keeps one entry: (x0 + kk % 2, y0 + kk / 2)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const double2 keep = kk & 1 ? acc[4 + e] : acc[e], send = kk & 1 ? acc[e] : acc[4 + e];
+          acc[e] = make_double2(keep.x + dpp<0xB1>(send.x), keep.y + dpp<0xB1>(send.y));
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const double2 keep = kk & 2 ? acc[2 * e + 1] : acc[2 * e], send = kk & 2 ? acc[2 * e] : acc[2 * e + 1];
+          acc[e] = make_double2(keep.x + dpp<0x4E>(send.x), keep.y + dpp<0x4E>(send.y));
+        }
+        {
+          // lanes i and i ^ 4 through the mirrored halves: their low bits flip, so
+          // the quad is turned back first
+          const double2 keep = kk & 4 ? acc[1] : acc[0], send = kk & 4 ? acc[0] : acc[1];
+          acc[0] = make_double2(keep.x + dpp<0x141>(dpp<0x1B>(send.x)), keep.y + dpp<0x141>(dpp<0x1B>(send.y)));
+        }
+        part[((p & 1) * kLdsWorkers + wid) * 64 + (x0 + (kk & 1)) * 8 + y0 + ((kk >> 1) & 1) + 2 * (kk >> 2)] = acc[0];
+      }
+      __syncthreads();
+      if (p > 0 && rp == 0) ++layer_prev;   // step p starts a layer
+      rp = rp + 1 == n ? 0 : rp + 1;
+    }
+    snapshot(s + 1);
+  }
+  if (s == a.nsweeps) {
+    rebuild();
+    if (ref) fid = overlap_ref();
+  }
+  if (ref && tid == 0) a.fidelity[(size_t)b * (a.nsweeps + 1) + a.nsweeps] = fid;
+  if (a.sweeps_done && tid == 0) a.sweeps_done[b] = a.goal ? (use_goal ? done : 0) : a.nsweeps;
+  if (a.circuit_out)
+    for (int l = tid; l < (int)len; l += kLdsThreads) a.circuit_out[(size_t)b * len + l] = sP[lds_at<S>(l)];
+}
+
+template <typename S>
+hipError_t launch_lds_sweep(const LdsSweepArgs<S>& a, int batch, hipStream_t st) {
+  constexpr size_t parts = 2 * kLdsWorkers * 64 * sizeof(double2);
+  static_assert(parts >= kLdsChunk * 16 * sizeof(double2), "a stage of gates fits the partials' space");
+  // the limit is set to the largest need, so that launches from several host
+  // threads never lower it under each other
+  const size_t most = (2 * sizeof(S) << lds_sweep_qubits(sizeof(S))) + parts;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(lds_sweep_kernel<S>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(lds_sweep_kernel<S>, dim3(batch), dim3(kLdsThreads), (2 * sizeof(S) << a.n) + parts, st, a);
+  return hipGetLastError();
+}
+template hipError_t launch_lds_sweep<float2>(const LdsSweepArgs<float2>&, int, hipStream_t);
+template hipError_t launch_lds_sweep<double2>(const LdsSweepArgs<double2>&, int, hipStream_t);
+
 template <typename S>
 void launch_fwd_pass(const FwdArgs<S>& a, int nblk, int batch, hipStream_t st) {
   size_t shm = sizeof(S) << a.t;
