@@ -18,45 +18,77 @@ namespace qmx {
 
 // ------------------------------------------------------------------ gram ----
 // part[b][chunk] (nmax x nmax) = sum over the chunk's rows of conj(Y)[:, p] Y[:, q]
+// 16 T x 16 T entries per block, T x T per thread (every fourth of its tile's
+// columns: neighbouring lanes read neighbouring LDS words), rows in steps of
+// 16 fetched into registers one step ahead.  Bound by FP64 FMA at T = 4; T = 2
+// reads LDS twice as often for the same products and takes the launches whose
+// 64 x 64 tiles would leave CUs idle.  32 states of 2^13 x 128: 0.78 ms,
+// with 32 x 32 tiles and 1 x 4 entries per thread 1.04.
+constexpr int kGemmFill = 512;   // two blocks per CU
+template <int T>
 __global__ __launch_bounds__(256) void gram_kernel(const double2* __restrict__ y, size_t y_stride,
                                                    const int* ncols_dev, int rows_log2, int nmax,
                                                    double2* part, int nchunks) {
-  __shared__ double2 ya[32][33];
-  __shared__ double2 yb[32][33];
+  constexpr int kTile = 16 * T, kStep = 16;
+  __shared__ double2 ya[kStep][kTile];
+  __shared__ double2 yb[kStep][kTile];
   const int b = blockIdx.z;
   const int nc = ncols_dev[b];
-  const int ntile = (nmax + 31) / 32;
-  const int ti = blockIdx.x / ntile, tj = blockIdx.x % ntile;
-  if (ti * 32 >= nc || tj * 32 >= nc) return;
+  const int ntile = (nmax + kTile - 1) / kTile;
+  const int p0 = blockIdx.x / ntile * kTile, q0 = blockIdx.x % ntile * kTile;
+  if (p0 >= nc || q0 >= nc) return;
   const size_t rows = (size_t)1 << rows_log2;
   const size_t per = (rows + nchunks - 1) / nchunks;
   const size_t r0 = per * blockIdx.y;
   const size_t r1 = (r0 + per < rows) ? r0 + per : rows;
-  const double2* yb0 = y + (size_t)b * y_stride;
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  double2 acc[4] = {cz(), cz(), cz(), cz()};
-  for (size_t rb = r0; rb < r1; rb += 32) {
-    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-      int rr = e >> 5, cc = e & 31;
-      size_t row = rb + rr;
-      int ca = ti * 32 + cc, cb = tj * 32 + cc;
-      ya[rr][cc] = (row < r1 && ca < nc) ? yb0[row * nc + ca] : cz();
-      yb[rr][cc] = (row < r1 && cb < nc) ? yb0[row * nc + cb] : cz();
+  const double2* src = y + (size_t)b * y_stride;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+  double2 acc[T][T], fa[T], fb[T];
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = cz();
+  auto fetch = [&](size_t rb) {
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int e = threadIdx.x + 256 * u, rr = e / kTile, cc = e % kTile;
+      const size_t row = rb + rr;
+      fa[u] = row < r1 && p0 + cc < nc ? src[row * nc + p0 + cc] : cz();
+      fb[u] = row < r1 && q0 + cc < nc ? src[row * nc + q0 + cc] : cz();
+    }
+  };
+  fetch(r0);
+  for (size_t rb = r0; rb < r1; rb += kStep) {
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      ya[e / kTile][e % kTile] = fa[u];
+      yb[e / kTile][e % kTile] = fb[u];
     }
     __syncthreads();
+    if (rb + kStep < r1) fetch(rb + kStep);
 #pragma unroll 4
-    for (int rr = 0; rr < 32; ++rr) {
-      double2 q = yb[rr][tx];
+    for (int rr = 0; rr < kStep; ++rr) {
+      double2 av[T], bv[T];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] = cfmac(ya[rr][ty * 4 + j], q, acc[j]);
+      for (int i = 0; i < T; ++i) av[i] = ya[rr][ty + 16 * i];
+#pragma unroll
+      for (int j = 0; j < T; ++j) bv[j] = yb[rr][tx + 16 * j];
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j) acc[i][j] = cfmac(av[i], bv[j], acc[i][j]);
     }
     __syncthreads();
   }
   double2* out = part + ((size_t)b * nchunks + blockIdx.y) * nmax * nmax;
-  for (int j = 0; j < 4; ++j) {
-    int p = ti * 32 + ty * 4 + j, q = tj * 32 + tx;
-    if (p < nc && q < nc) out[(size_t)p * nmax + q] = acc[j];
-  }
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) {
+      const int p = p0 + ty + 16 * i, q = q0 + tx + 16 * j;
+      if (p < nc && q < nc) out[(size_t)p * nmax + q] = acc[i][j];
+    }
 }
 
 __global__ void gram_reduce_kernel(const double2* part, int nchunks, const int* ncols_dev, int nmax,
@@ -1013,126 +1045,146 @@ __global__ __launch_bounds__(256) void bj_store_kernel(const double2* cur_all, c
 // Sort eigenvalues (diag of A) in decreasing order, pick k (rsum2 cutoff and
 // max bond chi; k = n when n <= chi), and write the sorted eigenvectors into
 // the columns of w (same layout as v).  k_out[b] = k; spectra (optional).
+// Every block of a state sorts for itself and copies its rows of w; the first
+// one also picks k.  SELFIG
+constexpr int kSelectRows = 16;
 __global__ __launch_bounds__(512) void select_kernel(const double2* a_all, const double2* v_all,
                                                      double2* w_all, size_t stride,
                                                      const int* ncols_dev, int ld, int chi,
                                                      double cutoff, int* k_out, int kstride,
                                                      double* spectra, size_t spec_stride) {
-  __shared__ double lam[2 * kJacobiMaxPairs];
+  __shared__ double val[2 * kJacobiMaxPairs], lam[2 * kJacobiMaxPairs];
   __shared__ int perm[2 * kJacobiMaxPairs];
-  const int b = blockIdx.x;
-  const int n = ncols_dev[b];
+  const int b = blockIdx.y;
+  const int n = ncols_dev[b], row0 = blockIdx.x * kSelectRows;
+  if (row0 >= n) return;
   const double2* a = a_all + (size_t)b * stride;
   const double2* v = v_all + (size_t)b * stride;
   double2* w = w_all + (size_t)b * stride;
   // (entries that are not numbers have no rank: perm stays in range for them)
   for (int j = threadIdx.x; j < n; j += blockDim.x) {
+    val[j] = a[(size_t)j * ld + j].x;
     lam[j] = 0.0;
     perm[j] = j;
   }
   __syncthreads();
   for (int j = threadIdx.x; j < n; j += blockDim.x) {
-    double lj = a[(size_t)j * ld + j].x;
+    const double lj = val[j];
     int rank = 0;
+#pragma unroll 8
     for (int i = 0; i < n; ++i) {
-      double li = a[(size_t)i * ld + i].x;
-      if (li > lj || (li == lj && i < j)) ++rank;
+      const double li = val[i];
+      rank += li > lj || (li == lj && i < j);
     }
     lam[rank] = lj;
     perm[rank] = j;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int k;
-    if (n <= chi) {
-      k = n;
-    } else {
-      double total = 0.0;
-      for (int i = 0; i < n; ++i) total += fmax(lam[i], 0.0);
-      k = n;
-      if (total > 0.0 && cutoff > 0.0) {
-        double tail = 0.0;
-        for (int j = n - 1; j > 0; --j) {
-          tail += fmax(lam[j], 0.0);
-          if (tail <= cutoff * total) k = j; else break;
+  if (row0 == 0) {
+    if (threadIdx.x == 0) {
+      int k;
+      if (n <= chi) {
+        k = n;
+      } else {
+        double total = 0.0;
+#pragma unroll 8
+        for (int i = 0; i < n; ++i) total += fmax(lam[i], 0.0);
+        k = n;
+        if (total > 0.0 && cutoff > 0.0) {
+          double tail = 0.0;
+          for (int j = n - 1; j > 0; --j) {
+            tail += fmax(lam[j], 0.0);
+            if (tail <= cutoff * total) k = j; else break;
+          }
         }
+        if (k > chi) k = chi;
+        if (k < 1) k = 1;
       }
-      if (k > chi) k = chi;
-      if (k < 1) k = 1;
+      k_out[(size_t)b * kstride] = k;
     }
-    k_out[(size_t)b * kstride] = k;
+    if (spectra)
+      for (int j = threadIdx.x; j < n; j += blockDim.x) spectra[(size_t)b * spec_stride + j] = lam[j];
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < n * n; e += blockDim.x) {
-    int i = e / n, c = e % n;
-    w[(size_t)i * ld + c] = v[(size_t)i * ld + perm[c]];
-  }
-  if (spectra)
-    for (int j = threadIdx.x; j < n; j += blockDim.x) spectra[(size_t)b * spec_stride + j] = lam[j];
+  for (int i = row0; i < min(row0 + kSelectRows, n); ++i)
+    for (int c = threadIdx.x; c < n; c += blockDim.x) w[(size_t)i * ld + c] = v[(size_t)i * ld + perm[c]];
 }
 
 // ------------------------------------------------------------------ gemm ----
 // C (m x nc, ld nc) = A (m x kd, ld kd) * op(B); B has leading dimension ldb.
-// 64 x 64 output tile per block, 4 x 4 per thread, K in chunks of 16.
+// 16 T x 16 T entries per block, T x T per thread, K in chunks of 16 fetched
+// into registers one chunk ahead; T as in gram_kernel.  512 x
+// 600 x 300: 27 us with T = 2, 96 with 40 tiles of T = 4; 32 states of 2^13 x 128
+// x 64 and smaller: 197 us on average with T = 4.
+template <int T>
 __global__ __launch_bounds__(256) void gemm_kernel(const double2* __restrict__ a_all, size_t a_stride,
                                                    const double2* __restrict__ b_all, size_t b_stride,
                                                    double2* c_all, size_t c_stride, int rows_log2,
                                                    const int* kdim, const int* ncols, int dim_stride,
                                                    int kmax, int nmax, int ldb, int conj_b) {
-  __shared__ double2 as[64][17];
-  __shared__ double2 bs[16][65];
+  constexpr int kTile = 16 * T;
+  __shared__ double2 as[kTile][17];
+  __shared__ double2 bs[16][kTile + 1];
   const int b = blockIdx.z;
   const int kd = kdim ? kdim[(size_t)b * dim_stride] : kmax;
   const int nc = ncols ? ncols[(size_t)b * dim_stride] : nmax;
   const size_t m = (size_t)1 << rows_log2;
-  const size_t row0 = (size_t)blockIdx.y * 64;
-  const int col0 = blockIdx.x * 64;
+  const size_t row0 = (size_t)blockIdx.y * kTile;
+  const int col0 = blockIdx.x * kTile;
   if (col0 >= nc || row0 >= m) return;
   const double2* A = a_all + (size_t)b * a_stride;
   const double2* B = b_all + (size_t)b * b_stride;
   double2* C = c_all + (size_t)b * c_stride;
   const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  double2 acc[4][4];
+  double2 acc[T][T], fa[T], fb[T];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < T; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = cz();
-  for (int k0 = 0; k0 < kd; k0 += 16) {
-    for (int e = threadIdx.x; e < 64 * 16; e += 256) {
-      int rr = e >> 4, kk = e & 15;
-      size_t row = row0 + rr;
-      int kc = k0 + kk;
-      as[rr][kk] = (row < m && kc < kd) ? A[row * kd + kc] : cz();
+    for (int j = 0; j < T; ++j) acc[i][j] = cz();
+  // (B^H: the chunk index runs fastest, as it does in memory)
+  auto b_kk = [&](int e) { return conj_b ? e & 15 : e / kTile; };
+  auto b_cc = [&](int e) { return conj_b ? e >> 4 : e % kTile; };
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      const size_t row = row0 + (e >> 4);
+      const int ka = k0 + (e & 15), kb = k0 + b_kk(e), col = col0 + b_cc(e);
+      fa[u] = row < m && ka < kd ? A[row * kd + ka] : cz();
+      fb[u] = cz();
+      if (kb < kd && col < nc) fb[u] = conj_b ? cconj(B[(size_t)col * ldb + kb]) : B[(size_t)kb * ldb + col];
     }
-    for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-      int kk = e >> 6, cc = e & 63;
-      int kc = k0 + kk, col = col0 + cc;
-      double2 val = cz();
-      if (kc < kd && col < nc) val = conj_b ? cconj(B[(size_t)col * ldb + kc]) : B[(size_t)kc * ldb + col];
-      bs[kk][cc] = val;
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < kd; k0 += 16) {
+#pragma unroll
+    for (int u = 0; u < T; ++u) {
+      const int e = threadIdx.x + 256 * u;
+      as[e >> 4][e & 15] = fa[u];
+      bs[b_kk(e)][b_cc(e)] = fb[u];
     }
     __syncthreads();
+    if (k0 + 16 < kd) fetch(k0 + 16);
 #pragma unroll 4
     for (int kk = 0; kk < 16; ++kk) {
-      double2 av[4], bv[4];
+      double2 av[T], bv[T];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = as[ty * 4 + i][kk];
+      for (int i = 0; i < T; ++i) av[i] = as[ty + 16 * i][kk];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = bs[kk][tx * 4 + j];
+      for (int j = 0; j < T; ++j) bv[j] = bs[kk][tx + 16 * j];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = cfma(av[i], bv[j], acc[i][j]);
+        for (int j = 0; j < T; ++j) acc[i][j] = cfma(av[i], bv[j], acc[i][j]);
     }
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    size_t row = row0 + ty * 4 + i;
+  for (int i = 0; i < T; ++i) {
+    const size_t row = row0 + ty + 16 * i;
     if (row >= m) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      int col = col0 + tx * 4 + j;
+    for (int j = 0; j < T; ++j) {
+      const int col = col0 + tx + 16 * j;
       if (col < nc) C[row * nc + col] = acc[i][j];
     }
   }
@@ -1141,9 +1193,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(const double2* __restrict__ a
 // ------------------------------------------------------------- launchers ----
 void launch_gram(const double2* y, size_t y_stride, const int* ncols_dev, int rows_log2,
                  int ncols_max, double2* part, int nchunks, int batch, hipStream_t st) {
-  int nt = (ncols_max + 31) / 32;
-  hipLaunchKernelGGL(gram_kernel, dim3(nt * nt, nchunks, batch), dim3(256), 0, st, y, y_stride,
-                     ncols_dev, rows_log2, ncols_max, part, nchunks);
+  const long nt = (ncols_max + 63) / 64;
+  if (ncols_max > 32 && nt * nt * nchunks * batch >= kGemmFill) {
+    hipLaunchKernelGGL(gram_kernel<4>, dim3(nt * nt, nchunks, batch), dim3(256), 0, st, y, y_stride,
+                       ncols_dev, rows_log2, ncols_max, part, nchunks);
+  } else {
+    const int ns = (ncols_max + 31) / 32;
+    hipLaunchKernelGGL(gram_kernel<2>, dim3(ns * ns, nchunks, batch), dim3(256), 0, st, y, y_stride,
+                       ncols_dev, rows_log2, ncols_max, part, nchunks);
+  }
 }
 
 void launch_gram_reduce(const double2* part, int nchunks, const int* ncols_dev, int ncols_max,
@@ -1280,7 +1338,7 @@ int launch_osj(double2* a, double2* v, size_t stride, const int* ncols_dev, int 
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,
                    const int* ncols_dev, int ncols_max, int chi, double cutoff, int* k_out,
                    int kstride, double* spectra, size_t spec_stride, int batch, hipStream_t st) {
-  hipLaunchKernelGGL(select_kernel, dim3(batch), dim3(512), 0, st, a, v, w, stride, ncols_dev,
+  hipLaunchKernelGGL(select_kernel, dim3((ncols_max + kSelectRows - 1) / kSelectRows, batch), dim3(std::min(512, (ncols_max + 63) / 64 * 64)), 0, st, a, v, w, stride, ncols_dev,
                      ncols_max, chi, cutoff, k_out, kstride, spectra, spec_stride);
 }
 
@@ -1354,9 +1412,16 @@ void launch_live_list(const int* skip, int batch, int* list, hipStream_t st) {
 void launch_gemm(const double2* a, size_t a_stride, const double2* bm, size_t b_stride, double2* c,
                  size_t c_stride, const GemmDims& d, int conj_b, int batch, hipStream_t st) {
   size_t m = (size_t)1 << d.rows_log2;
-  dim3 grid((d.nmax + 63) / 64, (unsigned)((m + 63) / 64), batch);
-  hipLaunchKernelGGL(gemm_kernel, grid, dim3(256), 0, st, a, a_stride, bm, b_stride, c, c_stride,
-                     d.rows_log2, d.kdim, d.ncols, d.dim_stride, d.kmax, d.nmax, d.ldb, conj_b);
+  const size_t big = (size_t)((d.nmax + 63) / 64) * ((m + 63) / 64) * batch;
+  if (d.nmax > 32 && m > 32 && big >= (size_t)kGemmFill) {
+    dim3 grid((d.nmax + 63) / 64, (unsigned)((m + 63) / 64), batch);
+    hipLaunchKernelGGL(gemm_kernel<4>, grid, dim3(256), 0, st, a, a_stride, bm, b_stride, c, c_stride,
+                       d.rows_log2, d.kdim, d.ncols, d.dim_stride, d.kmax, d.nmax, d.ldb, conj_b);
+  } else {
+    dim3 grid((d.nmax + 31) / 32, (unsigned)((m + 31) / 32), batch);
+    hipLaunchKernelGGL(gemm_kernel<2>, grid, dim3(256), 0, st, a, a_stride, bm, b_stride, c, c_stride,
+                       d.rows_log2, d.kdim, d.ncols, d.dim_stride, d.kmax, d.nmax, d.ldb, conj_b);
+  }
 }
 
 }  // namespace qmx
