@@ -205,7 +205,8 @@ struct ChiLayout {
   int* kk;
   int* ncur;
   int* error;
-  int* jrank;        // one-sided Jacobi: Cholesky factors' column counts (nmax <= 128)
+  int* jrank;        // one-sided Jacobi: Cholesky factors' column counts (nmax > 128: 3 per state)
+  double* jdiag;     // and their remaining diagonals, then squared column norms (nmax > 128)
   double* jlog;      // two-sided LDS Jacobi: rotation log (nmax <= 128)
   int* jstate;
   char* jblock;      // block Jacobi state (nmax > 512)
@@ -236,6 +237,10 @@ ChiLayout chi_layout(Carver& c, int n, int batch, int chi, bool need_psi) {
     L.w = c.take<double2>(nm2 * batch * (i_first + 1));
     L.part = c.take<double2>(nm2 * batch * L.nchunks_max);
     if (osj_fits(L.nmax)) L.jrank = c.take<int>(batch);
+    if (osj_wide_fits(L.nmax)) {
+      L.jrank = c.take<int>(3 * static_cast<size_t>(batch));
+      L.jdiag = c.take<double>(static_cast<size_t>(L.nmax + 1) * batch);
+    }
     if (jacobi_lds_fits(L.nmax)) {
       L.jlog = c.take<double>(jacobi_lds_log_doubles(L.nmax) * batch);
       L.jstate = c.take<int>(2 * static_cast<size_t>(batch));
@@ -548,6 +553,15 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
     timer.stop(1);
     return QMX_OK;
   }
+  // Above 128 columns the one-sided solver reads its convergence on the host
+  // once per sweep, so a capturing stream keeps the two-sided ones (up to 512
+  // columns they can be captured).
+  bool wide = false;
+  if (!h->two_sided && L.jdiag) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    QMX_HIP(h, hipStreamIsCapturing(st, &cs));
+    wide = cs == hipStreamCaptureStatusNone;
+  }
   const int nmax = L.nmax;
   const size_t nm2 = static_cast<size_t>(nmax) * nmax;
   const int kmax = std::min(chi, nmax);
@@ -560,16 +574,21 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
     int nchunks = std::max(1, std::min(L.nchunks_max, rows / 256));
     launch_gram(y, len, L.ncur, i, nmax, L.part, nchunks, batch, st);
     launch_gram_reduce(L.part, nchunks, L.ncur, nmax, L.a, nm2, batch, st);
-    // sweep limits of the three eigensolvers; QMX_OPT_JACOBI_SWEEP_CAP lowers them
+    // sweep limits of the eigensolvers; QMX_OPT_JACOBI_SWEEP_CAP lowers them
     auto cap = [&](int limit) { return h->jacobi_sweep_cap > 0 ? std::min(limit, h->jacobi_sweep_cap) : limit; };
-    if (L.jblock) {
+    if (wide) {
+      std::vector<int> conv(batch);
+      if (launch_osj_wide(L.a, L.v, nm2, L.ncur, nmax, rows, batch, spectra ? 0 : chi, L.jrank, L.jdiag, conv.data(),
+                          cap(kJacobiBlockSweeps), L.error, st) != 0)
+        return fail(h, QMX_ERR_HIP, "one-sided Jacobi");
+    } else if (L.jblock) {
       std::vector<int> conv(batch);
       if (launch_jacobi_block(L.a, L.v, nm2, L.ncur, nmax, batch, L.jblock, conv.data(), cap(kJacobiBlockSweeps),
                               L.error, st) != 0)
         return fail(h, QMX_ERR_HIP, "block Jacobi");
     } else if (h->two_sided && L.jlog && jacobi_lds_setup(nmax) == hipSuccess) {
       launch_jacobi_lds(L.a, L.v, nm2, L.ncur, nmax, batch, L.jlog, L.jstate, cap(kJacobiSweeps), L.error, st);
-    } else if (!h->two_sided && L.jrank) {
+    } else if (!h->two_sided && L.jrank && !L.jdiag) {
       // (the spectra of bonds that are not truncated are wanted too if any are)
       if (launch_osj(L.a, L.v, nm2, L.ncur, nmax, batch, spectra ? 0 : chi, L.jrank, cap(kJacobiSweeps), L.error,
                      st) != 0)

@@ -331,6 +331,10 @@ void launch_jacobi_lds(double2* a, double2* v, size_t stride, const int* ncols_d
 bool osj_fits(int ncols_max);
 int launch_osj(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int batch, int keep_all,
                int* rank, int max_sweeps, int* error, hipStream_t st);
+bool osj_wide_fits(int ncols_max);
+int launch_osj_wide(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int rows, int batch,
+                    int keep_all, int* state, double* diag, int* conv_host_buf, int max_sweeps, int* error,
+                    hipStream_t st);
 void launch_jacobi(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max,
                    int batch, int max_sweeps, int* error, hipStream_t);
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,

@@ -3,7 +3,7 @@
 // Step i of the right-to-left truncated projection chain works on
 // Y_i = X_{i+1} viewed as a (2^i x n_i) row-major complex128 matrix:
 //   rho_i = Y_i^H Y_i             gram + gram_reduce   (n_i x n_i, ld = nmax)
-//   rho_i = V diag(lam) V^H       one-sided / two-sided / block Jacobi by size
+//   rho_i = V diag(lam) V^H       one-sided Jacobi (two-sided by option)
 //   W_i   = V[:, top k_i]         select               (rsum2 cutoff, max bond chi)
 //   X_i   = Y_i W_i               gemm
 // and the state is contracted back with Z_{i+1} = Z_i W_i^H (gemm, conj_b).
@@ -105,6 +105,7 @@ __global__ void gram_reduce_kernel(const double2* part, int nchunks, const int* 
 }
 
 // ---------------------------------------------------------------- jacobi ----
+// QMX_OPT_TWO_SIDED_JACOBI, and capturing streams, for 129 to 512 columns.
 // Parallel cyclic two-sided Jacobi for a Hermitian n x n matrix (n even,
 // n <= 2 * 256), one block per state.  Round r pairs the indices by the circle
 // method; all n/2 rotations of a round are disjoint, so the update
@@ -455,8 +456,8 @@ __global__ void jacobi_lds_check_kernel(const int* state, int batch, int* error)
 }
 
 // ------------------------------------ one-sided Jacobi on L -----------------
-// Eigensolver for up to 128 columns: one-sided Jacobi on the pivoted Cholesky
-// factor of the Gram matrix.
+// Eigensolver of the chain: one-sided Jacobi on the pivoted Cholesky factor of
+// the Gram matrix.
 //
 //   A = L L^H       pivoted Cholesky (largest remaining diagonal first), cut at
 //                   eps * trace: L has as many columns as A has rank
@@ -499,6 +500,12 @@ template <int NR> QMX_DEV double2 col_dot(const Col<NR>& a, const Col<NR>& b) {
   return s;
 }
 
+// the total over each quad of lanes, on all of them
+QMX_DEV double sum4(double v) {
+  v += dpp<kDppSwap>(v);
+  return v + dpp<kDppCol2>(v);
+}
+
 // Rotates the four disjoint pairs (p_k, q_k) to orthogonality.  al, be: squared
 // norms of p_k and q_k in row k of the wave, updated.  With g = p^H q and
 // d = |q|^2 - |p|^2 the smaller root of t^2 + t d / |g| - 1 = 0 gives
@@ -507,36 +514,54 @@ template <int NR> QMX_DEV double2 col_dot(const Col<NR>& a, const Col<NR>& b) {
 //   |p'|^2 = |p|^2 - t |g|,  |q'|^2 = |q|^2 + t |g|.
 // The four pairs' parameters are computed once, one pair per row, and read back
 // as scalars.  Returns whether any pair was rotated (uniform over the wave).
-template <int NR>
-QMX_DEV bool rotate4(Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>& p2, Col<NR>& q2, Col<NR>& p3,
-                     Col<NR>& q3, double& al, double& be) {
-  const double2 g0 = col_dot(p0, q0), g1 = col_dot(p1, q1), g2 = col_dot(p2, q2), g3 = col_dot(p3, q3);
-  const double2 g = make_double2(rows_total(g0.x, g1.x, g2.x, g3.x), rows_total(g0.y, g1.y, g2.y, g3.y));
+struct Rotation { double2 te; double c; };
+// (al, be, g: a pair per row of lanes; whether it is rotated in the result)
+QMX_DEV bool rotation(double2 g, double& al, double& be, double tol, Rotation& t) {
   const double ag2 = cabs2(g);
-  const bool rot = ag2 > kOsjTol * kOsjTol * al * be && ag2 > 0.0;
-  if (!__any(rot)) return false;
+  const bool rot = ag2 > tol * tol * al * be && ag2 > 0.0;
   const double d = be - al;
   const double q = fma(4.0, ag2, d * d);
   double f = 2.0 * rcp_newton(fma(q, rsqrt_newton(q), fabs(d)));
   f = rot ? (d >= 0.0 ? f : -f) : 0.0;
-  const double2 te = rot ? cscale(g, f) : cz();
-  const double c = rsqrt_newton(1.0 + cabs2(te));
+  t.te = rot ? cscale(g, f) : cz();
+  t.c = rsqrt_newton(1.0 + cabs2(t.te));
   const double tg = rot ? ag2 * f : 0.0;
   al -= tg;
   be += tg;
-  auto apply = [&](Col<NR>& p, Col<NR>& q, int k) {
-    const double tx = lane_value(te.x, 16 * k), ty = lane_value(te.y, 16 * k), cc = lane_value(c, 16 * k);
+  return rot;
+}
+// pair k's rotation, from row k of the wave
+template <int NR> QMX_DEV void rotate_pair(Col<NR>& p, Col<NR>& q, const Rotation& t, int k) {
+  const double tx = lane_value(t.te.x, 16 * k), ty = lane_value(t.te.y, 16 * k), cc = lane_value(t.c, 16 * k);
 #pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      const double2 u = p.v[r], w = q.v[r];
-      p.v[r] = make_double2(cc * fma(-tx, w.x, fma(-ty, w.y, u.x)), cc * fma(-tx, w.y, fma(ty, w.x, u.y)));
-      q.v[r] = make_double2(cc * fma(tx, u.x, fma(-ty, u.y, w.x)), cc * fma(tx, u.y, fma(ty, u.x, w.y)));
-    }
-  };
-  apply(p0, q0, 0);
-  apply(p1, q1, 1);
-  apply(p2, q2, 2);
-  apply(p3, q3, 3);
+  for (int r = 0; r < NR; ++r) {
+    const double2 u = p.v[r], w = q.v[r];
+    p.v[r] = make_double2(cc * fma(-tx, w.x, fma(-ty, w.y, u.x)), cc * fma(-tx, w.y, fma(ty, w.x, u.y)));
+    q.v[r] = make_double2(cc * fma(tx, u.x, fma(-ty, u.y, w.x)), cc * fma(tx, u.y, fma(ty, u.x, w.y)));
+  }
+}
+template <int NR>
+QMX_DEV double2 dots4(const Col<NR>& p0, const Col<NR>& q0, const Col<NR>& p1, const Col<NR>& q1, const Col<NR>& p2,
+                      const Col<NR>& q2, const Col<NR>& p3, const Col<NR>& q3) {
+  const double2 g0 = col_dot(p0, q0), g1 = col_dot(p1, q1), g2 = col_dot(p2, q2), g3 = col_dot(p3, q3);
+  return make_double2(rows_total(g0.x, g1.x, g2.x, g3.x), rows_total(g0.y, g1.y, g2.y, g3.y));
+}
+template <int NR>
+QMX_DEV double norms4(const Col<NR>& p0, const Col<NR>& p1, const Col<NR>& p2, const Col<NR>& p3) {
+  return rows_total(col_norm(p0), col_norm(p1), col_norm(p2), col_norm(p3));
+}
+// (total: sums a value per row of lanes over the waves that share the columns)
+template <int NR, typename F>
+QMX_DEV bool rotate4(Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>& p2, Col<NR>& q2, Col<NR>& p3,
+                     Col<NR>& q3, double& al, double& be, double tol, F total) {
+  const double2 g = total(dots4(p0, q0, p1, q1, p2, q2, p3, q3));
+  if (!__any(cabs2(g) > tol * tol * al * be)) return false;
+  Rotation t;
+  rotation(g, al, be, tol, t);
+  rotate_pair(p0, q0, t, 0);
+  rotate_pair(p1, q1, t, 1);
+  rotate_pair(p2, q2, t, 2);
+  rotate_pair(p3, q3, t, 3);
   return true;
 }
 
@@ -702,6 +727,7 @@ __global__ __launch_bounds__(NR == 2 ? 1024 : 512) void osj_kernel(double2* a_al
     nrm = nbuf[s][lane >> 4];
   };
   bool converged = false;
+  auto own = [](double2 g) { return g; };   // a column is one wave's
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
     bool rot = false;
     double nt = 0.0, nq = 0.0;   // squared norms: row k of the wave, column k of the top / bottom block
@@ -710,7 +736,7 @@ __global__ __launch_bounds__(NR == 2 ? 1024 : 512) void osj_kernel(double2* a_al
                         Col<NR>& q3) {
         double al = rows_total(col_norm(p0), col_norm(p1), col_norm(p2), col_norm(p3));
         double be = rows_total(col_norm(q0), col_norm(q1), col_norm(q2), col_norm(q3));
-        rot |= rotate4(p0, q0, p1, q1, p2, q2, p3, q3, al, be);
+        rot |= rotate4(p0, q0, p1, q1, p2, q2, p3, q3, al, be, kOsjTol, own);
       };
       inside(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
       inside(x[0], x[2], x[1], x[3], x[4], x[6], x[5], x[7]);
@@ -722,13 +748,13 @@ __global__ __launch_bounds__(NR == 2 ? 1024 : 512) void osj_kernel(double2* a_al
       if (live) {
         // set s: pairs (top k, bottom (k + s) % 4); the bottom norms move up one row per set
         auto next = [&]() { nq = __shfl(nq, (lane + 16) & 63, 64); };
-        rot |= rotate4(x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7], nt, nq);
+        rot |= rotate4(x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7], nt, nq, kOsjTol, own);
         next();
-        rot |= rotate4(x[0], x[5], x[1], x[6], x[2], x[7], x[3], x[4], nt, nq);
+        rot |= rotate4(x[0], x[5], x[1], x[6], x[2], x[7], x[3], x[4], nt, nq, kOsjTol, own);
         next();
-        rot |= rotate4(x[0], x[6], x[1], x[7], x[2], x[4], x[3], x[5], nt, nq);
+        rot |= rotate4(x[0], x[6], x[1], x[7], x[2], x[4], x[3], x[5], nt, nq, kOsjTol, own);
         next();
-        rot |= rotate4(x[0], x[7], x[1], x[4], x[2], x[5], x[3], x[6], nt, nq);
+        rot |= rotate4(x[0], x[7], x[1], x[4], x[2], x[5], x[3], x[6], nt, nq, kOsjTol, own);
         next();
       }
       if (m == 1) continue;   // two blocks: the only pair
@@ -787,9 +813,322 @@ QMX_DEV void circle_pair(int n, int r, int m, int& p, int& q) {
   if (p > q) { const int t = p; p = q; q = t; }
 }
 
+// ------------------------------------------- 129 to 1024 columns -----------
+// The same eigensolver with a state's columns spread over the chip.
+//
+// Cholesky: panels of kPcPanel pivots.  One block per state takes a panel's
+// pivots (thread = row, its entries of the panel's columns in registers; the
+// pivot search and one column of A per step, two barriers), then the whole grid
+// subtracts the panel from A.  Bound by the latency of the panel's steps; each
+// panel reads and writes A once, which a step by step update would do
+// kPcPanel times.
+// Jacobi: L's columns lie one after the other in V's storage, 4 to a block of
+// columns; one launch per round of the circle method, one thread block per pair
+// of column blocks: rows spread over its four waves, one to a SIMD, the columns
+// in registers, each set of four pairs' products summed over the waves through
+// LDS.  Blocks of 8 columns would halve the launches, but run twice the sets on
+// half the CUs (21 us a round against 8.4 at 600 columns, two rows a lane).  The launches of a sweep are bound by their own latency while a
+// state has at most 512 columns (7.2 us a round at 512 to
+// 600 columns, 3.4 to 4 without rotations; 8 to 9 sweeps).  One state of N = 18
+// at chi = 300: 16.2 ms here and 1.7 in the Cholesky factors of five matrices of
+// 512 and 600 columns; the two-sided block Jacobi below 176 + 108 ms.
+// L is cut at max_rank columns, the number of rows the Gram matrix was formed
+// from: more are rounding errors.
+constexpr int kOsjWide = 1024;
+constexpr int kPcPanel = 16;
+
+// Panel k0 of the pivoted Cholesky factor.  diag: the remaining diagonal
+// (-infinity: a pivot already) and, at ld, the trace.  rank: columns of L so
+// far, the result once a panel comes out short; -1 as in chol_kernel.
+__global__ __launch_bounds__(kOsjWide) void pchol_panel_kernel(const double2* a_all, double2* l_all, size_t stride,
+                                                               const int* ncols_dev, int ld, int keep_all, int k0,
+                                                               int max_rank, int* rank_all, double* diag_all) {
+  __shared__ double wbest[16];
+  __shared__ int wpiv[16];
+  __shared__ double2 lp[kPcPanel];
+  const int b = blockIdx.x;
+  const int n = ncols_dev[b];
+  const double2* a = a_all + (size_t)b * stride;
+  double2* l_out = l_all + (size_t)b * stride;
+  double* diag = diag_all + (size_t)b * (ld + 1);
+  const int row = threadIdx.x, lane = row & 63, wave = __builtin_amdgcn_readfirstlane(row >> 6);
+  const double inf = __builtin_inf();
+  double d, tr;
+  if (row < 16) wbest[row] = k0 == 0 ? 0.0 : -inf;   // (waves that a narrow launch has not)
+  __syncthreads();
+  if (k0 == 0) {
+    if (n <= keep_all) {
+      if (row == 0) rank_all[b] = -1;
+      return;
+    }
+    d = row < n ? a[(size_t)row * ld + row].x : 0.0;
+    const double w = rows_sum(sum16(d));
+    if (lane == 0) wbest[wave] = w;
+    __syncthreads();
+    tr = 0.0;
+    for (int k = 0; k < 16; ++k) tr += wbest[k];
+    __syncthreads();   // (wbest is written again below)
+    if (!(tr > 0.0) || !(tr < 1e300)) {
+      if (row == 0) rank_all[b] = -1;
+      return;
+    }
+    if (row == 0) diag[ld] = tr;
+    if (row < 16) wbest[row] = -inf;
+    if (row >= n) d = -inf;
+  } else {
+    if (rank_all[b] != k0) return;
+    d = row < n ? diag[row] : -inf;
+    tr = diag[ld];
+  }
+  double2 l[kPcPanel];
+#pragma unroll
+  for (int t = 0; t < kPcPanel; ++t) l[t] = cz();
+  int rank = k0;
+  bool run = true;
+#pragma unroll
+  for (int j = 0; j < kPcPanel; ++j) {
+    if (run) {
+      // largest remaining diagonal entry, lowest index on ties
+      auto max16 = [](double v) {
+        v = fmax(v, dpp<kDppRow2>(v));
+        v = fmax(v, dpp<kDppRow1>(v));
+        v = fmax(v, dpp<kDppCol2>(v));
+        return fmax(v, dpp<kDppSwap>(v));
+      };
+      double m = max16(d);
+      m = fmax(m, __shfl_xor(m, 16, 64));
+      m = fmax(m, __shfl_xor(m, 32, 64));
+      const unsigned long long at = __ballot(d == m);
+      if (lane == 0) {
+        wbest[wave] = m;
+        wpiv[wave] = 64 * wave + __ffsll(at) - 1;
+      }
+      __syncthreads();
+      const double wm = wbest[lane & 15], best = max16(wm);
+      const int wsel = __ffsll(__ballot(wm == best)) - 1;
+      const int p = __builtin_amdgcn_readfirstlane(wpiv[wsel & 15]);
+      if (best > kEps * tr && rank < max_rank && rank < n) {
+        // (a column of the Hermitian matrix is its conjugated row: contiguous loads)
+        double2 x = row < n ? cconj(a[(size_t)p * ld + row]) : cz();
+        if (row == p)
+#pragma unroll
+          for (int t = 0; t < kPcPanel; ++t) lp[t] = l[t];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < j; ++t) {
+          const double2 c = lp[t];   // x -= l conj(c)
+          x.x = fma(-l[t].x, c.x, fma(-l[t].y, c.y, x.x));
+          x.y = fma(-l[t].y, c.x, fma(l[t].x, c.y, x.y));
+        }
+        const double inv = rsqrt_newton(best);
+        x = d == -inf ? cz() : (row == p ? make_double2(best * inv, 0.0) : cscale(x, inv));
+        l[j] = x;
+        if (row < n) l_out[(size_t)rank * ld + row] = x;
+        d = row == p ? -inf : d - cabs2(x);
+        ++rank;
+      } else {
+        run = false;
+      }
+    }
+  }
+  if (row < n) diag[row] = d;
+  if (row == 0) rank_all[b] = rank;
+}
+
+// A -= L_panel L_panel^H, 64 x 64 entries per block, for the states whose panel
+// k0 is full
+__global__ __launch_bounds__(256) void pchol_update_kernel(double2* a_all, const double2* l_all, size_t stride,
+                                                           const int* ncols_dev, int ld, int k0, int ntile,
+                                                           const int* rank_all) {
+  __shared__ double2 li[kPcPanel][64], lj[kPcPanel][64];
+  const int b = blockIdx.y;
+  const int n = ncols_dev[b], i0 = blockIdx.x / ntile * 64, j0 = blockIdx.x % ntile * 64;
+  if (rank_all[b] < k0 + kPcPanel || i0 >= n || j0 >= n) return;
+  double2* a = a_all + (size_t)b * stride;
+  const double2* l = l_all + (size_t)b * stride + (size_t)k0 * ld;
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  for (int e = tid; e < kPcPanel * 64; e += 256) {
+    const int t = e >> 6, r = e & 63;
+    li[t][r] = i0 + r < n ? l[(size_t)t * ld + i0 + r] : cz();
+    lj[t][r] = j0 + r < n ? l[(size_t)t * ld + j0 + r] : cz();
+  }
+  __syncthreads();
+  double2 acc[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) acc[u][w] = cz();
+#pragma unroll 2
+  for (int t = 0; t < kPcPanel; ++t) {
+    double2 x[4], y[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = li[t][ty + 16 * u];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) y[w] = lj[t][tx + 16 * w];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) acc[u][w] = cfmac(y[w], x[u], acc[u][w]);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * w;
+      if (i < n && j < n) {
+        double2* e = a + (size_t)i * ld + j;
+        *e = csub(*e, acc[u][w]);
+      }
+    }
+}
+
+// Round r of a sweep over nb blocks of four columns: pair blockIdx.x of state
+// blockIdx.y.  Round 0 also rotates the pairs inside the blocks and forms the
+// squared norms, which later rounds read from nrm and update.
+template <int NR>
+__global__ __launch_bounds__(256) void osj_round_kernel(double2* l_all, size_t stride, int ld, const int* ncols_dev,
+                                                        const int* rank_all, int nb, int r, double tol,
+                                                        double* nrm_all, const int* conv, int* rot_all) {
+  __shared__ double2 gpart[2][4][4];
+  const int b = blockIdx.y;
+  const int rank = rank_all[b];
+  if (conv[b]) return;
+  int I, J;
+  circle_pair(nb, r, blockIdx.x, I, J);
+  if (4 * (r == 0 ? I : J) >= rank) return;   // I < J: nothing but zero columns to pair
+  const int n = ncols_dev[b];
+  double2* l = l_all + (size_t)b * stride;
+  double* nrm = nrm_all + (size_t)b * (ld + 1);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = wave * 64 * NR + lane;
+  auto column = [&](int c) { return c < 4 ? 4 * I + c : 4 * J + c - 4; };
+  Col<NR> x[8];   // block I, block J
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+      const int k = column(c), row = row0 + 64 * h;
+      x[c].v[h] = k < rank && row < n ? l[(size_t)k * ld + row] : cz();
+    }
+  int par = 0;
+  auto total = [&](double2 g) {
+    if ((lane & 15) == 0) gpart[par][lane >> 4][wave] = g;
+    __syncthreads();
+    const double2 t = gpart[par][lane >> 4][lane & 3];
+    par ^= 1;   // the next sum's values go to the other half: one barrier per sum
+    return make_double2(sum4(t.x), sum4(t.y));
+  };
+  bool rot = false;
+  double nt, nq;   // squared norms: row k of the wave, column k of block I / J
+  if (r == 0) {
+    auto inside = [&](Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>& p2, Col<NR>& q2, Col<NR>& p3,
+                      Col<NR>& q3) {
+      double2 t = total(make_double2(norms4(p0, p1, p2, p3), norms4(q0, q1, q2, q3)));
+      rot |= rotate4(p0, q0, p1, q1, p2, q2, p3, q3, t.x, t.y, tol, total);
+    };
+    inside(x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]);
+    inside(x[0], x[2], x[1], x[3], x[4], x[6], x[5], x[7]);
+    inside(x[0], x[3], x[1], x[2], x[4], x[7], x[5], x[6]);
+    const double2 t = total(make_double2(norms4(x[0], x[1], x[2], x[3]), norms4(x[4], x[5], x[6], x[7])));
+    nt = t.x;
+    nq = t.y;
+  } else {
+    const int k = lane >> 4;
+    nt = 4 * I + k < rank ? nrm[4 * I + k] : 0.0;
+    nq = 4 * J + k < rank ? nrm[4 * J + k] : 0.0;
+  }
+  // set s: pairs (top k, bottom (k + s) % 4); the bottom norms move up one row per set
+  auto next = [&]() { nq = __shfl(nq, (lane + 16) & 63, 64); };
+  rot |= rotate4(x[0], x[4], x[1], x[5], x[2], x[6], x[3], x[7], nt, nq, tol, total);
+  next();
+  rot |= rotate4(x[0], x[5], x[1], x[6], x[2], x[7], x[3], x[4], nt, nq, tol, total);
+  next();
+  rot |= rotate4(x[0], x[6], x[1], x[7], x[2], x[4], x[3], x[5], nt, nq, tol, total);
+  next();
+  rot |= rotate4(x[0], x[7], x[1], x[4], x[2], x[5], x[3], x[6], nt, nq, tol, total);
+  next();
+  if (wave == 0 && (lane & 15) == 0 && (rot || r == 0)) {
+    const int k = lane >> 4;
+    if (4 * I + k < rank) nrm[4 * I + k] = nt;
+    if (4 * J + k < rank) nrm[4 * J + k] = nq;
+  }
+  if (!rot) return;
+  if (threadIdx.x == 0) rot_all[b] = 1;
+#pragma unroll
+  for (int c = 0; c < 8; ++c)
+#pragma unroll
+    for (int h = 0; h < NR; ++h) {
+      const int k = column(c), row = row0 + 64 * h;
+      if (k < rank && row < n) l[(size_t)k * ld + row] = x[c].v[h];
+    }
+}
+
+__global__ void osj_wide_begin_kernel(const int* rank_all, int* conv, int* rot, int batch) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= batch) return;
+  conv[b] = rank_all[b] <= 1;
+  rot[b] = 0;
+}
+
+// eigenvalues to A's diagonal, one wave per column
+__global__ __launch_bounds__(256) void osj_values_kernel(double2* a_all, const double2* l_all, size_t stride, int ld,
+                                                         const int* ncols_dev, const int* rank_all, const int* conv,
+                                                         int* error) {
+  const int b = blockIdx.y;
+  const int n = ncols_dev[b], rank = rank_all[b];
+  const int k = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (k == 0 && lane == 0 && !conv[b]) atomicOr(error, kErrEigNoConv);
+  if (rank < 0 || k >= n) return;
+  double s = 0.0;
+  if (k < rank)
+    for (int row = lane; row < n; row += 64) s += cabs2(l_all[(size_t)b * stride + (size_t)k * ld + row]);
+  s = rows_sum(sum16(s));
+  if (lane == 0) a_all[(size_t)b * stride + (size_t)k * ld + k] = make_double2(s, 0.0);
+}
+
+// eigenvectors: V[row][k] = L[k][row] / |L_k|, transposed in place by pairs of
+// 32 x 32 tiles; the identity for a state that is not truncated
+__global__ __launch_bounds__(256) void osj_vectors_kernel(const double2* a_all, double2* v_all, size_t stride, int ld,
+                                                          const int* ncols_dev, const int* rank_all, int ntile) {
+  __shared__ double2 t0[32][33], t1[32][33];
+  const int b = blockIdx.y;
+  const int n = ncols_dev[b], rank = rank_all[b];
+  const int ti = blockIdx.x / ntile, tj = blockIdx.x % ntile;
+  if (ti > tj || 32 * ti >= n || 32 * tj >= n) return;
+  const double2* a = a_all + (size_t)b * stride;
+  double2* v = v_all + (size_t)b * stride;
+  const int x = threadIdx.x & 31, y0 = threadIdx.x >> 5;
+  auto load = [&](double2 (&t)[32][33], int tk, int tr) {   // columns of tile tk, rows of tile tr
+    for (int y = y0; y < 32; y += 8) {
+      const int k = 32 * tk + y, row = 32 * tr + x;
+      double2 e = cz();
+      if (k < n && row < n) {
+        if (rank < 0) {
+          e = make_double2(k == row ? 1.0 : 0.0, 0.0);
+        } else if (k < rank) {
+          const double nn = a[(size_t)k * ld + k].x;
+          e = cscale(v[(size_t)k * ld + row], nn > 0.0 ? rsqrt_newton(nn) : 0.0);
+        }
+      }
+      t[y][x] = e;
+    }
+  };
+  auto store = [&](const double2 (&t)[32][33], int tk, int tr) {
+    for (int y = y0; y < 32; y += 8) {
+      const int row = 32 * tr + y, k = 32 * tk + x;
+      if (k < n && row < n) v[(size_t)row * ld + k] = t[x][y];
+    }
+  };
+  load(t0, ti, tj);
+  if (ti != tj) load(t1, tj, ti);
+  __syncthreads();
+  store(t0, ti, tj);
+  if (ti != tj) store(t1, tj, ti);
+}
+
 // ----------------------------------------------------- block Jacobi -------
-// For Gram matrices too large for one workgroup (n > 512, chi > 256): a
-// two-sided block Jacobi over blocks of kBjBs columns.  The matrix is copied
+// QMX_OPT_TWO_SIDED_JACOBI for Gram matrices too large for one workgroup (n >
+// 512, chi > 256): a two-sided block Jacobi over blocks of kBjBs columns.  The matrix is copied
 // into an npad x npad buffer (npad = n rounded up to 2 kBjBs, zero padding:
 // padded indices are never rotated, as every off-diagonal entry they have is
 // zero), and the nb = npad / kBjBs blocks are paired by the same circle
@@ -1332,6 +1671,49 @@ int launch_osj(double2* a, double2* v, size_t stride, const int* ncols_dev, int 
     hipLaunchKernelGGL(osj_kernel<2>, dim3(batch), dim3(64 * waves), shm, st, a, v, stride, ncols_dev, ncols_max,
                        rank, max_sweeps, error);
   }
+  return 0;
+}
+
+bool osj_wide_fits(int ncols_max) { return ncols_max > kOsjMax && ncols_max <= kOsjWide; }
+
+// state: 3 ints per state (rank, converged, rotated); diag: ncols_max + 1
+// doubles per state.  rows: of the matrix that the Gram matrices belong to.
+int launch_osj_wide(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max, int rows, int batch,
+                    int keep_all, int* state, double* diag, int* conv_host_buf, int max_sweeps, int* error,
+                    hipStream_t st) {
+  const int max_rank = std::min(ncols_max, rows);
+  int *rank = state, *conv = state + batch, *rot = conv + batch;
+  const int ut = (ncols_max + 63) / 64, vt = (ncols_max + 31) / 32;
+  const int threads = (ncols_max + 63) / 64 * 64;
+  for (int k0 = 0; k0 < max_rank; k0 += kPcPanel) {
+    hipLaunchKernelGGL(pchol_panel_kernel, dim3(batch), dim3(threads), 0, st, a, v, stride, ncols_dev, ncols_max,
+                       keep_all, k0, max_rank, rank, diag);
+    if (k0 + kPcPanel < max_rank)
+      hipLaunchKernelGGL(pchol_update_kernel, dim3(ut * ut, batch), dim3(256), 0, st, a, v, stride, ncols_dev,
+                         ncols_max, k0, ut, rank);
+  }
+  hipLaunchKernelGGL(osj_wide_begin_kernel, dim3((batch + 255) / 256), dim3(256), 0, st, rank, conv, rot, batch);
+  const int nb = ((max_rank + 3) / 4 + 1) & ~1;
+  auto* const round = ncols_max <= 256 ? osj_round_kernel<1> : ncols_max <= 512 ? osj_round_kernel<2>
+                    : ncols_max <= 768 ? osj_round_kernel<3> : osj_round_kernel<4>;
+  const double tol = kOsjTol * std::sqrt(std::max(1.0, ncols_max / 128.0));
+  for (int s = 0; s < max_sweeps; ++s) {
+    for (int r = 0; r < nb - 1; ++r)
+      hipLaunchKernelGGL(round, dim3(nb / 2, batch), dim3(256), 0, st, v, stride, ncols_max,
+                         ncols_dev, rank, nb, r, tol, diag, conv, rot);
+    hipLaunchKernelGGL(bj_sweep_end_kernel, dim3((batch + 255) / 256), dim3(256), 0, st, conv, rot, batch);
+    // stop once every state has converged (one host read per sweep)
+    if (hipMemcpyAsync(conv_host_buf, conv, sizeof(int) * batch, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess)
+      return -1;
+    bool all = true;
+    for (int b = 0; b < batch; ++b) all = all && conv_host_buf[b];
+    if (all) break;
+  }
+  hipLaunchKernelGGL(osj_values_kernel, dim3((ncols_max + 3) / 4, batch), dim3(256), 0, st, a, v, stride, ncols_max,
+                     ncols_dev, rank, conv, error);
+  hipLaunchKernelGGL(osj_vectors_kernel, dim3(vt * vt, batch), dim3(256), 0, st, a, v, stride, ncols_max, ncols_dev,
+                     rank, vt);
   return 0;
 }
 

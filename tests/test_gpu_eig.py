@@ -1,8 +1,8 @@
 """The chi-truncation's one-sided Jacobi at the edges of its sizes and ranks.
 
-Column counts n = 2 chi around 8 (one wave), 64 and 128 (its limits), with
-Gram matrices of full rank, of fewer rows than columns, and with clusters of
-equal eigenvalues.
+Column counts n = 2 chi around 8 (one wave), 64 and 128 (the one-block limits)
+and up to 800 (spread over the chip), with Gram matrices of full rank, of fewer
+rows than columns, and with clusters of equal eigenvalues.
 """
 
 import numpy as np
@@ -60,6 +60,41 @@ def test_equal_eigenvalues(gpu, pairs, chi):
     for sv, m in ((psi, n), (wide, n + 1)):
         _, target, _ = eng.chi_truncate(eng.as_device_states(sv), chi)
         assert np.linalg.norm(target[0].cpu().numpy() - sv) < 1e-7, m
+
+
+@pytest.mark.parametrize("n,chi,kind", [(14, 65, "uniform"), (14, 65, "mps"), (15, 100, "mps"), (16, 128, "uniform"),
+                                        (16, 129, "uniform"), (17, 200, "mps"), (17, 256, "uniform"),
+                                        (17, 257, "mps"), (19, 400, "uniform")])
+def test_truncation_above_128_columns(gpu, n, chi, kind):
+    """130 to 800 columns, one to four rows per lane, Gram matrices of full
+    rank and of fewer rows than columns; same bars as above."""
+    eng = _engine()
+    seeds = (1, 2) if n < 17 else (1,)
+    svs = [O.random_uniform_state(n, s) if kind == "uniform" else O.random_mps_state(n, chi + chi // 2, s)
+           for s in seeds]
+    _, target, spec = eng.chi_truncate(eng.as_device_states(np.stack(svs)), chi, spectra=True)
+    _, plain, _ = eng.chi_truncate(eng.as_device_states(np.stack(svs)), chi)
+    for k, sv in enumerate(svs):
+        ref, ref_spec = O.chi_truncate(O.ket(sv), n, chi)
+        for got in (target, plain):
+            err = np.linalg.norm(got[k].cpu().numpy() - ref) / np.linalg.norm(ref)
+            print(f"n={n} chi={chi} {kind} state {k} rel.err {err:.2e}")
+            assert err < (1e-10 if kind == "uniform" else 1e-9)
+        for i, lam in enumerate(ref_spec):
+            if lam is not None:
+                kk = min(len(lam), chi)
+                assert np.max(np.abs(spec[k, i, :kk].cpu().numpy() - lam[:kk])) < 1e-12 * lam[0]
+
+
+def test_wide_batch_with_a_state_that_is_not_a_number(gpu):
+    eng = _engine()
+    sv = np.stack([O.random_uniform_state(14, s) for s in (4, 5, 6)])
+    _, ref, _ = eng.chi_truncate(eng.as_device_states(sv), 70)
+    bad = sv.copy()
+    bad[1, 3] = np.nan
+    _, got, _ = eng.chi_truncate(eng.as_device_states(bad), 70)
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[2], ref[2])
+    assert not bool(torch.isfinite(torch.view_as_real(got[1])).all())
 
 
 def test_state_that_is_not_a_number_stays_alone(gpu):
