@@ -77,6 +77,25 @@ def test_mlp_backward_matches_oracle(gpu, rows, width):
         assert err < 2e-2, name
 
 
+@pytest.mark.parametrize("rows,width", [(1, 33), (31, 100), (257, 66), (300, 30), (1030, 24), (4100, 520)])
+def test_mlp_odd_sizes(gpu, rows, width):
+    """Rows and widths off the tile edges, operands that wide loads cannot
+    take, and a grid of 64 x 64 tiles; the bars of the two tests above, which
+    are those of BF16 operands."""
+    net = _net(width)
+    p = _rand_params(net, 7)
+    xg, x = _rand_x(rows, net.in_dim, 8)
+    rng = np.random.default_rng(9)
+    dy = rng.standard_normal((rows, net.out_dim)).astype(np.float32)
+    dims = (net.in_dim, width, net.out_dim)
+    y = net.forward(xg).cpu().numpy().astype(np.float64)
+    g = net.backward(xg, torch.from_numpy(dy).cuda()).cpu().numpy().astype(np.float64)
+    want, cache = M.forward(x, p, dims)
+    assert np.linalg.norm(y - want) < 5e-3 * np.linalg.norm(want)
+    for a, b in zip(M.unpack(g, *dims), M.unpack(M.backward(dy.astype(np.float64), cache, dims), *dims)):
+        assert np.linalg.norm(a - b) < 2e-2 * max(np.linalg.norm(b), 1e-30)
+
+
 def test_adam_matches_oracle(gpu):
     net = _net(64)
     p = _rand_params(net, 6)
