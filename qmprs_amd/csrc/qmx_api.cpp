@@ -625,6 +625,7 @@ int run_generate_layer(qmx_handle* h, int n, int batch, int lmax, int layer, dou
     Chain2Args a{};
     a.n = n;
     a.step = i;
+    a.serial = h->two_sided;
     a.cutoff = cutoff;
     a.psi = psi_w;
     a.xa = L.xa;

@@ -250,6 +250,15 @@ QMX_DEV double rows_sum(double v) {
   return swap_add16(v, v);
 }
 
+template <int J> QMX_DEV double quad_bcast(double v) { return dpp<J * 0x55>(v); }
+template <int J> QMX_DEV double2 quad_bcast2(double2 v) { return make_double2(quad_bcast<J>(v.x), quad_bcast<J>(v.y)); }
+// The totals over the wave of four per-lane values: row k (lanes 16 k ..
+// 16 k + 15) holds the total of v_k on every lane.  Two half-swaps merge the
+// four registers, then four DPP steps add inside the rows.
+QMX_DEV double rows_total(double v0, double v1, double v2, double v3) {
+  return sum16(swap_add16(swap_add32(v0, v2), swap_add32(v1, v3)));
+}
+
 // 1 / x to rounding: the hardware estimate and two Newton steps
 QMX_DEV double rcp_newton(double x) {
   double r = __builtin_amdgcn_rcp(x);
@@ -263,6 +272,78 @@ QMX_DEV double rsqrt_newton(double x) {
   const double h = 0.5 * x;
   r = fma(r, fma(-h * r, r, 0.5), r);
   return fma(r, fma(-h * r, r, 0.5), r);
+}
+
+// ---- 4 x 4 Hermitian eigenproblem on one wave -----------------------------------
+// Two-sided Jacobi with entry (i, j) of A and V in lane 4 i + j: the two
+// disjoint rotations of a round run side by side (rounds pair an index with
+// itself ^ X, X = 1, 2, 3), every entry is updated by its own lane.  With
+// d = a_qq - a_pp, g = a_pq, the rotation p' = c (p - conj(te) q), q' = c (q +
+// te p) has te = 2 g sign(d) / (|d| + sqrt(d^2 + 4 |g|^2)) and c = 1 / sqrt(1 +
+// |te|^2); w is the weight of an index's partner, -conj(te) or te.
+// Bound by the chain of a round's dependent operations; a step of the layers'
+// chain at N = 10, which is mostly this, takes 11.3 us, with the one-lane solver
+// above 28.
+template <int X> QMX_DEV double2 row_partner(double2 v) {   // lane ^ 4 X
+  if constexpr (X == 2) return make_double2(dpp<kDppRow2>(v.x), dpp<kDppRow2>(v.y));
+  // mirrored within 8 or 16 lanes, the quads turned back
+  constexpr int mirror = X == 1 ? 0x141 : 0x140;
+  return make_double2(dpp<mirror>(dpp<0x1b>(v.x)), dpp<mirror>(dpp<0x1b>(v.y)));
+}
+template <int X> QMX_DEV double2 col_partner(double2 v) {   // lane ^ X
+  constexpr int perm = X == 1 ? kDppSwap : X == 2 ? kDppCol2 : 0x1b;
+  return make_double2(dpp<perm>(v.x), dpp<perm>(v.y));
+}
+template <int X> QMX_DEV void herm_eig4_round(double2& a, double2& v, int i, int j) {
+  constexpr int kP = X == 1 ? 2 : 1, kQ = kP ^ X;   // the pair beside (0, X)
+  const bool jf = j == 0 || j == X, jq = j > (j ^ X), fi = i == 0 || i == X, iq = i > (i ^ X);
+  const double al = jf ? lane_value(a.x, 0) : lane_value(a.x, 5 * kP);
+  const double be = jf ? lane_value(a.x, 5 * X) : lane_value(a.x, 5 * kQ);
+  const double2 g = make_double2(jf ? lane_value(a.x, X) : lane_value(a.x, 4 * kP + kQ),
+                                 jf ? lane_value(a.y, X) : lane_value(a.y, 4 * kP + kQ));
+  const double ag2 = cabs2(g), d = be - al;
+  const bool rot = ag2 > 1e-280;
+  const double q = fma(4.0, ag2, d * d);
+  double f = 2.0 * rcp_newton(fma(q, rsqrt_newton(q), fabs(d)));
+  f = rot ? (d >= 0.0 ? f : -f) : 0.0;
+  const double2 te = rot ? cscale(g, f) : cz();
+  const double c = rsqrt_newton(1.0 + cabs2(te));
+  const double2 w = jq ? te : make_double2(-te.x, te.y);
+  // the same of this lane's row index, from its quad
+  const double2 w0 = quad_bcast2<0>(w), w1 = quad_bcast2<kP>(w);
+  const double cr = fi ? quad_bcast<0>(c) : quad_bcast<kP>(c);
+  double2 wr = fi ? w0 : w1;                      // of the pair's first index: -conj(te)
+  if (iq) wr = make_double2(-wr.x, wr.y);
+  const double2 ac = cscale(cfma(w, col_partner<X>(a), a), c);
+  v = cscale(cfma(w, col_partner<X>(v), v), c);
+  a = cscale(cfmac(wr, row_partner<X>(ac), ac), cr);
+  if (i == j) a.y = 0.0;
+  if (rot && i == (j ^ X)) a = cz();
+}
+// Eigenvalues of the matrix a (entry (i, j) in lane 4 i + j, the same in each
+// row of 16 lanes) in decreasing order to lam[4] and the eigenvectors to the columns of vec[16],
+// both in LDS; a matrix that is not finite gives vectors that are not.
+QMX_DEV void herm_eig4_wave(double2 a, int lane, double* lam, double2* vec) {
+  const int i = (lane >> 2) & 3, j = lane & 3;
+  double2 v = make_double2(i == j ? 1.0 : 0.0, 0.0);
+  const double all = sum16(cabs2(a));
+  for (int sweep = 0; sweep < 40; ++sweep) {
+    const double off = sum16(i < j ? cabs2(a) : 0.0), diag = sum16(i == j ? a.x * a.x : 0.0);
+    if (off <= 1e-32 * diag || off < 1e-270) break;
+    herm_eig4_round<1>(a, v, i, j);
+    herm_eig4_round<2>(a, v, i, j);
+    herm_eig4_round<3>(a, v, i, j);
+  }
+  // place of column j: stable, decreasing
+  const double l0 = lane_value(a.x, 0), l1 = lane_value(a.x, 5), l2 = lane_value(a.x, 10), l3 = lane_value(a.x, 15);
+  const double lj = j == 0 ? l0 : j == 1 ? l1 : j == 2 ? l2 : l3;
+  const int at = (l0 > lj || (l0 == lj && 0 < j)) + (l1 > lj || (l1 == lj && 1 < j)) +
+                 (l2 > lj || (l2 == lj && 2 < j)) + (l3 > lj || (l3 == lj && 3 < j));
+  const double bad = 0.0 * all;
+  if (lane < 16) {
+    vec[4 * i + at] = make_double2(v.x + bad, v.y + bad);
+    if (i == j) lam[at] = lj;
+  }
 }
 
 // ---- 4 x 4 complex products on the matrix cores --------------------------------
@@ -371,8 +452,6 @@ QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc)
 // (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry (i, j) of
 // the factor.  False where the Jacobi path decides (30600 cycles); 2700
 // cycles, against 5300 to 7500 with the whole problem in every lane.
-template <int J> QMX_DEV double quad_bcast(double v) { return dpp<J * 0x55>(v); }
-template <int J> QMX_DEV double2 quad_bcast2(double2 v) { return make_double2(quad_bcast<J>(v.x), quad_bcast<J>(v.y)); }
 // sum over the 4 rows i
 QMX_DEV double col_total(double v) {
   v += dpp<kDppRow2>(v);

@@ -199,6 +199,7 @@ struct WinFinArgs {
 
 struct Chain2Args {
   int n, step;
+  int serial;          // the kept subspace in one lane (QMX_OPT_TWO_SIDED_JACOBI)
   double cutoff;
   const double2* psi;  // X_N (normalised working state)
   double2* xa;

@@ -126,14 +126,23 @@ QMX_DEV uint64_t gate_bits(int n, int site, int width) {
 }
 
 // Block-wide sum of NV doubles held per thread; result valid in red[0..NV-1]
-// for all threads after return.  red must hold NV * (blockDim/64) doubles.
-template <int NV>
+// for all threads after return.  red must hold NV * (blockDim/64) doubles.  Four
+// values at a time share a wave's DPP steps (kOneByOne: each by itself).
+template <int NV, bool kOneByOne = NV % 4 != 0>
 QMX_DEV void block_sum(double (&v)[NV], double* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  if constexpr (!kOneByOne) {
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    double s = wave_sum(v[j]);
-    if (lane == 0) red[wid * NV + j] = s;
+    for (int j = 0; j < NV; j += 4) {
+      const double s = rows_total(v[j], v[j + 1], v[j + 2], v[j + 3]);
+      if ((lane & 15) == 0) red[wid * NV + j + (lane >> 4)] = s;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const double s = wave_sum(v[j]);
+      if (lane == 0) red[wid * NV + j] = s;
+    }
   }
   __syncthreads();
   if (threadIdx.x < NV) {
@@ -561,11 +570,15 @@ __global__ __launch_bounds__(256) void sweep_step_kernel(SweepArgs<S> a) {
 //   X_{i+1} = Y_{i+1} W_{i+1}   (Y_{i+1} = X_{i+2} viewed as 2^{i+1} x 2 r_{i+2})
 //   rho_i   = Y_i^H Y_i         (Y_i = X_{i+1} viewed as 2^i x 2 r_{i+1})
 // The last block of each state finds the kept subspace of rho_i (FP64 Jacobi,
-// rsum2 cutoff, max bond 2) and stores its canonical basis W_i and r_i.
+// rsum2 cutoff, max bond 2) and stores its canonical basis W_i and r_i.  kSerial
+// (QMX_OPT_TWO_SIDED_JACOBI) keeps the one-lane eigensolver and the order of its
+// sums, and so their exact rounding, at 88 us a step against 50 (32 states of
+// N = 20, average of a layer).
 constexpr int kC2Rows = 256;   // rows of Y_i per chunk (= threads per block)
 // LDS tile index with one 16-byte pad per 8 entries (rows of 4 entries per lane)
 QMX_DEV int c2pad(int l) { return l + (l >> 3); }
 
+template <bool kSerial>
 __global__ __launch_bounds__(256) void chain2_step_kernel(Chain2Args a) {
   __shared__ double2 sx[2 * kC2Rows * 4 + (2 * kC2Rows * 4) / 8];
   __shared__ double red[4 * 32];
@@ -683,22 +696,39 @@ __global__ __launch_bounds__(256) void chain2_step_kernel(Chain2Args a) {
     }
     __syncthreads();   // before the next chunk's loads overwrite the tile
   }
-  block_sum<20>(e, red);
+  block_sum<20, kSerial>(e, red);
   double* pb = a.part + (size_t)b * gridDim.x * 20;
   if (publish_partial<20>(red, pb, a.counter + b, gridDim.x, &s_flag)) {
     reduce_partials<20>(pb, gridDim.x, scratch, tot);
+    // the Hermitian matrix from its upper triangle, zero-padded to 4 x 4
+    double2* vec = sx;   // (the tile is done with)
+    if (!kSerial && threadIdx.x < 64) {
+      const int lane = threadIdx.x, p = min((lane >> 2) & 3, lane & 3), q = max((lane >> 2) & 3, lane & 3);
+      const int t = 2 * (p * (7 - p) / 2 + q);
+      const double im = p == q ? 0.0 : tot[t + 1];
+      herm_eig4_wave(make_double2(tot[t], (lane & 3) >= ((lane >> 2) & 3) ? im : -im), lane, scratch, vec);
+      __builtin_amdgcn_wave_barrier();
+    }
     if (threadIdx.x == 0) {
-      double2 rho[16], v[16], w[16];
+      double2 v[16], w[16];
       double lam[4];
-      int t = 0;
-      for (int p = 0; p < 4; ++p)   // Hermitian matrix from its upper triangle
-        for (int q = p; q < 4; ++q) {
-          const double2 h = make_double2(tot[2 * t], p == q ? 0.0 : tot[2 * t + 1]);
-          rho[p * 4 + q] = h;
-          rho[q * 4 + p] = cconj(h);
-          ++t;
-        }
-      herm_eig4(rho, v, lam);   // rho is zero-padded to 4 x 4
+      if constexpr (kSerial) {
+        double2 rho[16];
+        int t = 0;
+        for (int p = 0; p < 4; ++p)
+          for (int q = p; q < 4; ++q) {
+            const double2 h = make_double2(tot[2 * t], p == q ? 0.0 : tot[2 * t + 1]);
+            rho[p * 4 + q] = h;
+            rho[q * 4 + p] = cconj(h);
+            ++t;
+          }
+        herm_eig4(rho, v, lam);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) lam[j] = scratch[j];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = vec[j];
+      }
       int k = keep_count(lam, 4, 2, a.cutoff);
       int found = canonical_basis4(k, v, w, kGsTol);
       if (found < k) {
@@ -921,7 +951,10 @@ void launch_fill_int(int* p, int v, int count, hipStream_t st) {
 }
 
 void launch_chain2_step(const Chain2Args& a, int nblk, int batch, hipStream_t st) {
-  hipLaunchKernelGGL(chain2_step_kernel, dim3(nblk, batch), dim3(256), 0, st, a);
+  if (a.serial)
+    hipLaunchKernelGGL(chain2_step_kernel<true>, dim3(nblk, batch), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(chain2_step_kernel<false>, dim3(nblk, batch), dim3(256), 0, st, a);
 }
 
 void launch_ran_gates(const RanArgs& a, int batch, hipStream_t st) {

@@ -477,13 +477,6 @@ constexpr double kEps = 2.220446049250313e-16;
 // a 128-term product is about sqrt(128) eps
 constexpr double kOsjTol = 2e-15;
 
-// The totals over the wave of four per-lane values: row k (lanes 16 k ..
-// 16 k + 15) holds the total of v_k on every lane.  Two half-swaps merge the
-// four registers, then four DPP steps add inside the rows.
-QMX_DEV double rows_total(double v0, double v1, double v2, double v3) {
-  return sum16(swap_add16(swap_add32(v0, v2), swap_add32(v1, v3)));
-}
-
 // NR entries of one column: rows lane, lane + 64, ...
 template <int NR> struct Col { double2 v[NR]; };
 

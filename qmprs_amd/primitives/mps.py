@@ -10,6 +10,7 @@ for Ran layers).
 
 from __future__ import annotations
 
+import contextlib
 from typing import Literal, TypeAlias
 
 import numpy as np
@@ -51,6 +52,18 @@ def _input_states(statevector) -> torch.Tensor:
     if float(torch.linalg.vector_norm(states)) == 0.0:
         raise ValueError("The statevector must be non-zero.")
     return states
+
+
+# Up to this many qubits the layers amplify their own rounding little (N=6, four
+# layers: below 6e-11 in 60 circuits of random states); at N=10 and six layers it
+# reaches 4e-10 in one of 60, at N=17 and five layers 3e-9 in one of 48.
+_FAST_LAYER_QUBITS = 8
+
+
+def layer_rounding(num_qubits: int):
+    """Context in which layers are extracted: above _FAST_LAYER_QUBITS the
+    drop-in path keeps one eigensolver's rounding here too (see _truncate)."""
+    return contextlib.nullcontext() if num_qubits <= _FAST_LAYER_QUBITS else _lib.two_sided_jacobi()
 
 
 def _truncate(states: torch.Tensor, bond_dimension: int):
@@ -163,7 +176,8 @@ class MPS:
     def generate_bond_D_unitary_layer(self) -> UnitaryLayer:
         """Bond-2 compression + Ran unitaries of the current state."""
         work = (self._state / self.norm).contiguous()
-        gates, widths, _ = engine.generate_layer(work)
+        with layer_rounding(self.num_sites):
+            gates, widths, _ = engine.generate_layer(work)
         return engine.gates_to_layers(gates.cpu().numpy()[0][None], widths.cpu().numpy()[0][None], 1)[0]
 
     def apply_unitary_layer(self, unitary_layer: UnitaryLayer, inverse: bool = False) -> None:

@@ -15,7 +15,7 @@ __all__ = ["Sequential"]
 import torch
 
 from qmprs_amd import _lib, engine
-from qmprs_amd.primitives.mps import MPS, UnitaryLayer
+from qmprs_amd.primitives.mps import MPS, UnitaryLayer, layer_rounding
 from qmprs_amd.synthesis.mps_encoding.base import MPSEncoder
 
 
@@ -77,8 +77,9 @@ class Sequential(MPSEncoder):
     # -- GPU phases ---------------------------------------------------------
     def _device_layers(self, mps: MPS, num_layers: int):
         work = (mps.state / mps.norm).contiguous()
-        gates, widths, used, amp0, _ = engine.extract_layers(
-            work, num_layers, self.fidelity_threshold)
+        with layer_rounding(mps.num_sites):
+            gates, widths, used, amp0, _ = engine.extract_layers(
+                work, num_layers, self.fidelity_threshold)
         return gates, widths, used, amp0
 
     def _get_unitary_layers(self, mps: MPS, num_layers: int) -> list[UnitaryLayer]:

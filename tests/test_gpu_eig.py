@@ -126,3 +126,60 @@ def test_two_sided_option(gpu):
     assert float(torch.linalg.vector_norm(one - two) / torch.linalg.vector_norm(two)) < 1e-10
     with pytest.raises(ValueError):
         _lib.set_option(_lib.QMX_OPT_TWO_SIDED_JACOBI, 2)
+
+
+@pytest.mark.parametrize("kind", ["bond2", "product", "ghz", "near_product", "real"])
+@pytest.mark.parametrize("n", [2, 3, 5, 9, 13])
+def test_layer_eigensolvers_agree(gpu, n, kind):
+    """The layers' 4 x 4 eigenproblems on one wave and in one lane: the same
+    bonds and widths, and gates that agree.  Both find the kept subspace to
+    eps over its gap; the kept and dropped eigenvalues differ by 1e-4 of the
+    trace or more (bond-2 states drop nothing but zeros; the near-product ones
+    keep 1e-4 and drop 1e-8), so to 1e-11 a step, amplified by the gates that
+    follow: 1e-8."""
+    eng = _engine()
+    from qmprs_amd import _lib
+    rng = np.random.default_rng(n)
+    if kind == "ghz":
+        sv = np.zeros(2 ** n, dtype=np.complex128)
+        sv[0] = sv[-1] = 2 ** -0.5
+    elif kind in ("product", "near_product"):
+        sv = np.ones(1, dtype=np.complex128)
+        for _ in range(n):
+            sv = np.kron(sv, rng.standard_normal(2) + 1j * rng.standard_normal(2))
+        sv /= np.linalg.norm(sv)
+        if kind == "near_product":
+            sv = sv + 0.01 * O.ket(O.random_mps_state(n, 2, 5))
+    else:
+        sv = O.random_mps_state(n, 2, 5)
+        sv = sv.real.astype(np.complex128) if kind == "real" else sv
+    psi = O.ket(sv)
+    out = []
+    for serial in (False, True):
+        work = eng.as_device_states(psi).clone()
+        if serial:
+            with _lib.two_sided_jacobi():
+                g, w, b = eng.generate_layer(work)
+        else:
+            g, w, b = eng.generate_layer(work)
+        out.append((g.cpu().numpy(), w.cpu().numpy(), b.cpu().numpy()))
+    (g0, w0, b0), (g1, w1, b1) = out
+    assert np.array_equal(w0, w1) and np.array_equal(b0, b1)
+    if kind != "real":       # (a real part of a bond-2 state has bond 4 and drops what it may)
+        assert np.abs(g0 - g1).max() < 1e-8
+    for gate, width in zip(g0[0].reshape(-1, 4, 4), w0[0].reshape(-1)):
+        d = 4 if width == 2 else 2
+        assert np.abs(gate[:d, :d] @ gate[:d, :d].conj().T - np.eye(d)).max() < 1e-12
+
+
+def test_layer_of_a_state_that_is_not_a_number_is_refused(gpu):
+    """With the same error from both eigensolvers."""
+    eng = _engine()
+    from qmprs_amd import _lib
+    sv = O.random_mps_state(6, 4, 1)
+    sv[5] = np.nan
+    with pytest.raises((ValueError, RuntimeError)) as wave:
+        eng.extract_layers(torch.from_numpy(sv).to(gpu).unsqueeze(0).contiguous(), 1)
+    with _lib.two_sided_jacobi(), pytest.raises((ValueError, RuntimeError)) as lane:
+        eng.extract_layers(torch.from_numpy(sv).to(gpu).unsqueeze(0).contiguous(), 1)
+    assert wave.type is lane.type and str(wave.value) == str(lane.value)
