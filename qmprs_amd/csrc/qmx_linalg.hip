@@ -232,6 +232,12 @@ __global__ __launch_bounds__(512) void jacobi_kernel(double2* a_all, double2* v_
 // entries passes the rotation test at the start of a sweep is converged (that
 // sweep would rotate nothing and is not run), as is one whose sweep rotated
 // nothing, and every later launch returns at once for it.
+// One round of n = 128 takes 2.8 us, most of it the FP64 and address
+// instructions of 2016 blocks on one CU's four SIMDs (3.3 us with the diagonal
+// blocks as a third pass over the threads and addresses formed per access); the
+// rows' kernel, bound by its rounds' LDS round trips, 40 us a sweep with a wave
+// per row (72 with a barrier per round).  Every product keeps the operands and
+// order that fix its rounding.
 constexpr int kJacobiLdsMax = 128;
 constexpr int kJacobiRowsPerBlock = 16;
 
@@ -242,9 +248,8 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
                                                                 double4* log_all, size_t log_stride,
                                                                 int* state, int sweep) {
   extern __shared__ double2 tri[];
-  __shared__ int pp[kJacobiLdsMax / 2], qq[kJacobiLdsMax / 2];
-  __shared__ double jc[kJacobiLdsMax / 2], js[kJacobiLdsMax / 2];
-  __shared__ double2 je[kJacobiLdsMax / 2];
+  __shared__ int4 pq[kJacobiLdsMax / 2];             // p, q and their rows' places
+  __shared__ double2 jcs[kJacobiLdsMax / 2], je[kJacobiLdsMax / 2];
   __shared__ int any_rot;
   __shared__ double s_scale;
   const int b = blockIdx.x;
@@ -258,19 +263,17 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
   double2* a = a_all + (size_t)b * stride;
   double4* lg = log_all + (size_t)b * log_stride;
   const int tid = threadIdx.x, nt = blockDim.x;
-  const int ntri = n * (n + 1) / 2;
-  for (int e = tid; e < ntri; e += nt) {
-    // row i: the largest i with tri_index(i, i) <= e
-    int i = (int)((2.0 * n + 1.0 - sqrt((2.0 * n + 1.0) * (2.0 * n + 1.0) - 8.0 * e)) * 0.5);
-    while (i > 0 && tri_index(i, i, n) > e) --i;
-    while (i + 1 < n && tri_index(i + 1, i + 1, n) <= e) ++i;
-    const int j = i + (e - tri_index(i, i, n));
-    tri[e] = a[(size_t)i * ld + j];
-  }
+  const int lane = tid & 63, wave = tid >> 6, waves = nt >> 6;
+  // entry (i, j) of the triangle is at rowbase(i) + j; a wave per row
+  auto rowbase = [&](int i) { return i * (2 * n - i + 1) / 2 - i; };
+  for (int i = wave; i < n; i += waves)
+    for (int j = i + lane; j < n; j += 64) tri[rowbase(i) + j] = a[(size_t)i * ld + j];
+  __syncthreads();
   if (tid == 0) {
     any_rot = 0;
     double tr = 0.0;
-    for (int i = 0; i < n; ++i) tr += fabs(a[(size_t)i * ld + i].x);
+#pragma unroll 16
+    for (int i = 0; i < n; ++i) tr += fabs(tri[rowbase(i) + i].x);
     s_scale = tr;
   }
   __syncthreads();
@@ -278,15 +281,12 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
   const double abs_tol = kJacobiAbsTol * s_scale + 1e-300;
   // a sweep would rotate nothing iff no off-diagonal entry passes the rotation
   // test now: then the state is converged and the sweep is not run
-  for (int e = tid; e < ntri; e += nt) {
-    int i = (int)((2.0 * n + 1.0 - sqrt((2.0 * n + 1.0) * (2.0 * n + 1.0) - 8.0 * e)) * 0.5);
-    while (i > 0 && tri_index(i, i, n) > e) --i;
-    while (i + 1 < n && tri_index(i + 1, i + 1, n) <= e) ++i;
-    const int j = i + (e - tri_index(i, i, n));
-    if (j == i) continue;
-    const double ag = cabs_(tri[e]);
-    if (ag > abs_tol && ag > 1e-15 * sqrt(fabs(tri[tri_index(i, i, n)].x * tri[tri_index(j, j, n)].x)))
-      any_rot = 1;
+  for (int i = wave; i < n; i += waves) {
+    const double al = tri[rowbase(i) + i].x;
+    for (int j = i + 1 + lane; j < n; j += 64) {
+      const double ag = cabs_(tri[rowbase(i) + j]);
+      if (ag > abs_tol && ag > 1e-15 * sqrt(fabs(al * tri[rowbase(j) + j].x))) any_rot = 1;
+    }
   }
   __syncthreads();
   const bool go = any_rot;
@@ -297,37 +297,47 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
   }
   if (tid == 0) any_rot = 0;
   __syncthreads();
-  // this thread's pair blocks (P, Q), P <= Q, row-major over the upper
-  // triangle of pair blocks; the same in every round (the kernel is
-  // launched with 1024 threads: kBlkPer * 1024 covers every block)
-  constexpr int kBlkPer = (kJacobiLdsMax / 2 * (kJacobiLdsMax / 2 + 1) / 2 + 1023) / 1024;
-  const int nblocks = np * (np + 1) / 2;
+  // this thread's pair blocks (P, Q), P < Q, row-major over the strict upper
+  // triangle of pair blocks; the same in every round (the kernel is launched
+  // with 1024 threads: two blocks each cover the 2016 of n = 128).  The diagonal
+  // blocks belong to the threads that find their rotations.
+  constexpr int kBlkPer = (kJacobiLdsMax / 2 * (kJacobiLdsMax / 2 - 1) / 2 + 1023) / 1024;
+  const int nblocks = np * (np - 1) / 2;
   int bP[kBlkPer], bQ[kBlkPer];
 #pragma unroll
   for (int k = 0; k < kBlkPer; ++k) {
     const int e = tid + k * nt;
+    // block (P, Q) of the strict triangle of np: entry (P, Q - 1) of the triangle of np - 1
+    const int m = np - 1;
     int P = 0, Q = 0;
     if (e < nblocks) {
-      P = (int)((2.0 * np + 1.0 - sqrt((2.0 * np + 1.0) * (2.0 * np + 1.0) - 8.0 * e)) * 0.5);
-      while (P > 0 && tri_index(P, P, np) > e) --P;
-      while (P + 1 < np && tri_index(P + 1, P + 1, np) <= e) ++P;
-      Q = P + (e - tri_index(P, P, np));
+      P = (int)((2.0 * m + 1.0 - sqrt((2.0 * m + 1.0) * (2.0 * m + 1.0) - 8.0 * e)) * 0.5);
+      while (P > 0 && tri_index(P, P, m) > e) --P;
+      while (P + 1 < m && tri_index(P + 1, P + 1, m) <= e) ++P;
+      Q = P + (e - tri_index(P, P, m)) + 1;
     }
     bP[k] = P;
     bQ[k] = Q;
   }
   for (int r = 0; r < n - 1; ++r) {
+    double c = 1.0, sn = 0.0;
+    double2 em = make_double2(1.0, 0.0), g = cz(), app = cz(), aqq = cz();
+    int ipp = 0, ipq = 0, iqq = 0;
     if (tid < np) {
       const int m = tid;
       int p = (m == 0) ? n - 1 : (r + m) % (n - 1);
       int q = (r + n - 1 - m) % (n - 1);
       if (m == 0) q = r % (n - 1);
       if (p > q) { int t = p; p = q; q = t; }
-      const double al = tri[tri_index(p, p, n)].x, be = tri[tri_index(q, q, n)].x;
-      const double2 g = tri[tri_index(p, q, n)];
+      const int bp = rowbase(p), bq = rowbase(q);
+      ipp = bp + p;
+      ipq = bp + q;
+      iqq = bq + q;
+      app = tri[ipp];
+      aqq = tri[iqq];
+      g = tri[ipq];
+      const double al = app.x, be = aqq.x;
       const double ag = cabs_(g);
-      double c = 1.0, sn = 0.0;
-      double2 em = make_double2(1.0, 0.0);
       // one comparison against the larger threshold: the diagonal reads are
       // issued together with the off-diagonal one
       if (ag > fmax(abs_tol, 1e-15 * sqrt(fabs(al * be)))) {
@@ -338,58 +348,62 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
         em = make_double2(g.x / ag, -g.y / ag);   // e^{-i phi}
         any_rot = 1;
       }
-      pp[m] = p; qq[m] = q; jc[m] = c; js[m] = sn; je[m] = em;
+      pq[m] = make_int4(p, q, bp, bq);
+      jcs[m] = make_double2(c, sn);
+      je[m] = em;
       lg[(size_t)r * np + m] = make_double4(c, sn, em.x, em.y);
     }
     __syncthreads();
     // blocks (P, Q), P <= Q: B' = J_P^H B J_Q with B = A[{p0, p1}][{q0, q1}];
     // (Q, P) is its conjugate transpose and is never stored separately
-#pragma unroll
-    for (int k = 0; k < kBlkPer; ++k) {
-      if (tid + k * nt >= nblocks) break;
-      const int P = bP[k], Q = bQ[k];
-      const int p0 = pp[P], p1 = qq[P], q0 = pp[Q], q1 = qq[Q];
-      // one LDS access per entry: (i, j) with i > j is the conjugate of (j, i)
-      auto get = [&](int i, int j) {
-        const bool lo = i > j;
-        const double2 v = tri[tri_index(lo ? j : i, lo ? i : j, n)];
-        return make_double2(v.x, lo ? -v.y : v.y);
-      };
-      auto put = [&](int i, int j, double2 v) {
-        const bool lo = i > j;
-        tri[tri_index(lo ? j : i, lo ? i : j, n)] = make_double2(v.x, lo ? -v.y : v.y);
-      };
-      const double2 J00 = make_double2(jc[Q], 0.0), J01 = make_double2(js[Q], 0.0);
-      const double2 J10 = cscale(je[Q], -js[Q]), J11 = cscale(je[Q], jc[Q]);
-      const double2 K00 = make_double2(jc[P], 0.0), K01 = make_double2(js[P], 0.0);
-      const double2 K10 = cscale(je[P], -js[P]), K11 = cscale(je[P], jc[P]);
-      const double2 a00 = get(p0, q0), a01 = get(p0, q1), a10 = get(p1, q0), a11 = get(p1, q1);
+    auto turn = [](double2 a00, double2 a01, double2 a10, double2 a11, double2 kcs, double2 ke, double2 qcs,
+                   double2 qe, double2& c00, double2& c01, double2& c10, double2& c11) {
+      const double2 J00 = make_double2(qcs.x, 0.0), J01 = make_double2(qcs.y, 0.0);
+      const double2 J10 = cscale(qe, -qcs.y), J11 = cscale(qe, qcs.x);
+      const double2 K00 = make_double2(kcs.x, 0.0), K01 = make_double2(kcs.y, 0.0);
+      const double2 K10 = cscale(ke, -kcs.y), K11 = cscale(ke, kcs.x);
       const double2 b00 = cadd(cmul(a00, J00), cmul(a01, J10));
       const double2 b01 = cadd(cmul(a00, J01), cmul(a01, J11));
       const double2 b10 = cadd(cmul(a10, J00), cmul(a11, J10));
       const double2 b11 = cadd(cmul(a10, J01), cmul(a11, J11));
-      double2 c00 = cadd(cmulc(K00, b00), cmulc(K10, b10));
-      double2 c01 = cadd(cmulc(K00, b01), cmulc(K10, b11));
-      double2 c10 = cadd(cmulc(K01, b00), cmulc(K11, b10));
-      double2 c11 = cadd(cmulc(K01, b01), cmulc(K11, b11));
-      if (P == Q) {
-        c00.y = 0.0; c11.y = 0.0;
-        c01 = cz();
-        put(p0, q0, c00); put(p0, q1, c01); put(p1, q1, c11);
-      } else {
-        put(p0, q0, c00); put(p0, q1, c01); put(p1, q0, c10); put(p1, q1, c11);
-      }
+      c00 = cadd(cmulc(K00, b00), cmulc(K10, b10));
+      c01 = cadd(cmulc(K00, b01), cmulc(K10, b11));
+      c10 = cadd(cmulc(K01, b00), cmulc(K11, b10));
+      c11 = cadd(cmulc(K01, b01), cmulc(K11, b11));
+    };
+    if (tid < np) {
+      double2 c00, c01, c10, c11;
+      // (the diagonal's zero imaginary parts come from memory, so that the
+      // compiler cannot fold them and round these blocks otherwise)
+      turn(app, g, cconj(g), aqq, make_double2(c, sn), em, make_double2(c, sn), em, c00, c01, c10, c11);
+      tri[ipp] = make_double2(c00.x, 0.0);
+      tri[ipq] = cz();
+      tri[iqq] = make_double2(c11.x, 0.0);
+    }
+#pragma unroll
+    for (int k = 0; k < kBlkPer; ++k) {
+      if (tid + k * nt >= nblocks) break;
+      const int P = bP[k], Q = bQ[k];
+      const int4 u = pq[P], w = pq[Q];
+      // one LDS access per entry: (i, j) with i > j is the conjugate of (j, i)
+      auto at = [&](int i, int bi, int j, int bj) { return i > j ? bj + i : bi + j; };
+      const int i00 = at(u.x, u.z, w.x, w.z), i01 = at(u.x, u.z, w.y, w.w);
+      const int i10 = at(u.y, u.w, w.x, w.z), i11 = at(u.y, u.w, w.y, w.w);
+      auto flip = [](double2 v, bool lo) { return make_double2(v.x, lo ? -v.y : v.y); };
+      const double2 a00 = flip(tri[i00], u.x > w.x), a01 = flip(tri[i01], u.x > w.y);
+      const double2 a10 = flip(tri[i10], u.y > w.x), a11 = flip(tri[i11], u.y > w.y);
+      double2 c00, c01, c10, c11;
+      turn(a00, a01, a10, a11, jcs[P], je[P], jcs[Q], je[Q], c00, c01, c10, c11);
+      tri[i00] = flip(c00, u.x > w.x);
+      tri[i01] = flip(c01, u.x > w.y);
+      tri[i10] = flip(c10, u.y > w.x);
+      tri[i11] = flip(c11, u.y > w.y);
     }
     __syncthreads();
   }
   // write the triangle back (the lower part stays stale: readers use i <= j)
-  for (int e = tid; e < ntri; e += nt) {
-    int i = (int)((2.0 * n + 1.0 - sqrt((2.0 * n + 1.0) * (2.0 * n + 1.0) - 8.0 * e)) * 0.5);
-    while (i > 0 && tri_index(i, i, n) > e) --i;
-    while (i + 1 < n && tri_index(i + 1, i + 1, n) <= e) ++i;
-    const int j = i + (e - tri_index(i, i, n));
-    a[(size_t)i * ld + j] = tri[e];
-  }
+  for (int i = wave; i < n; i += waves)
+    for (int j = i + lane; j < n; j += 64) a[(size_t)i * ld + j] = tri[rowbase(i) + j];
   if (tid == 0) {
     state[gridDim.x + b] = sweep + 1;
     // a sweep that rotated nothing leaves the log at identity: converged
@@ -408,31 +422,51 @@ __global__ __launch_bounds__(1024) void jacobi_lds_rows_kernel(double2* v_all, s
   if (state[gridDim.y + b] != sweep + 1) return;
   const int n = ncols_dev[b];
   const int r0 = blockIdx.x * kJacobiRowsPerBlock;
-  if (n < 2 || r0 >= n) return;
-  double2* v = v_all + (size_t)b * stride;
-  const double4* lg = log_all + (size_t)b * log_stride;
-  const int nr = min(kJacobiRowsPerBlock, n - r0);
+  // a wave per row, a lane per pair: the rows need no barrier between rounds
+  const int i = threadIdx.x >> 6, m = threadIdx.x & 63;
+  if (n < 2 || r0 + i >= n) return;
+  double2* v = v_all + (size_t)b * stride + (size_t)(r0 + i) * ld;
   const int np = n / 2;
-  for (int e = threadIdx.x; e < nr * n; e += blockDim.x) rows[e / n][e % n] = v[(size_t)(r0 + e / n) * ld + e % n];
-  __syncthreads();
-  for (int r = 0; r < n - 1; ++r) {
-    for (int e = threadIdx.x; e < nr * np; e += blockDim.x) {
-      const int i = e / np, m = e % np;
-      int p = (m == 0) ? n - 1 : (r + m) % (n - 1);
-      int q = (r + n - 1 - m) % (n - 1);
-      if (m == 0) q = r % (n - 1);
-      if (p > q) { int t = p; p = q; q = t; }
-      const double4 R = lg[(size_t)r * np + m];
-      const double2 em = make_double2(R.z, R.w);
-      const double2 J00 = make_double2(R.x, 0.0), J01 = make_double2(R.y, 0.0);
-      const double2 J10 = cscale(em, -R.y), J11 = cscale(em, R.x);
-      const double2 x = rows[i][p], y = rows[i][q];
-      rows[i][p] = cadd(cmul(x, J00), cmul(y, J10));
-      rows[i][q] = cadd(cmul(x, J01), cmul(y, J11));
+  const double4* lg = log_all + (size_t)b * log_stride + m;
+  double2* row = rows[i];
+  for (int e = m; e < n; e += 64) row[e] = v[e];
+  __builtin_amdgcn_wave_barrier();
+  // the log is read kAhead rounds before its use
+  constexpr int kAhead = 4;
+  double4 R[kAhead];
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k)
+    if (m < np && k < n - 1) R[k] = lg[(size_t)k * np];
+  auto round = [&](int r, double4& Rr) {
+    if (m >= np) return;
+    const double4 w = Rr;
+    if (r + kAhead < n - 1) Rr = lg[(size_t)(r + kAhead) * np];
+    // p = (r + m) % (n - 1), q = (r - m) % (n - 1); pair 0 is (n - 1, r)
+    int p = r + m, q = r - m;
+    p = m == 0 ? n - 1 : (p >= n - 1 ? p - (n - 1) : p);
+    q = q < 0 ? q + n - 1 : q;
+    if (p > q) { const int t = p; p = q; q = t; }
+    const double2 em = make_double2(w.z, w.w);
+    const double2 J00 = make_double2(w.x, 0.0), J01 = make_double2(w.y, 0.0);
+    const double2 J10 = cscale(em, -w.y), J11 = cscale(em, w.x);
+    const double2 x = row[p], y = row[q];
+    row[p] = cadd(cmul(x, J00), cmul(y, J10));
+    row[q] = cadd(cmul(x, J01), cmul(y, J11));
+  };
+  int r = 0;
+  for (; r + kAhead <= n - 1; r += kAhead) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      round(r + k, R[k]);
+      __builtin_amdgcn_wave_barrier();
     }
-    __syncthreads();
   }
-  for (int e = threadIdx.x; e < nr * n; e += blockDim.x) v[(size_t)(r0 + e / n) * ld + e % n] = rows[e / n][e % n];
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k) {
+    if (r + k < n - 1) round(r + k, R[k]);
+    __builtin_amdgcn_wave_barrier();
+  }
+  for (int e = m; e < n; e += 64) v[e] = row[e];
 }
 
 __global__ void jacobi_lds_init_kernel(double2* v_all, size_t stride, const int* ncols_dev, int ld, int* state,
