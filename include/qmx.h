@@ -211,7 +211,9 @@ int qmx_extract_layers(qmx_handle* h, int num_qubits, int batch, int num_layers,
  * num_sweeps passes over the gates in reverse circuit order; per gate
  * phi <- G^dagger phi, E = <T'|phi>_rest, G' = conj(polar(E)), T' <- G'^dagger T'.
  *   target      device, B x 2^N of storage_dtype: the chi-MPS state
- *   gates       device, in/out (updated in place)
+ *   gates       device, in/out (updated in place); unitary: a gate is removed
+ *               from the state by its adjoint, and what the gates of the first
+ *               circuit layer act on is |0> once they are removed
  *   psi_ref     device or NULL, B x 2^N complex128: fidelity reference
  *   fidelity    device or NULL, B x (num_sweeps+1) complex128: <psi_ref|C|0>
  *               before sweep s (s < num_sweeps) and after the last sweep

@@ -236,6 +236,21 @@ QMX_DEV int gate_code(uint64_t mask, int n, int site, int w) {
   return hb * 2 + (w == 2 ? 1 : 0);
 }
 
+// Support of phi in a state's last n steps (its first circuit layer, whose
+// gates act on |0..0>): once the gates of steps up to s are removed, the bits
+// below s % n are in |0>.  They are set to exactly zero there, which leaves the
+// environments' null columns exact, and tiles that have such a bit set are not
+// visited: neither phi nor T', which only ever meets phi, is needed there again.
+QMX_DEV uint64_t dead_bits(int n, int kb, int s0) {
+  return s0 > kb - n && s0 > 0 ? (1ull << ((s0 - 1) % n)) - 1ull : 0ull;
+}
+// place inside the set `mask` of the bit that the removal of step s's gate
+// leaves in |0>, or -1
+QMX_DEV int dead_after(uint64_t mask, int n, int kb, int s) {
+  const int h = s % n;
+  return s >= kb - n && h > 0 ? __popcll(mask & ((1ull << (h - 1)) - 1ull)) : -1;
+}
+
 // complex64 fits 4 waves per SIMD without spills; complex128 runs at 2 (a
 // 4-wave budget would spill its FP64 groups)
 // STAGED: the tiles of T' and phi are copied between HBM and LDS in tile
@@ -252,7 +267,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   using c2 = typename T::c2;
   extern __shared__ char wsm[];
   __shared__ c2 gmat[2 * kMaxWindow][16];
-  __shared__ int gcode[2 * kMaxWindow];
+  __shared__ int gcode[2 * kMaxWindow], gdead[2 * kMaxWindow];
   // group element offsets, [side][x]: side 0 = T' over the previous set,
   // side 1 = phi over the current set; global (state) and tile-local
   __shared__ uint32_t xog[2][16];
@@ -280,7 +295,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     step_gate(n, s, layer, site);
     const size_t gi = ((size_t)b * a.lmax + layer) * n + site;
     gmat[j][e] = T::mk(a.gates[gi * 16 + e]);
-    if (e == 0) gcode[j] = gate_code(j < np ? a.gp.mask : a.gu.mask, n, site, wsane(n, site, a.widths[gi]));
+    if (e == 0) {
+      gcode[j] = gate_code(j < np ? a.gp.mask : a.gu.mask, n, site, wsane(n, site, a.widths[gi]));
+      gdead[j] = j < np ? -1 : dead_after(a.gu.mask, n, kb, s);
+    }
   }
   // staged copies: tile-local index l -> state offset (l & lomask) + hoff[l >> c0]
   const uint64_t pbits = ((1ull << n) - 1ull) & ~a.qmask;
@@ -299,7 +317,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   const S* tsrc = (a.p0 == 0 ? a.target : a.tprime) + (size_t)b * len;
   S* tdst = a.tprime + (size_t)b * len;
   S* phi = a.phi + (size_t)b * len;
-  const long ntiles = 1l << (n - t);
+  const uint64_t qmask = a.qmask & ~dead_bits(n, kb, a.s0);   // the live tiles' bits
+  const long ntiles = 1l << __popcll(qmask);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ngroups = 1 << (t - 4);
   // lanes [0, ngroups): T' groups over the previous set; [ngroups, 2 ngroups): phi groups
@@ -343,7 +362,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     for (int x = 0; x < 16; ++x) v[x] = T::mk(to_c(src[g + xg[x]]));
   };
   if (!STAGED && active && (long)blockIdx.x < ntiles)
-    load_group((uint32_t)wdeposit((uint64_t)blockIdx.x, a.qmask) + roffg);
+    load_group((uint32_t)wdeposit((uint64_t)blockIdx.x, qmask) + roffg);
   // Staged tiles of 2^kWinTileBits amplitudes over 256 threads: the 128
   // T'-side threads copy the T' tile (16 amplitudes each, tile order), the
   // 128 phi-side threads the phi tile, through the group registers v.  The
@@ -363,9 +382,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = T::mk(to_c(src[tb + ust[i] + sl0]));
   };
-  if (fast_stage && (long)blockIdx.x < ntiles) load_stage((uint32_t)wdeposit((uint64_t)blockIdx.x, a.qmask));
+  if (fast_stage && (long)blockIdx.x < ntiles) load_stage((uint32_t)wdeposit((uint64_t)blockIdx.x, qmask));
   for (long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const uint32_t base = (uint32_t)wdeposit((uint64_t)tile, a.qmask);
+    const uint32_t base = (uint32_t)wdeposit((uint64_t)tile, qmask);
     const uint32_t gb = base + roffg;
     const long nxt = tile + gridDim.x;
     if (STAGED) {
@@ -392,16 +411,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
           for (int x = 0; x < 16; ++x)
             lds[swz(roffl + xl[x])] = from_c<S>(make_double2(v[x].x, v[x].y));
         }
-        if (j < ngate) grp_apply<C>(gcode[g0 + j], v, gmat[g0 + j]);
+        if (j < ngate) {
+          grp_apply<C>(gcode[g0 + j], v, gmat[g0 + j]);
+          const int z = gdead[g0 + j];
+          if (z >= 0) {
+#pragma unroll
+            for (int x = 0; x < 16; ++x)
+              if ((x >> z) & 1) v[x] = c2{0, 0};
+          }
+        }
       }
       if (!STAGED && store_dst) {
 #pragma unroll
         for (int x = 0; x < 16; ++x) dst[gb + xg[x]] = from_c<S>(make_double2(v[x].x, v[x].y));
       }
       if (!STAGED) {
-        if (nxt < ntiles) load_group((uint32_t)wdeposit((uint64_t)nxt, a.qmask) + roffg);
+        if (nxt < ntiles) load_group((uint32_t)wdeposit((uint64_t)nxt, qmask) + roffg);
       }
-      if (fast_stage && tside && nxt < ntiles) load_stage((uint32_t)wdeposit((uint64_t)nxt, a.qmask));
+      if (fast_stage && tside && nxt < ntiles) load_stage((uint32_t)wdeposit((uint64_t)nxt, qmask));
     }
     __syncthreads();
     // R += conj(T') phi^T over this tile: A[x][k] = conj(T'[x, r]), B[k][y] = phi[y, r]
@@ -426,7 +453,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 #pragma unroll
         for (int x = 0; x < 16; ++x) sP[swz(roffl + xl[x])] = from_c<S>(make_double2(v[x].x, v[x].y));
       }
-      if (fast_stage && !tside && nxt < ntiles) load_stage((uint32_t)wdeposit((uint64_t)nxt, a.qmask));
+      if (fast_stage && !tside && nxt < ntiles) load_stage((uint32_t)wdeposit((uint64_t)nxt, qmask));
     }
     if (STAGED && a.store) {
       __syncthreads();
@@ -838,7 +865,7 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
   __shared__ double2 q[256];
   __shared__ double2 qn[256];
   __shared__ double2 gm[kMaxWindow][16];
-  __shared__ int gw[kMaxWindow], gh[kMaxWindow], gl[kMaxWindow];
+  __shared__ int gw[kMaxWindow], gh[kMaxWindow], gl[kMaxWindow], gz[kMaxWindow];
   __shared__ double2 gnew[16];
   __shared__ double2 es[16];
   __shared__ double2 rm[16];
@@ -864,6 +891,7 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
       const int hb = n - 1 - site;
       gh[j] = __popcll(a.umask & ((1ull << hb) - 1ull));
       gl[j] = w == 2 ? __popcll(a.umask & ((1ull << (hb - 1)) - 1ull)) : 0;
+      gz[j] = dead_after(a.umask, n, kb, a.s0 + j);
     }
   }
   // R = sum of the block partials (slots 0, ps, 2 ps, ...) in a fixed order
@@ -936,7 +964,8 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
           const int yp = (y & ~m2) | (w2 == 2 ? ((pg >> 1) << hb2) | ((pg & 1) << lb2) : pg << hb2);
           s = cfmac(gm[j + 1][pg * 4 + yg], q[x * 16 + yp], s);
         }
-        qn[e] = s;
+        const int z2 = gz[j + 1];
+        qn[e] = z2 >= 0 && ((y >> z2) & 1) ? cz() : s;
       }
     }
     if (!more) break;   // Q is not read after the window's last gate
@@ -968,8 +997,8 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
 //   T'  <- G'_{p-2}^dagger T',   phi <- G_p^dagger phi,
 //   R_p[x][y] = sum_r conj(T'[x, r]) phi[y, r]
 // over the set V of the bits of steps p - 1 and p (three of them, the steps
-// descend one site at a time), an 8 x 8 matrix.  G'_{p-1}, which R_p still lacks, acts inside V, so the
-// next phase's environment is
+// descend one site at a time), an 8 x 8 matrix.  G'_{p-1}, which R_p still
+// lacks, acts inside V, so the next phase's environment is
 //   E_p[o][i] = sum_z sum_x' G'_{p-1}[x'_g][x_g] R_p[x'][y],  x = (o, z), y = (i, z).
 // Each worker owns a quarter of the indices r outside U = V and step p - 2's
 // bits in a phase, so updates and products need no barrier between them, and

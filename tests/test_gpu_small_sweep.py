@@ -1,5 +1,6 @@
-"""Sweeps of small states in one block (the automatic mode) against the
-gate-by-gate and windowed sweeps."""
+"""Sweeps of small states in one block (the automatic mode) and windowed sweeps
+whose passes leave out what the first circuit layer's gates no longer touch,
+against the gate-by-gate sweep."""
 
 import numpy as np
 import pytest
@@ -35,6 +36,18 @@ def _random_layers(n, b, layers, gpu, seed):
                                            (5, 3, [3, 1, 0]), (6, 2, [2, 2]), (7, 1, [1]), (9, 2, [2]),
                                            (11, 2, [1, 2]), (12, 1, [1]), (12, 3, [3]), (13, 2, [2])])
 def test_one_block_sweep(gpu, dtype, n, layers, used):
+    _against_steps(gpu, "auto", dtype, n, layers, used)
+
+
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+@pytest.mark.parametrize("n,layers,used", [(10, 1, [1, 0]), (11, 2, [2, 1]), (12, 3, [3, 1, 2]), (13, 1, [1]),
+                                           (14, 2, [2]), (15, 3, [1, 3, 0]), (16, 1, [1]), (17, 2, [2, 2]),
+                                           (18, 1, [1])])
+def test_windowed_sweep(gpu, dtype, n, layers, used):
+    _against_steps(gpu, "window", dtype, n, layers, used)
+
+
+def _against_steps(gpu, sweep_mode, dtype, n, layers, used):
     """Random targets under random circuits: fidelities, overlaps, circuit
     states, gates, snapshots and the goal's stop.  The environments are generic
     but in the first circuit layer, whose gates act on |0> and are determined
@@ -53,7 +66,7 @@ def test_one_block_sweep(gpu, dtype, n, layers, used):
     gates0, widths = _random_layers(n, b, layers, gpu, 11 * n + layers)
     lu = torch.tensor(used, dtype=torch.int32, device=gpu)
     out = {}
-    for mode in ("auto", "step"):
+    for mode in (sweep_mode, "step"):
         try:
             _lib.set_sweep_mode(mode)
             gates = gates0.clone()
@@ -63,7 +76,7 @@ def test_one_block_sweep(gpu, dtype, n, layers, used):
             out[mode] = (gates, snaps, res)
         finally:
             _lib.set_sweep_mode("auto")
-    (ga, sa, ra), (gs, ss, rs) = out["auto"], out["step"]
+    (ga, sa, ra), (gs, ss, rs) = out[sweep_mode], out["step"]
     tol = 3e-9 if dtype == torch.complex128 else 2e-5
     assert torch.equal(sa[0], gates0)
     for i, k in enumerate(used):
@@ -84,14 +97,18 @@ def test_one_block_sweep(gpu, dtype, n, layers, used):
     live = [i for i, k in enumerate(used) if k > 0]
     assert (ra.overlap[live] - rs.overlap[live]).abs().max() < tol
     assert (ra.circuit - rs.circuit).abs().max() < (tol if dtype == torch.complex128 else 2e-3)
-    # a goal: met from the start, met after one sweep, out of reach
-    f = ra.fidelity.abs().real
-    for goal, want in ((f[:, 0] - 1e-3, 0), ((f[:, 0] + f[:, 1]) / 2, 1), (f[:, 0] * 0 + 2.0, 2)):
-        gates = gates0.clone()
-        r = engine.sweep(target, gates, widths, lu, 2, psi_ref=ref, goal=goal.contiguous(), circuit_out=True)
-        done = r.sweeps_done.cpu().tolist()
-        for i in live:
-            if want != 1 or f[i, 1] > f[i, 0] + 1e-3:
-                assert done[i] == want
-            after = [gates0, sa[1], ga][done[i]][i]
-            assert (gates[i] - after).abs().max() < 1e-14
+    try:
+        _lib.set_sweep_mode(sweep_mode)
+        # a goal: met from the start, met after one sweep, out of reach
+        f = ra.fidelity.abs().real
+        for goal, want in ((f[:, 0] - 1e-3, 0), ((f[:, 0] + f[:, 1]) / 2, 1), (f[:, 0] * 0 + 2.0, 2)):
+            gates = gates0.clone()
+            r = engine.sweep(target, gates, widths, lu, 2, psi_ref=ref, goal=goal.contiguous(), circuit_out=True)
+            done = r.sweeps_done.cpu().tolist()
+            for i in live:
+                if want != 1 or f[i, 1] > f[i, 0] + 1e-3:
+                    assert done[i] == want
+                after = [gates0, sa[1], ga][done[i]][i]
+                assert (gates[i] - after).abs().max() < 1e-14
+    finally:
+        _lib.set_sweep_mode("auto")
