@@ -366,6 +366,7 @@ QMX_DEV double mat4_tmul(Mat4 m, Mat4 b, bool even) {
   return __builtin_amdgcn_mfma_f64_4x4x4f64(im, b.o, d, 0, 0, 0);
 }
 
+QMX_DEV bool polar4_rank2(double2& x, int l, const double2* es, int h, double fro, double* nuc);
 // Unitary polar factor of es 2^h (|.|_F^2 = fro, near 1) by the scaled
 // Newton-Schulz iteration
 //   X <- X (a - b X^H X),  a = 3 s / 2,  b = s^3 / 2,
@@ -387,7 +388,8 @@ QMX_DEV double mat4_tmul(Mat4 m, Mat4 b, bool even) {
 // 1e-16 times the condition number over 5).
 // u: this lane's part of the factor in the split layout.  False after 34
 // unscaled steps (a condition number above about 1e6).
-QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane, Mat4& u) {
+QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane, Mat4& u, double2& x2, double& nuc2,
+                                  bool& rank2) {
   const int i = lane >> 4, j = lane & 3;
   const bool even = !(lane & 4);
   const double r = rsqrt_newton(fro);
@@ -410,6 +412,15 @@ QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane
   step(1.5019149323066294, 0.5019173779907503, gram());  // 0.9974
   for (int it = 0; it < 34; ++it) {
     const double y = gram();
+    if (it == 0) {
+      // Two singular values that are zero, or below 1e-4 or so, leave the trace
+      // of X^H X, by now about the number of the others, no larger than 2
+      const double tr = (lane_value(y, 0) + lane_value(y, 17)) + (lane_value(y, 34) + lane_value(y, 51));
+      if (tr < 2.0001 && polar4_rank2(x2, lane & 15, es, h, fro, &nuc2)) {
+        rank2 = true;
+        return true;
+      }
+    }
     const bool last = __all(fabs(y - one) <= 3e-9);
     step(1.5, 0.5, y);
     if (last) {
@@ -441,6 +452,37 @@ QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc)
   return true;
 }
 
+// sum over the 4 rows i
+QMX_DEV double col_total(double v) {
+  v += dpp<kDppRow2>(v);
+  return v + dpp<kDppRow1>(v);
+}
+// sum over the 4 columns j
+QMX_DEV double row_total(double v) {
+  v += dpp<kDppSwap>(v);
+  return v + dpp<kDppCol2>(v);
+}
+// Two unit vectors beside q_0, q_1 (rows in the lanes' i), as polar4_jacobi
+// completes: residuals of the first e_k, in order, whose squared norm is above 1/4
+QMX_DEV bool complete_two(int i, double2 q0, double2 q1, double2& q2, double2& q3) {
+  // squared residual of e_i against q_0, q_1; the first above 1/4
+  const double res = 1.0 - cabs2(q0) - cabs2(q1);
+  const unsigned m2 = (unsigned)__ballot(res > 0.25) & 0x1111u;
+  if (!m2) return false;
+  const int e2 = __builtin_amdgcn_readfirstlane((__ffs(m2) - 1) >> 2);
+  auto row = [&](double2 v, int k) { return make_double2(lane_value(v.x, 4 * k), lane_value(v.y, 4 * k)); };
+  double2 t = cadd(cmulc(row(q0, e2), q0), cmulc(row(q1, e2), q1));
+  q2 = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
+  q2 = cscale(q2, rsqrt_newton(col_total(cabs2(q2))));
+  const unsigned m3 = (unsigned)__ballot(i > e2 && res - cabs2(q2) > 0.25) & 0x1111u;
+  if (!m3) return false;
+  const int e3 = __builtin_amdgcn_readfirstlane((__ffs(m3) - 1) >> 2);
+  t = cadd(cadd(cmulc(row(q0, e3), q0), cmulc(row(q1, e3), q1)), cmulc(row(q2, e3), q2));
+  q3 = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
+  q3 = cscale(q3, rsqrt_newton(col_total(cabs2(q3))));
+  return true;
+}
+
 // The environments of the gates next to a site still in |0>: two columns of E
 // are zero (to 1e-14 of its norm; the Jacobi path drops singular values below
 // 1e-13 of the largest).  With Q R = the two columns left (Gram-Schmidt, two
@@ -452,11 +494,6 @@ QMX_DEV bool polar2(double2& a, double2& b, double2& c, double2& d, double* nuc)
 // (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry (i, j) of
 // the factor.  False where the Jacobi path decides (30600 cycles); 2700
 // cycles, against 5300 to 7500 with the whole problem in every lane.
-// sum over the 4 rows i
-QMX_DEV double col_total(double v) {
-  v += dpp<kDppRow2>(v);
-  return v + dpp<kDppRow1>(v);
-}
 QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, unsigned zero, double fro, double* nuc) {
   const unsigned live = ~zero & 15u;
   const int c0 = __ffs(live) - 1, c1 = 31 - __clz(live), z0 = __ffs(zero) - 1, z1 = 31 - __clz(zero);
@@ -480,21 +517,8 @@ QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, uns
   const double2 q1 = cscale(quad_bcast2<1>(y), i1);
   double2 p11 = make_double2(n1 * i1, 0.0);
   if (!polar2(p00, p01, p10, p11, nuc)) return false;
-  // squared residual of e_i against q_0, q_1; the first above 1/4
-  const double res = 1.0 - cabs2(q0) - cabs2(q1);
-  const unsigned m2 = (unsigned)__ballot(res > 0.25) & 0x1111u;
-  if (!m2) return false;
-  const int e2 = __builtin_amdgcn_readfirstlane((__ffs(m2) - 1) >> 2);
-  auto row = [&](double2 v, int k) { return make_double2(lane_value(v.x, 4 * k), lane_value(v.y, 4 * k)); };
-  double2 t = cadd(cmulc(row(q0, e2), q0), cmulc(row(q1, e2), q1));
-  double2 q2 = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
-  q2 = cscale(q2, rsqrt_newton(col_total(cabs2(q2))));
-  const unsigned m3 = (unsigned)__ballot(i > e2 && res - cabs2(q2) > 0.25) & 0x1111u;
-  if (!m3) return false;
-  const int e3 = __builtin_amdgcn_readfirstlane((__ffs(m3) - 1) >> 2);
-  t = cadd(cadd(cmulc(row(q0, e3), q0), cmulc(row(q1, e3), q1)), cmulc(row(q2, e3), q2));
-  double2 q3 = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
-  q3 = cscale(q3, rsqrt_newton(col_total(cabs2(q3))));
+  double2 q2, q3;
+  if (!complete_two(i, q0, q1, q2, q3)) return false;
   // out column z_1: q_2, z_2: q_3, the live ones: Q polar(R)
   const double2 a = j == c0 ? p00 : p01, b = j == c0 ? p10 : p11;
   x = cadd(cmul(q0, a), cmul(q1, b));
@@ -534,6 +558,93 @@ QMX_DEV bool polar4_one_column(double2& x, int l, const double2* es, int h, unsi
     if (j == slot) x = q[k];
     ++slot;
   }
+  return true;
+}
+
+// one of four by two selects (a chain of comparisons becomes a table in memory)
+QMX_DEV double2 pick4(int k, double2 a, double2 b, double2 c, double2 d) {
+  const double2 lo = make_double2(k & 1 ? b.x : a.x, k & 1 ? b.y : a.y);
+  const double2 hi = make_double2(k & 1 ? d.x : c.x, k & 1 ? d.y : c.y);
+  return make_double2(k & 2 ? hi.x : lo.x, k & 2 ? hi.y : lo.y);
+}
+// A dense E of rank 2, the environment of the first site's gate above the first
+// circuit layer, whose state has Schmidt rank 2 beside it: E = Q L W^H by
+// column-pivoted Gram-Schmidt and again on the rows, and the factor is
+// Q polar(L) W^H with both sides completed as polar4_jacobi completes them.
+// Taken when nothing above 3e-14 of the norm is left beside Q (the Jacobi path
+// drops singular values below 1e-13).  7900 cycles with the six steps that find
+// it out; it is met once a sweep, and the Jacobi path took 64000 there.
+QMX_DEV bool polar4_rank2(double2& x, int l, const double2* es, int h, double fro, double* nuc) {
+  const int i = l >> 2, j = l & 3;
+  auto at = [&](int c) {
+    const double2 e = es[4 * i + c];
+    return make_double2(ldexp(e.x, h), ldexp(e.y, h));
+  };
+  double2 y = at(j);
+  auto largest = [&](double n) {   // the column of the largest n (the same down each column)
+    const double n0 = lane_value(n, 0), n1 = lane_value(n, 1), n2 = lane_value(n, 2), n3 = lane_value(n, 3);
+    const int a = n1 > n0 ? 1 : 0, b = n3 > n2 ? 3 : 2;
+    return fmax(n2, n3) > fmax(n0, n1) ? b : a;
+  };
+  auto project = [&](double2 q, double2& r) {   // y -= q (q^H y), r += q^H y
+#pragma unroll
+    for (int pass = 0; pass < 2; ++pass) {
+      const double2 t = cmulc(q, y);
+      const double2 d = make_double2(col_total(t.x), col_total(t.y));
+      r = cadd(r, d);
+      y = csub(y, cmul(q, d));
+    }
+  };
+  double n = col_total(cabs2(y));
+  const int c0 = largest(n);
+  double2 q0 = at(c0);
+  q0 = cscale(q0, rsqrt_newton(col_total(cabs2(q0))));
+  double2 r0 = cz(), r1 = cz();
+  project(q0, r0);
+  n = col_total(cabs2(y));
+  const int c1 = largest(n);
+  double2 q1 = quad_bcast2<0>(y);
+  if (c1 == 1) q1 = quad_bcast2<1>(y);
+  if (c1 == 2) q1 = quad_bcast2<2>(y);
+  if (c1 == 3) q1 = quad_bcast2<3>(y);
+  const double n1 = col_total(cabs2(q1));
+  if (!(n1 > 1e-26 * fro)) return false;
+  q1 = cscale(q1, rsqrt_newton(n1));
+  project(q1, r1);
+  if (!(sum16(cabs2(y)) < 1e-27 * fro)) return false;
+  // rows r_0, r_1 = L W^H
+  const double m0 = row_total(cabs2(r0)), i0 = rsqrt_newton(m0);
+  double2 w0 = cscale(cconj(r0), i0), l10 = cz();
+#pragma unroll
+  for (int pass = 0; pass < 2; ++pass) {
+    const double2 t = cmul(r1, w0);
+    const double2 d = make_double2(row_total(t.x), row_total(t.y));
+    l10 = cadd(l10, d);
+    r1 = csub(r1, cmul(d, cconj(w0)));
+  }
+  const double m1 = row_total(cabs2(r1));
+  if (!(m1 > 1e-26 * fro)) return false;
+  const double i1 = rsqrt_newton(m1);
+  double2 w1 = cscale(cconj(r1), i1);
+  double2 p00 = make_double2(m0 * i0, 0.0), p01 = cz(), p10 = l10, p11 = make_double2(m1 * i1, 0.0);
+  if (!polar2(p00, p01, p10, p11, nuc)) return false;
+  double2 u2, u3, v2, v3;
+  if (!complete_two(i, q0, q1, u2, u3)) return false;
+  // W's entries by the lanes' i for its completion, and that by their j
+  auto by_row = [&](double2 v) {
+    const double2 a = quad_bcast2<0>(v), b = quad_bcast2<1>(v), c = quad_bcast2<2>(v), d = quad_bcast2<3>(v);
+    return pick4(i, a, b, c, d);
+  };
+  auto by_col = [&](double2 v) {
+    auto row = [&](int k) { return make_double2(lane_value(v.x, 4 * k), lane_value(v.y, 4 * k)); };
+    const double2 a = row(0), b = row(1), c = row(2), d = row(3);
+    return pick4(j, a, b, c, d);
+  };
+  if (!complete_two(i, by_row(w0), by_row(w1), v2, v3)) return false;
+  v2 = by_col(v2);
+  v3 = by_col(v3);
+  const double2 a = cadd(cmul(q0, p00), cmul(q1, p10)), b = cadd(cmul(q0, p01), cmul(q1, p11));
+  x = cadd(cadd(cmul(a, cconj(w0)), cmul(b, cconj(w1))), cadd(cmul(u2, cconj(v2)), cmul(u3, cconj(v3))));
   return true;
 }
 
@@ -596,7 +707,13 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int
     return true;
   }
   Mat4 u;
-  if (!polar4_newton_schulz(es, h, fro, lane, u)) return false;
+  bool singular = false;
+  if (!polar4_newton_schulz(es, h, fro, lane, u, x, s, singular)) return false;
+  if (singular) {
+    if (lane < 16) out[l] = make_double2(x.x, sgn * x.y);
+    *nuc = ldexp(s, -h);
+    return true;
+  }
   if (!(lane & 12)) out[4 * (lane >> 4) + (lane & 3)] = make_double2(u.v, sgn * u.o);
   if (want) {   // Re tr(U^H E)
     __builtin_amdgcn_wave_barrier();
@@ -607,8 +724,8 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int
 }
 
 // Unitary polar factor U V^H of the d x d (d = 2 or 4) matrix e (row-major,
-// stride 4) in one lane, for the inputs that polar4_wave leaves to it: a
-// one-sided (Hestenes) Jacobi SVD on a 4 x 4 working matrix (a
+// stride 4, zero outside the block) for the inputs that polar4_wave leaves to
+// it: a one-sided (Hestenes) Jacobi SVD on a 4 x 4 working matrix (a
 // 2 x 2 problem is embedded as diag(E, |E| I), whose padded columns are
 // orthogonal to E's and never rotate).  Rotations: cyclic pairs p < q, when
 // |a_p^H a_q| > 1e-16 |a_p| |a_q|.  Pairs (u_j, v_j) with sigma_j >
@@ -616,137 +733,123 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int
 // the next unit vector e_0, e_1, ... whose two-pass Gram-Schmidt residual
 // against the columns already set has norm > 1/2, on both the U and V sides.
 // The result then depends only on the well-determined singular subspaces.
-// *nuc = sum of E's singular values.  Compile-time indices only.
-QMX_DEV void polar4_jacobi(int d, const double2* e, double2* out, double* nuc) {
-  double2 a[16], v[16];
+// *nuc = sum of E's singular values.
+// Lane k of a quad holds row k of both matrices, every quad the same, and the
+// loops that need not be unrolled are not: with everything in one lane's
+// registers this was 70 KiB of code, and a call, which found none of it in the
+// instruction cache, took 64000 cycles and left the rest of the sweep to be
+// fetched again.  A matrix of rank 3: 48000 cycles against 190000 (4000 blocks).
+QMX_DEV void polar4_jacobi(int d, const double2* e, double2* out, double sgn, int lane, double* nuc) {
+  const int i = lane & 3;
+  double2 a[4], v[4];
   double fro = 0.0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    a[i] = e[i];
-    fro += cabs2(e[i]);
-    v[i] = make_double2((i % 5) == 0 ? 1.0 : 0.0, 0.0);
+  for (int c = 0; c < 4; ++c) {
+    a[c] = e[4 * i + c];
+    fro += cabs2(a[c]);
+    v[c] = make_double2(i == c ? 1.0 : 0.0, 0.0);
   }
-  if (d == 2) {
-    double s = sqrt(fro);
-    if (s == 0.0) s = 1.0;
+  fro = row_total(fro);
+  // exact scaling to a squared norm near 1
+  const int h = fro > 0.0 && fro < __builtin_inf() ? -(__builtin_amdgcn_frexp_exp(fro) >> 1) : 0;
+  const double s = fro > 0.0 ? sqrt(ldexp(fro, 2 * h)) : 1.0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      int r = i / 4, c = i % 4;
-      if (r >= 2 || c >= 2) a[i] = make_double2((r == c) ? s : 0.0, 0.0);
-    }
+  for (int c = 0; c < 4; ++c) {
+    a[c] = make_double2(ldexp(a[c].x, h), ldexp(a[c].y, h));
+    if (d == 2 && (i >= 2 || c >= 2)) a[c] = make_double2(i == c ? s : 0.0, 0.0);
   }
+  auto dot = [](double2 x, double2 y) {   // x^H y
+    const double2 t = cmulc(x, y);
+    return make_double2(row_total(t.x), row_total(t.y));
+  };
+#pragma unroll 1
   for (int sweep = 0; sweep < 60; ++sweep) {
     bool rotated = false;
 #pragma unroll
     for (int p = 0; p < 3; ++p)
 #pragma unroll
       for (int q = p + 1; q < 4; ++q) {
-        double al = 0.0, be = 0.0;
-        double2 g = cz();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          al += cabs2(a[i * 4 + p]);
-          be += cabs2(a[i * 4 + q]);
-          g = cfmac(a[i * 4 + p], a[i * 4 + q], g);  // a_p^H a_q
-        }
-        double ag = cabs_(g);
-        if (ag != 0.0 && ag > 1e-16 * sqrt(al * be)) {
+        const double al = row_total(cabs2(a[p])), be = row_total(cabs2(a[q]));
+        const double2 g = dot(a[p], a[q]);
+        const double ag2 = cabs2(g);
+        if (ag2 > 0.0 && ag2 > 1e-32 * (al * be)) {
           rotated = true;
-          double2 ph = make_double2(g.x / ag, g.y / ag);
-          double zeta = (be - al) / (2.0 * ag);
-          double t = (zeta >= 0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-          double c = 1.0 / sqrt(1.0 + t * t), sn = t * c;
-          // [a_p, a_q] <- [a_p, a_q] [[c, s e^{i phi}], [-s e^{-i phi}, c]]
-          double2 sp = cscale(ph, sn), sm = cscale(cconj(ph), -sn);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            double2 x = a[i * 4 + p], y = a[i * 4 + q];
-            a[i * 4 + p] = cadd(cscale(x, c), cmul(y, sm));
-            a[i * 4 + q] = cadd(cmul(x, sp), cscale(y, c));
-            double2 vx = v[i * 4 + p], vy = v[i * 4 + q];
-            v[i * 4 + p] = cadd(cscale(vx, c), cmul(vy, sm));
-            v[i * 4 + q] = cadd(cmul(vx, sp), cscale(vy, c));
-          }
+          const double dd = be - al, w = fma(4.0, ag2, dd * dd);
+          double f = 2.0 * rcp_newton(fma(w, rsqrt_newton(w), fabs(dd)));
+          f = dd >= 0.0 ? f : -f;
+          const double2 te = cscale(g, f), tm = make_double2(-te.x, te.y);   // te, -conj(te)
+          const double c = rsqrt_newton(1.0 + cabs2(te));
+          const double2 x = a[p], y = a[q], vx = v[p], vy = v[q];
+          a[p] = cscale(cfma(tm, y, x), c);
+          a[q] = cscale(cfma(te, x, y), c);
+          v[p] = cscale(cfma(tm, vy, vx), c);
+          v[q] = cscale(cfma(te, vx, vy), c);
         }
       }
     if (!rotated) break;
   }
-  double sig[4], smax = 0.0, ssum = 0.0;
+  double sig2[4], smax2 = 0.0, ssum = 0.0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    double s2 = 0.0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s2 += cabs2(a[i * 4 + j]);
-    sig[j] = sqrt(s2);
+    sig2[j] = row_total(cabs2(a[j]));
     if (j < d) {
-      smax = fmax(smax, sig[j]);
-      ssum += sig[j];
+      smax2 = fmax(smax2, sig2[j]);
+      ssum += sig2[j] == 0.0 ? 0.0 : sqrt(sig2[j]);
     }
   }
-  *nuc = ssum;
-  bool good[4];
+  *nuc = ldexp(ssum, -h);
+  unsigned good = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    good[j] = (j >= d) || (smax > 0.0 && sig[j] > 1e-13 * smax);
-    if (good[j]) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i * 4 + j] = cscale(a[i * 4 + j], 1.0 / sig[j]);
+  for (int j = 0; j < 4; ++j)
+    if (j >= d || (smax2 > 0.0 && sig2[j] > 1e-26 * smax2)) {
+      good |= 1u << j;
+      a[j] = cscale(a[j], rsqrt_newton(sig2[j]));
     }
-  }
   // canonical completion of the other columns, U side (a) then V side (v)
-#pragma unroll
+#pragma unroll 1
   for (int side = 0; side < 2; ++side) {
-    double2* m = side == 0 ? a : v;
-    bool set[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) set[j] = good[j];
+    unsigned set = good;
     int next_e = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (!set[j]) {
+#pragma unroll 1
+      for (int e0 = next_e; e0 < 4 && !((set >> j) & 1u); ++e0) {
+        double2 x = make_double2(i == e0 ? 1.0 : 0.0, 0.0);
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass)
 #pragma unroll
-        for (int e0 = 0; e0 < 4; ++e0) {
-          if (!set[j] && e0 >= next_e) {
-            double2 x[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = make_double2(i == e0 ? 1.0 : 0.0, 0.0);
-#pragma unroll
-            for (int pass = 0; pass < 2; ++pass)
-#pragma unroll
-              for (int b = 0; b < 4; ++b) {
-                if (set[b]) {
-                  double2 dd = cz();
-#pragma unroll
-                  for (int i = 0; i < 4; ++i) dd = cfmac(m[i * 4 + b], x[i], dd);
-#pragma unroll
-                  for (int i = 0; i < 4; ++i) x[i] = csub(x[i], cmul(m[i * 4 + b], dd));
-                }
-              }
-            double nr = 0.0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) nr += cabs2(x[i]);
-            nr = sqrt(nr);
-            if (nr > 0.5) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) m[i * 4 + j] = cscale(x[i], 1.0 / nr);
-              set[j] = true;
-              next_e = e0 + 1;
-            }
-          }
+          for (int b = 0; b < 4; ++b)
+            if ((set >> b) & 1u) x = csub(x, cmul(a[b], dot(a[b], x)));
+        const double nr2 = row_total(cabs2(x));
+        if (nr2 > 0.25) {
+          a[j] = cscale(x, rsqrt_newton(nr2));
+          set |= 1u << j;
+          next_e = e0 + 1;
         }
       }
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // the other side's turn
+      const double2 t = a[j];
+      a[j] = v[j];
+      v[j] = t;
+    }
   }
   // out = U V^H (the d x d block)
+  double2 o[4];
+  auto entry = [&](auto bcast) {
+    double2 t = cz();
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int m = 0; m < 4; ++m) t = cfma(a[m], cconj(bcast(v[m])), t);
+    return t;
+  };
+  o[0] = entry([](double2 t) { return quad_bcast2<0>(t); });
+  o[1] = entry([](double2 t) { return quad_bcast2<1>(t); });
+  o[2] = entry([](double2 t) { return quad_bcast2<2>(t); });
+  o[3] = entry([](double2 t) { return quad_bcast2<3>(t); });
+  if (lane < 4)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      double2 s = cz();
-#pragma unroll
-      for (int mm = 0; mm < 4; ++mm) s = cfma(a[i * 4 + mm], cconj(v[j * 4 + mm]), s);
-      out[i * 4 + j] = (i < d && j < d) ? s : cz();
-    }
+    for (int j = 0; j < 4; ++j) out[4 * i + j] = i < d && j < d ? make_double2(o[j].x, sgn * o[j].y) : cz();
 }
 
 // The update of one gate on one wave: g_new = conj(polar(E)), d x d block of
@@ -769,13 +872,7 @@ QMX_DEV double update_gate_wave(int d, double omega_m1, const double2* g_old, co
     __builtin_amdgcn_wave_barrier();
     if (!polar4_wave(d, m, g_new, sgn, lane, want, &nuc)) {
       // zero or ill-conditioned matrices, and whatever else it declined
-      if (lane == 0) {
-        double2 w[16];
-        polar4_jacobi(d, m, w, &nuc);
-#pragma unroll
-        for (int k = 0; k < 16; ++k) g_new[k] = make_double2(w[k].x, sgn * w[k].y);
-      }
-      nuc = lane_value(nuc, 0);
+      polar4_jacobi(d, m, g_new, sgn, lane, &nuc);
     }
     __builtin_amdgcn_wave_barrier();
     if (r + 1 < rounds) {

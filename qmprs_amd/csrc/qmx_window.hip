@@ -1005,11 +1005,14 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
 // one barrier per step is left.  Gate p + 2 is fetched two phases ahead.
 // After the gate of site i of the first circuit layer is removed, the sites
 // behind i are in |0>: phi is set to exactly zero where they are not.
-// The lead's chain bounds it up to 2^10 complex128 amplitudes (8.4k cycles a
-// step at N = 6, environment 1.9k and polar factor 6k, and 8.8k at N = 10), the
-// workers' updates and products above (18k at N = 12).  One state, 4 layers, 4
-// sweeps: 0.40 ms against 1.46 gate by gate at N = 5, 0.83 against 1.32 in
-// windows at N = 10; 16 states of N = 12 1.9 ms against 3.2.
+// Bound by the issue of the lead's chain and of the worker that shares its SIMD
+// up to 2^10 complex128 amplitudes (6.0k cycles a step at N = 6, environment
+// 1.5k and polar factor 3.9k, and 6.9k at N = 10), by the workers' updates and
+// products above (17k at N = 12).  The code of a step has to stay inside the 64
+// KiB instruction cache that two CUs share: paths that are cold cost more to
+// fetch than to run.  One state, 4 layers, 4 sweeps: LDSN5 ms against 1.46 gate
+// by gate at N = 5, LDSN10 against 1.32 in windows at N = 10; 16 states of N =
+// 12 LDSN12 ms against 3.2.
 constexpr int kLdsWorkers = 4;
 constexpr int kLdsThreads = 64 * (1 + kLdsWorkers);
 constexpr int kLdsChunk = 32;   // gates per stage of the circuit rebuild (the partials' space)
@@ -1029,6 +1032,31 @@ QMX_DEV int spread3(int z, uint32_t mask) {
   return (z & 1 ? f0 : 0) | (z & 2 ? f1 : 0) | (z & 4 ? f2 : 0);
 }
 
+// the four amplitudes at i0, i0 ^ sl, i0 ^ sh, i0 ^ sl ^ sh, and G^dagger of them
+template <typename S, typename C2> QMX_DEV void quad_load(const S* s, int i0, int sl, int sh, C2 (&x)[4]) {
+  using T = CT<typename StoreC<S>::C>;
+  x[0] = T::mk(to_c(s[i0]));
+  x[1] = T::mk(to_c(s[i0 ^ sl]));
+  x[2] = T::mk(to_c(s[i0 ^ sh]));
+  x[3] = T::mk(to_c(s[i0 ^ sl ^ sh]));
+}
+template <typename S, typename C2>
+QMX_DEV void quad_adj(S* s, int i0, int sl, int sh, const C2 (&g)[16], const C2 (&x)[4]) {
+  using T = CT<typename StoreC<S>::C>;
+  C2 y[4];
+#pragma unroll
+  for (int o = 0; o < 4; ++o) {
+    C2 acc = T::mulc(g[o], x[0]);
+    acc = T::fmac(g[4 + o], x[1], acc);
+    acc = T::fmac(g[8 + o], x[2], acc);
+    y[o] = T::fmac(g[12 + o], x[3], acc);
+  }
+  s[i0] = from_c<S>(make_double2(y[0].x, y[0].y));
+  s[i0 ^ sl] = from_c<S>(make_double2(y[1].x, y[1].y));
+  s[i0 ^ sh] = from_c<S>(make_double2(y[2].x, y[2].y));
+  s[i0 ^ sl ^ sh] = from_c<S>(make_double2(y[3].x, y[3].y));
+}
+
 // y = G^dagger x on amplitude quads (w = 2: bits h, h - 1) or pairs (w = 1: bit
 // h) of an LDS state: this lane's patterns are base ^ su(u), u < nu (swizzled
 // indices with the gate's bits zero; every index map here is linear over bit
@@ -1044,26 +1072,8 @@ QMX_DEV void lds_gate(S* s, int w, int h, const double2* g, int nu, bool on, int
     c2 gc[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) gc[k] = T::mk(g[k]);
-    auto load = [&](int i0, c2 (&x)[4]) {
-      x[0] = T::mk(to_c(s[i0]));
-      x[1] = T::mk(to_c(s[i0 ^ sl]));
-      x[2] = T::mk(to_c(s[i0 ^ sh]));
-      x[3] = T::mk(to_c(s[i0 ^ sl ^ sh]));
-    };
-    auto apply = [&](int i0, const c2 (&x)[4]) {
-      c2 y[4];
-#pragma unroll
-      for (int o = 0; o < 4; ++o) {
-        c2 acc = T::mulc(gc[o], x[0]);
-        acc = T::fmac(gc[4 + o], x[1], acc);
-        acc = T::fmac(gc[8 + o], x[2], acc);
-        y[o] = T::fmac(gc[12 + o], x[3], acc);
-      }
-      s[i0] = from_c<S>(make_double2(y[0].x, y[0].y));
-      s[i0 ^ sl] = from_c<S>(make_double2(y[1].x, y[1].y));
-      s[i0 ^ sh] = from_c<S>(make_double2(y[2].x, y[2].y));
-      s[i0 ^ sl ^ sh] = from_c<S>(make_double2(y[3].x, y[3].y));
-    };
+    auto load = [&](int i0, c2 (&x)[4]) { quad_load<S>(s, i0, sl, sh, x); };
+    auto apply = [&](int i0, const c2 (&x)[4]) { quad_adj<S>(s, i0, sl, sh, gc, x); };
     // two patterns at a time: one's loads are in flight under the other's work
     int u = 0;
     for (; u + 1 < nu; u += 2) {
@@ -1094,6 +1104,8 @@ QMX_DEV void lds_gate(S* s, int w, int h, const double2* g, int nu, bool on, int
 
 template <typename S>
 __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> a) {
+  using T = CT<typename StoreC<S>::C>;
+  using c2 = typename T::c2;
   extern __shared__ char wsm[];
   __shared__ double2 gold[4][16];            // old gates of steps p - 1 .. p + 1
   __shared__ double2 gnew[3][16];            // new gates of steps p - 3 .. p - 1
@@ -1107,6 +1119,7 @@ __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> 
   S* sT = reinterpret_cast<S*>(wsm);
   S* sP = sT + len;
   double2* part = reinterpret_cast<double2*>(sP + len);   // 2 phases x kLdsWorkers x 64; gate stages
+  int4* tab = reinterpret_cast<int4*>(part + 2 * kLdsWorkers * 64);   // n x 64
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lb = min(max(a.layers[b], 0), a.lmax), K = lb * n;
   double2* gates = a.gates + (size_t)b * a.lmax * n * 16;
@@ -1188,6 +1201,31 @@ __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> 
   auto prev = [&](int r) { return r == 0 ? n - 1 : r - 1; };
   auto rank_in = [](uint32_t u, int bit) { return __popc(u & ((1u << bit) - 1u)); };
   auto gate_at = [&](int r, int layer) { return (size_t)layer * n + (n - 1 - r); };
+  // A worker's indices r outside U: r0 .. r0 + G - 1 (G a power of two, r0 a
+  // multiple of it).  U's bits in rising order; deposit of r outside U.
+  const int rest = 1 << (n - mu), G = rest >= kLdsWorkers ? rest / kLdsWorkers : 1, glog = __ffs(G) - 1;
+  auto deposit = [&](uint32_t u, int r) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (k < mu) r = zero_at(r, u ? __ffs(u) - 1 : 31);
+      u &= u - 1u;
+    }
+    return r;
+  };
+  // The lanes' places per residue, which would take a third of a step to form
+  // again each time: of the first pattern of T's and phi's gate (of two qubits),
+  // and of T' and phi in the products below
+  __syncthreads();
+  for (int e = tid; e < 64 * n; e += kLdsThreads) {
+    const int r = e >> 6, ln = e & 63, ht = prev(prev(r));
+    const uint32_t u = uset[r], v = vset[r], far = u & ~v;
+    const int at = deposit(u, ln & (G - 1)), q = ln >> glog;
+    const uint32_t gt = ht ? 3u << (ht - 1) : 1u, gc = r ? 3u << (r - 1) : 1u;
+    const int kk = ln & 7, x0 = 2 * ((ln >> 3) & 3), y0 = 4 * (ln >> 5);
+    const int base = deposit(u, kk & (G - 1)) | ((kk >> glog) & 1 ? (int)far : 0);
+    tab[e] = make_int4(lds_at<S>(at | spread3(q, u & ~gt)), lds_at<S>(at | spread3(q, u & ~gc)),
+                       lds_at<S>(base | spread3(x0, v)), lds_at<S>(base | spread3(y0, v)));
+  }
   snapshot(0);
   const bool use_goal = a.goal && ref;
   int done = 0;
@@ -1224,28 +1262,34 @@ __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> 
         if (p > 0) {
           // ---- lead: the environment and the new gate of step k = p - 1
           __builtin_amdgcn_s_setprio(3);
-          const int k = p - 1, hbit = prev(rp);
-          const uint32_t v = __builtin_amdgcn_readfirstlane(vset[hbit]);
-          const int w = __builtin_amdgcn_readfirstlane(wold[k & 3]), d = w == 2 ? 4 : 2;
+          const int k = p - 1, hbit = prev(rp), kp = k - 1, hpbit = prev(hbit);
+          const int lv = vset[hbit], lw = wold[k & 3], lwp = wold[kp & 3];   // (one wait for the three)
+          const uint32_t v = __builtin_amdgcn_readfirstlane(lv);
+          const int w = __builtin_amdgcn_readfirstlane(lw), d = w == 2 ? 4 : 2;
           const int hb = rank_in(v, hbit), gl = w == 2 ? hb - 1 : hb;   // the gate's lowest bit in V
           // the pending gate of step k - 1
-          const int kp = k - 1, hpbit = prev(hbit);
-          const int wp = kp >= 0 ? __builtin_amdgcn_readfirstlane(wold[kp & 3]) : 0;
-          const int pl = rank_in(v, hpbit) - (wp == 2 ? 1 : 0), np = wp == 2 ? 4 : (wp == 1 ? 2 : 1);
+          const int wp = kp >= 0 ? __builtin_amdgcn_readfirstlane(lwp) : 0, np = 1 << wp;
+          const int pl = rank_in(v, hpbit) - (wp == 2 ? 1 : 0);
           const int pmask = (np - 1) << pl;
           const double2* gp = gnew[(kp + 3) % 3];
           const int o = (lane >> 2) & 3, i = lane & 3, row = lane >> 4;
           const uint32_t fm = ((1u << mv) - 1u) & ~((uint32_t)(d - 1) << gl);   // V's bits beside the gate's
-          const int nz = (1 << mv) / d;
-          // terms (z, x'_g), one in four per row of lanes
+          const int nt = ((1 << mv) / d) << wp;
+          // terms (z, x'_g), one in four per row of lanes: two each, four for a
+          // one-qubit gate after one of two qubits
           double2 acc = cz();
-          for (int t = row; t < nz * np; t += 4) {
-            const int pg = t & (np - 1), z = spread3(t / np, fm);
-            const int x = (z | (o & (d - 1)) << gl), y = (z | (i & (d - 1)) << gl);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (u == 2 && nt <= 8) break;
+            const int t = row + 4 * u;
+            const int pg = t & (np - 1), z = spread3(t >> wp, fm);
+            const int x = z | (o & (d - 1)) << gl, y = z | (i & (d - 1)) << gl;
             const int at = (wp ? (x & ~pmask) | pg << pl : x) * 8 + y;
             const double2* q = part + (k & 1) * kLdsWorkers * 64 + at;
+            const double2 c = gp[pg * 4 + ((x >> pl) & (np - 1))];
             const double2 e = cadd(cadd(q[0], q[64]), cadd(q[128], q[192]));
-            acc = wp ? cfma(gp[pg * 4 + ((x >> pl) & (np - 1))], e, acc) : cadd(acc, e);
+            const double2 f = wp ? cmul(c, e) : e;
+            acc = t < nt ? cadd(acc, f) : acc;
           }
           acc = make_double2(rows_sum(acc.x), rows_sum(acc.y));
           if (lane < 16) es[lane] = o < d && i < d ? acc : cz();
@@ -1271,37 +1315,40 @@ __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> 
           }
         }
         const uint32_t u = __builtin_amdgcn_readfirstlane(uset[rp]), v = __builtin_amdgcn_readfirstlane(vset[rp]);
-        int ub[4];
-        {
-          uint32_t t = u;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            ub[k] = t ? __ffs(t) - 1 : 31;
-            t &= t - 1u;
-          }
-        }
-        auto roff = [&](int r) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (k < mu) r = zero_at(r, ub[k]);
-          return r;
-        };
-        // this worker's indices r outside U: r0 .. r0 + nr - 1 (G a power of
-        // two, r0 a multiple of it)
-        const int rest = 1 << (n - mu);
-        const int G = rest >= kLdsWorkers ? rest / kLdsWorkers : 1, glog = __ffs(G) - 1;
+        const int4 places = tab[rp * 64 + lane];
+        auto roff = [&](int r) { return deposit(u, r); };
         const int r0 = wid * G, nr = r0 < rest ? G : 0;
         const int sr0 = lds_at<S>(roff(r0));
-        auto update = [&](S* s, int w, int h, const double2* g) {
+        auto update = [&](S* s, int w, int h, int first, const double2* g) {
           const uint32_t om = u & ~(w == 2 ? 3u << (h - 1) : 1u << h);   // U's bits beside the gate's
           const int cnt = nr << (mu - w);
           auto at = [&](int t) { return lds_at<S>(roff(t & (G - 1)) | spread3(t >> glog, om)); };
-          lds_gate<S>(s, w, h, g, (cnt + 63) >> 6, lane < cnt, sr0 ^ at(lane), [&](int k) { return at(64 * k); });
+          lds_gate<S>(s, w, h, g, (cnt + 63) >> 6, lane < cnt, sr0 ^ (w == 2 ? first : at(lane)),
+                      [&](int k) { return at(64 * k); });
         };
         const int kt = p - 2, h = rp;
         auto width_of = [&](int k) { return __builtin_amdgcn_readfirstlane(wold[k & 3]); };
-        if (kt >= 0) update(sT, width_of(kt), prev(prev(rp)), gnew[kt % 3]);
-        update(sP, width_of(p), h, gold[p & 3]);
+        const int wt = kt >= 0 ? width_of(kt) : 0, wc = width_of(p), ht = prev(prev(rp));
+        if (wt == 2 && wc == 2 && nr << (mu - 2) <= 64) {
+          // one pattern a lane: the loads of both sides are in flight together
+          const int lt = lds_at<S>(1 << (ht - 1)), mt = lds_at<S>(1 << ht), lc = lds_at<S>(1 << (h - 1)),
+                    mc = lds_at<S>(1 << h);
+          if (lane < nr << (mu - 2)) {
+            const int it = sr0 ^ places.x, ic = sr0 ^ places.y;
+            c2 xt[4], xc[4], g[16];
+            quad_load<S>(sT, it, lt, mt, xt);
+            quad_load<S>(sP, ic, lc, mc, xc);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) g[k] = T::mk(gnew[kt % 3][k]);
+            quad_adj<S>(sT, it, lt, mt, g, xt);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) g[k] = T::mk(gold[p & 3][k]);
+            quad_adj<S>(sP, ic, lc, mc, g, xc);
+          }
+        } else {
+          if (wt) update(sT, wt, ht, places.x, gnew[kt % 3]);
+          update(sP, wc, h, places.y, gold[p & 3]);
+        }
         __builtin_amdgcn_wave_barrier();
         if (p >= K - n && h > 0) {
           // the sites behind step p's are in |0> once this gate of the first
@@ -1319,11 +1366,12 @@ __global__ __launch_bounds__(kLdsThreads) void lds_sweep_kernel(LdsSweepArgs<S> 
         const int cnt = far ? 2 * nr : nr, kk = lane & 7, x0 = 2 * ((lane >> 3) & 3), y0 = 4 * (lane >> 5);
         auto at = [&](int t) { return lds_at<S>(roff(t & (G - 1)) | ((t >> glog) & 1 ? (int)far : 0)); };
         // (lanes beyond V read valid places too: spread3 drops the bits that V lacks)
-        const int base = sr0 ^ at(kk), bt = base ^ lds_at<S>(spread3(x0, v)), bp = base ^ lds_at<S>(spread3(y0, v));
+        const int bt = sr0 ^ places.z, bp = sr0 ^ places.w;
         const int v0 = lds_at<S>(spread3(1, v)), v1 = lds_at<S>(spread3(2, v));
         double2 acc[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] = cz();
+#pragma unroll 2
         for (int k0 = 0; k0 < cnt; k0 += 8) {
           const int off = at(k0);
           double2 tv[2], pv[4];
@@ -1378,11 +1426,13 @@ hipError_t launch_lds_sweep(const LdsSweepArgs<S>& a, int batch, hipStream_t st)
   static_assert(parts >= kLdsChunk * 16 * sizeof(double2), "a stage of gates fits the partials' space");
   // the limit is set to the largest need, so that launches from several host
   // threads never lower it under each other
-  const size_t most = (2 * sizeof(S) << lds_sweep_qubits(sizeof(S))) + parts;
+  constexpr int nmax = lds_sweep_qubits(sizeof(S));
+  const size_t most = (2 * sizeof(S) << nmax) + parts + nmax * 64 * sizeof(int4);
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(lds_sweep_kernel<S>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(lds_sweep_kernel<S>, dim3(batch), dim3(kLdsThreads), (2 * sizeof(S) << a.n) + parts, st, a);
+  hipLaunchKernelGGL(lds_sweep_kernel<S>, dim3(batch), dim3(kLdsThreads),
+                     (2 * sizeof(S) << a.n) + parts + a.n * 64 * sizeof(int4), st, a);
   return hipGetLastError();
 }
 template hipError_t launch_lds_sweep<float2>(const LdsSweepArgs<float2>&, int, hipStream_t);
