@@ -1115,12 +1115,12 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
                    double2* snapshots = nullptr) {
   // Small states are swept by one block each, in one launch: their sweeps are
   // chains of polar factors, and a launch per window or gate costs more than
-  // its work (complex128, 4 layers, 4 sweeps: N=5 0.40 ms against 1.46 gate by
-  // gate; N=11 1.16 against 1.55 in windows, for 16 states 1.19 against 2.93).
+  // its work (complex128, 4 layers, 4 sweeps: N=5 0.30 ms against 0.86 gate by
+  // gate; N=11 1.10 against 1.50 in windows, for 16 states 1.10 against 2.90).
   // At the largest N a block has a CU for itself and is bound by its one CU's
-  // work, so a lone state (1.88 ms against 1.70 in windows at N=12) and batches
+  // work, so a lone state (1.8 ms against 1.65 in windows at N=12) and batches
   // that run in more than two rounds over the CUs (600 complex64 states of
-  // N=13: 10.2 against 8.8) stay in windows.  Snapshots with a goal keep the
+  // N=13: 10 against 6.4) stay in windows.  Snapshots with a goal keep the
   // windows too: whether one is written depends on the whole batch there.  And
   // so does a goal on a capturing stream: the windows' host check ends such a
   // capture with an error at every size.

@@ -1412,7 +1412,7 @@ __global__ __launch_bounds__(256) void bj_store_kernel(const double2* cur_all, c
 // max bond chi; k = n when n <= chi), and write the sorted eigenvectors into
 // the columns of w (same layout as v).  k_out[b] = k; spectra (optional).
 // Every block of a state sorts for itself and copies its rows of w; the first
-// one also picks k.  SELFIG
+// one also picks k (600 columns: 36 us, in one block 192).
 constexpr int kSelectRows = 16;
 __global__ __launch_bounds__(512) void select_kernel(const double2* a_all, const double2* v_all,
                                                      double2* w_all, size_t stride,
