@@ -102,12 +102,10 @@ const char* qmx_last_error(const qmx_handle* h);
 #define QMX_OPT_FAIL_UNITARITY 8
 /* QMX_OPT_TWO_SIDED_JACOBI: 1 takes the chi-truncation's eigenproblems through
  * the two-sided Jacobi instead of the one-sided one (0, the default, five to
- * fourteen times faster and closer to an SVD; above 128 columns it waits for
- * the stream once per sweep, so a capturing stream keeps the two-sided one
- * there), and the layers' 4 x 4 eigenproblems through one lane instead of a
- * wave.  Both give the truncated state to rounding; 1 keeps the exact rounding of the two-sided
- * solver, which the layers of a deep circuit amplify (see
- * qmprs_amd/primitives/mps.py). */
+ * fourteen times faster and closer to an SVD), and the layers' 4 x 4
+ * eigenproblems through one lane instead of a wave.  Both give the truncated
+ * state to rounding; 1 keeps the exact rounding of the two-sided solver, which
+ * the layers of a deep circuit amplify (see qmprs_amd/primitives/mps.py). */
 #define QMX_OPT_TWO_SIDED_JACOBI 10
 int qmx_set_option(qmx_handle* h, int option, int value);
 

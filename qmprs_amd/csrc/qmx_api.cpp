@@ -573,15 +573,6 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
     timer.stop(1);
     return QMX_OK;
   }
-  // Above 128 columns the one-sided solver reads its convergence on the host
-  // once per sweep, so a capturing stream keeps the two-sided ones (up to 512
-  // columns they can be captured).
-  bool wide = false;
-  if (!h->two_sided && L.jdiag) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    QMX_HIP(h, hipStreamIsCapturing(st, &cs));
-    wide = cs == hipStreamCaptureStatusNone;
-  }
   const int nmax = L.nmax;
   const size_t nm2 = static_cast<size_t>(nmax) * nmax;
   const int kmax = std::min(chi, nmax);
@@ -596,7 +587,7 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
     launch_gram_reduce(L.part, nchunks, L.ncur, nmax, L.a, nm2, batch, st);
     // sweep limits of the eigensolvers; QMX_OPT_JACOBI_SWEEP_CAP lowers them
     auto cap = [&](int limit) { return h->jacobi_sweep_cap > 0 ? std::min(limit, h->jacobi_sweep_cap) : limit; };
-    if (wide) {
+    if (!h->two_sided && L.jdiag) {   // above 128 columns
       std::vector<int> conv(batch);
       if (launch_osj_wide(L.a, L.v, nm2, L.ncur, nmax, rows, batch, spectra ? 0 : chi, L.jrank, L.jdiag, conv.data(),
                           cap(kJacobiBlockSweeps), L.error, st) != 0)

@@ -105,7 +105,7 @@ __global__ void gram_reduce_kernel(const double2* part, int nchunks, const int* 
 }
 
 // ---------------------------------------------------------------- jacobi ----
-// QMX_OPT_TWO_SIDED_JACOBI, and capturing streams, for 129 to 512 columns.
+// QMX_OPT_TWO_SIDED_JACOBI for 129 to 512 columns.
 // Parallel cyclic two-sided Jacobi for a Hermitian n x n matrix (n even,
 // n <= 2 * 256), one block per state.  Round r pairs the indices by the circle
 // method; all n/2 rotations of a round are disjoint, so the update
@@ -243,10 +243,18 @@ constexpr int kJacobiRowsPerBlock = 16;
 
 QMX_DEV int tri_index(int i, int j, int n) { return i * (2 * n - i + 1) / 2 + (j - i); }
 
-__global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, size_t stride,
+// kAll: V (n x n) is in LDS too and takes the rotations of a round with A, all
+// sweeps run in one launch (sweep = their limit; no log, no state).  The host
+// takes it up to kJacobiAllMax columns, where two launches per sweep, most of
+// them after the last one, cost more than the one CU that V then has (the chain
+// of one N = 15 state: 3.6 ms against 4.8 at 32 columns, 6.1 against 6.7 at 48,
+// 7.5 both at 56, 9.0 against 8.1 at 64).
+constexpr int kJacobiAllMax = 48;
+template <bool kAll>
+__global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, double2* v_all, size_t stride,
                                                                 const int* ncols_dev, int ld,
                                                                 double4* log_all, size_t log_stride,
-                                                                int* state, int sweep) {
+                                                                int* state, int sweep, int* error) {
   extern __shared__ double2 tri[];
   __shared__ int4 pq[kJacobiLdsMax / 2];             // p, q and their rows' places
   __shared__ double2 jcs[kJacobiLdsMax / 2], je[kJacobiLdsMax / 2];
@@ -254,49 +262,28 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
   __shared__ double s_scale;
   const int b = blockIdx.x;
   // state[b]: 0 = running, 1 = converged; state[batch + b] = sweeps run
-  if (state[b]) return;
+  if (!kAll && state[b]) return;
   const int n = ncols_dev[b];
+  double2* a = a_all + (size_t)b * stride;
+  double2* v = v_all + (size_t)b * stride;
   if (n < 2) {
-    if (threadIdx.x == 0) state[b] = 1;
+    if (threadIdx.x == 0) {
+      if (kAll && n == 1) v[0] = make_double2(1.0, 0.0);
+      if (!kAll) state[b] = 1;
+    }
     return;
   }
-  double2* a = a_all + (size_t)b * stride;
   double4* lg = log_all + (size_t)b * log_stride;
+  double2* vl = tri + ld * (ld + 1) / 2;
   const int tid = threadIdx.x, nt = blockDim.x;
   const int lane = tid & 63, wave = tid >> 6, waves = nt >> 6;
   // entry (i, j) of the triangle is at rowbase(i) + j; a wave per row
   auto rowbase = [&](int i) { return i * (2 * n - i + 1) / 2 - i; };
   for (int i = wave; i < n; i += waves)
     for (int j = i + lane; j < n; j += 64) tri[rowbase(i) + j] = a[(size_t)i * ld + j];
-  __syncthreads();
-  if (tid == 0) {
-    any_rot = 0;
-    double tr = 0.0;
-#pragma unroll 16
-    for (int i = 0; i < n; ++i) tr += fabs(tri[rowbase(i) + i].x);
-    s_scale = tr;
-  }
-  __syncthreads();
+  if constexpr (kAll)
+    for (int e = tid; e < n * n; e += nt) vl[e] = make_double2(e / n == e % n ? 1.0 : 0.0, 0.0);
   const int np = n / 2;
-  const double abs_tol = kJacobiAbsTol * s_scale + 1e-300;
-  // a sweep would rotate nothing iff no off-diagonal entry passes the rotation
-  // test now: then the state is converged and the sweep is not run
-  for (int i = wave; i < n; i += waves) {
-    const double al = tri[rowbase(i) + i].x;
-    for (int j = i + 1 + lane; j < n; j += 64) {
-      const double ag = cabs_(tri[rowbase(i) + j]);
-      if (ag > abs_tol && ag > 1e-15 * sqrt(fabs(al * tri[rowbase(j) + j].x))) any_rot = 1;
-    }
-  }
-  __syncthreads();
-  const bool go = any_rot;
-  __syncthreads();
-  if (!go) {
-    if (tid == 0) state[b] = 1;
-    return;
-  }
-  if (tid == 0) any_rot = 0;
-  __syncthreads();
   // this thread's pair blocks (P, Q), P < Q, row-major over the strict upper
   // triangle of pair blocks; the same in every round (the kernel is launched
   // with 1024 threads: two blocks each cover the 2016 of n = 128).  The diagonal
@@ -319,95 +306,151 @@ __global__ __launch_bounds__(1024) void jacobi_lds_sweep_kernel(double2* a_all, 
     bP[k] = P;
     bQ[k] = Q;
   }
-  for (int r = 0; r < n - 1; ++r) {
-    double c = 1.0, sn = 0.0;
-    double2 em = make_double2(1.0, 0.0), g = cz(), app = cz(), aqq = cz();
-    int ipp = 0, ipq = 0, iqq = 0;
-    if (tid < np) {
-      const int m = tid;
-      int p = (m == 0) ? n - 1 : (r + m) % (n - 1);
-      int q = (r + n - 1 - m) % (n - 1);
-      if (m == 0) q = r % (n - 1);
-      if (p > q) { int t = p; p = q; q = t; }
-      const int bp = rowbase(p), bq = rowbase(q);
-      ipp = bp + p;
-      ipq = bp + q;
-      iqq = bq + q;
-      app = tri[ipp];
-      aqq = tri[iqq];
-      g = tri[ipq];
-      const double al = app.x, be = aqq.x;
-      const double ag = cabs_(g);
-      // one comparison against the larger threshold: the diagonal reads are
-      // issued together with the off-diagonal one
-      if (ag > fmax(abs_tol, 1e-15 * sqrt(fabs(al * be)))) {
-        const double tau = (be - al) / (2.0 * ag);
-        const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-        c = 1.0 / sqrt(1.0 + t * t);
-        sn = t * c;
-        em = make_double2(g.x / ag, -g.y / ag);   // e^{-i phi}
-        any_rot = 1;
+  bool converged = false, ran = false;
+  for (int s = 0; s < (kAll ? sweep : 1); ++s) {
+    __syncthreads();
+    if (tid == 0) {
+      any_rot = 0;
+      double tr = 0.0;
+#pragma unroll 16
+      for (int i = 0; i < n; ++i) tr += fabs(tri[rowbase(i) + i].x);
+      s_scale = tr;
+    }
+    __syncthreads();
+    const double abs_tol = kJacobiAbsTol * s_scale + 1e-300;
+    // a sweep would rotate nothing iff no off-diagonal entry passes the rotation
+    // test now: then the state is converged and the sweep is not run
+    for (int i = wave; i < n; i += waves) {
+      const double al = tri[rowbase(i) + i].x;
+      for (int j = i + 1 + lane; j < n; j += 64) {
+        const double ag = cabs_(tri[rowbase(i) + j]);
+        if (ag > abs_tol && ag > 1e-15 * sqrt(fabs(al * tri[rowbase(j) + j].x))) any_rot = 1;
       }
-      pq[m] = make_int4(p, q, bp, bq);
-      jcs[m] = make_double2(c, sn);
-      je[m] = em;
-      lg[(size_t)r * np + m] = make_double4(c, sn, em.x, em.y);
     }
     __syncthreads();
-    // blocks (P, Q), P <= Q: B' = J_P^H B J_Q with B = A[{p0, p1}][{q0, q1}];
-    // (Q, P) is its conjugate transpose and is never stored separately
-    auto turn = [](double2 a00, double2 a01, double2 a10, double2 a11, double2 kcs, double2 ke, double2 qcs,
-                   double2 qe, double2& c00, double2& c01, double2& c10, double2& c11) {
-      const double2 J00 = make_double2(qcs.x, 0.0), J01 = make_double2(qcs.y, 0.0);
-      const double2 J10 = cscale(qe, -qcs.y), J11 = cscale(qe, qcs.x);
-      const double2 K00 = make_double2(kcs.x, 0.0), K01 = make_double2(kcs.y, 0.0);
-      const double2 K10 = cscale(ke, -kcs.y), K11 = cscale(ke, kcs.x);
-      const double2 b00 = cadd(cmul(a00, J00), cmul(a01, J10));
-      const double2 b01 = cadd(cmul(a00, J01), cmul(a01, J11));
-      const double2 b10 = cadd(cmul(a10, J00), cmul(a11, J10));
-      const double2 b11 = cadd(cmul(a10, J01), cmul(a11, J11));
-      c00 = cadd(cmulc(K00, b00), cmulc(K10, b10));
-      c01 = cadd(cmulc(K00, b01), cmulc(K10, b11));
-      c10 = cadd(cmulc(K01, b00), cmulc(K11, b10));
-      c11 = cadd(cmulc(K01, b01), cmulc(K11, b11));
-    };
-    if (tid < np) {
-      double2 c00, c01, c10, c11;
-      // (the diagonal's zero imaginary parts come from memory, so that the
-      // compiler cannot fold them and round these blocks otherwise)
-      turn(app, g, cconj(g), aqq, make_double2(c, sn), em, make_double2(c, sn), em, c00, c01, c10, c11);
-      tri[ipp] = make_double2(c00.x, 0.0);
-      tri[ipq] = cz();
-      tri[iqq] = make_double2(c11.x, 0.0);
+    const bool go = any_rot;
+    __syncthreads();
+    if (!go) {
+      converged = true;
+      break;
     }
+    if (tid == 0) any_rot = 0;
+    ran = true;
+    __syncthreads();
+    for (int r = 0; r < n - 1; ++r) {
+      double c = 1.0, sn = 0.0;
+      double2 em = make_double2(1.0, 0.0), g = cz(), app = cz(), aqq = cz();
+      int ipp = 0, ipq = 0, iqq = 0;
+      if (tid < np) {
+        const int m = tid;
+        int p = (m == 0) ? n - 1 : (r + m) % (n - 1);
+        int q = (r + n - 1 - m) % (n - 1);
+        if (m == 0) q = r % (n - 1);
+        if (p > q) { int t = p; p = q; q = t; }
+        const int bp = rowbase(p), bq = rowbase(q);
+        ipp = bp + p;
+        ipq = bp + q;
+        iqq = bq + q;
+        app = tri[ipp];
+        aqq = tri[iqq];
+        g = tri[ipq];
+        const double al = app.x, be = aqq.x;
+        const double ag = cabs_(g);
+        // one comparison against the larger threshold: the diagonal reads are
+        // issued together with the off-diagonal one
+        if (ag > fmax(abs_tol, 1e-15 * sqrt(fabs(al * be)))) {
+          const double tau = (be - al) / (2.0 * ag);
+          const double t = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+          c = 1.0 / sqrt(1.0 + t * t);
+          sn = t * c;
+          em = make_double2(g.x / ag, -g.y / ag);   // e^{-i phi}
+          any_rot = 1;
+        }
+        pq[m] = make_int4(p, q, bp, bq);
+        jcs[m] = make_double2(c, sn);
+        je[m] = em;
+        if constexpr (!kAll) lg[(size_t)r * np + m] = make_double4(c, sn, em.x, em.y);
+      }
+      __syncthreads();
+      // blocks (P, Q), P <= Q: B' = J_P^H B J_Q with B = A[{p0, p1}][{q0, q1}];
+      // (Q, P) is its conjugate transpose and is never stored separately
+      auto turn = [](double2 a00, double2 a01, double2 a10, double2 a11, double2 kcs, double2 ke, double2 qcs,
+                     double2 qe, double2& c00, double2& c01, double2& c10, double2& c11) {
+        const double2 J00 = make_double2(qcs.x, 0.0), J01 = make_double2(qcs.y, 0.0);
+        const double2 J10 = cscale(qe, -qcs.y), J11 = cscale(qe, qcs.x);
+        const double2 K00 = make_double2(kcs.x, 0.0), K01 = make_double2(kcs.y, 0.0);
+        const double2 K10 = cscale(ke, -kcs.y), K11 = cscale(ke, kcs.x);
+        const double2 b00 = cadd(cmul(a00, J00), cmul(a01, J10));
+        const double2 b01 = cadd(cmul(a00, J01), cmul(a01, J11));
+        const double2 b10 = cadd(cmul(a10, J00), cmul(a11, J10));
+        const double2 b11 = cadd(cmul(a10, J01), cmul(a11, J11));
+        c00 = cadd(cmulc(K00, b00), cmulc(K10, b10));
+        c01 = cadd(cmulc(K00, b01), cmulc(K10, b11));
+        c10 = cadd(cmulc(K01, b00), cmulc(K11, b10));
+        c11 = cadd(cmulc(K01, b01), cmulc(K11, b11));
+      };
+      if (tid < np) {
+        double2 c00, c01, c10, c11;
+        // (the diagonal's zero imaginary parts come from memory, so that the
+        // compiler cannot fold them and round these blocks otherwise)
+        turn(app, g, cconj(g), aqq, make_double2(c, sn), em, make_double2(c, sn), em, c00, c01, c10, c11);
+        tri[ipp] = make_double2(c00.x, 0.0);
+        tri[ipq] = cz();
+        tri[iqq] = make_double2(c11.x, 0.0);
+      }
 #pragma unroll
-    for (int k = 0; k < kBlkPer; ++k) {
-      if (tid + k * nt >= nblocks) break;
-      const int P = bP[k], Q = bQ[k];
-      const int4 u = pq[P], w = pq[Q];
-      // one LDS access per entry: (i, j) with i > j is the conjugate of (j, i)
-      auto at = [&](int i, int bi, int j, int bj) { return i > j ? bj + i : bi + j; };
-      const int i00 = at(u.x, u.z, w.x, w.z), i01 = at(u.x, u.z, w.y, w.w);
-      const int i10 = at(u.y, u.w, w.x, w.z), i11 = at(u.y, u.w, w.y, w.w);
-      auto flip = [](double2 v, bool lo) { return make_double2(v.x, lo ? -v.y : v.y); };
-      const double2 a00 = flip(tri[i00], u.x > w.x), a01 = flip(tri[i01], u.x > w.y);
-      const double2 a10 = flip(tri[i10], u.y > w.x), a11 = flip(tri[i11], u.y > w.y);
-      double2 c00, c01, c10, c11;
-      turn(a00, a01, a10, a11, jcs[P], je[P], jcs[Q], je[Q], c00, c01, c10, c11);
-      tri[i00] = flip(c00, u.x > w.x);
-      tri[i01] = flip(c01, u.x > w.y);
-      tri[i10] = flip(c10, u.y > w.x);
-      tri[i11] = flip(c11, u.y > w.y);
+      for (int k = 0; k < kBlkPer; ++k) {
+        if (tid + k * nt >= nblocks) break;
+        const int P = bP[k], Q = bQ[k];
+        const int4 u = pq[P], w = pq[Q];
+        // one LDS access per entry: (i, j) with i > j is the conjugate of (j, i)
+        auto at = [&](int i, int bi, int j, int bj) { return i > j ? bj + i : bi + j; };
+        const int i00 = at(u.x, u.z, w.x, w.z), i01 = at(u.x, u.z, w.y, w.w);
+        const int i10 = at(u.y, u.w, w.x, w.z), i11 = at(u.y, u.w, w.y, w.w);
+        auto flip = [](double2 v, bool lo) { return make_double2(v.x, lo ? -v.y : v.y); };
+        const double2 a00 = flip(tri[i00], u.x > w.x), a01 = flip(tri[i01], u.x > w.y);
+        const double2 a10 = flip(tri[i10], u.y > w.x), a11 = flip(tri[i11], u.y > w.y);
+        double2 c00, c01, c10, c11;
+        turn(a00, a01, a10, a11, jcs[P], je[P], jcs[Q], je[Q], c00, c01, c10, c11);
+        tri[i00] = flip(c00, u.x > w.x);
+        tri[i01] = flip(c01, u.x > w.y);
+        tri[i10] = flip(c10, u.y > w.x);
+        tri[i11] = flip(c11, u.y > w.y);
+      }
+      if constexpr (kAll) {
+        // V <- V J, a wave per row and a lane per pair
+        if (lane < np) {
+          const int4 u = pq[lane];
+          const double2 cs = jcs[lane], em = je[lane];
+          const double2 J00 = make_double2(cs.x, 0.0), J01 = make_double2(cs.y, 0.0);
+          const double2 J10 = cscale(em, -cs.y), J11 = cscale(em, cs.x);
+          for (int i = wave; i < n; i += waves) {
+            const double2 x = vl[i * n + u.x], y = vl[i * n + u.y];
+            vl[i * n + u.x] = cadd(cmul(x, J00), cmul(y, J10));
+            vl[i * n + u.y] = cadd(cmul(x, J01), cmul(y, J11));
+          }
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
+    if (!any_rot) {   // a sweep that rotated nothing leaves the log at identity
+      converged = true;
+      break;
+    }
   }
-  // write the triangle back (the lower part stays stale: readers use i <= j)
-  for (int i = wave; i < n; i += waves)
-    for (int j = i + lane; j < n; j += 64) a[(size_t)i * ld + j] = tri[rowbase(i) + j];
-  if (tid == 0) {
-    state[gridDim.x + b] = sweep + 1;
-    // a sweep that rotated nothing leaves the log at identity: converged
-    if (!any_rot) state[b] = 1;
+  if constexpr (kAll) {
+    __syncthreads();
+    for (int e = tid; e < n * n; e += nt) v[(size_t)(e / n) * ld + e % n] = vl[e];
+    for (int i = tid; i < n; i += nt) a[(size_t)i * ld + i] = tri[rowbase(i) + i];
+    if (tid == 0 && !converged && error) atomicOr(error, kErrEigNoConv);
+  } else {
+    // (a sweep that was not run has neither changed A nor a log)
+    if (tid == 0 && converged) state[b] = 1;
+    if (!ran) return;
+    // write the triangle back (the lower part stays stale: readers use i <= j)
+    for (int i = wave; i < n; i += waves)
+      for (int j = i + lane; j < n; j += 64) a[(size_t)i * ld + j] = tri[rowbase(i) + j];
+    if (tid == 0) state[gridDim.x + b] = sweep + 1;
   }
 }
 
@@ -1652,12 +1695,18 @@ void launch_jacobi_lds(double2* a, double2* v, size_t stride, const int* ncols_d
   const size_t tri_bytes = sizeof(double2) * (size_t)ncols_max * (ncols_max + 1) / 2;
   const size_t log_stride = (size_t)(ncols_max - 1) * (ncols_max / 2);
   double4* lg = reinterpret_cast<double4*>(log);
+  if (ncols_max <= kJacobiAllMax) {
+    hipLaunchKernelGGL(jacobi_lds_sweep_kernel<true>, dim3(batch), dim3(1024),
+                       tri_bytes + sizeof(double2) * (size_t)ncols_max * ncols_max, st, a, v, stride, ncols_dev,
+                       ncols_max, lg, log_stride, state, max_sweeps, error);
+    return;
+  }
   hipLaunchKernelGGL(jacobi_lds_init_kernel, dim3((ncols_max * ncols_max + 255) / 256, batch), dim3(256), 0,
                      st, v, stride, ncols_dev, ncols_max, state, batch);
   const int row_blocks = (ncols_max + kJacobiRowsPerBlock - 1) / kJacobiRowsPerBlock;
   for (int s = 0; s < max_sweeps; ++s) {
-    hipLaunchKernelGGL(jacobi_lds_sweep_kernel, dim3(batch), dim3(1024), tri_bytes, st, a, stride,
-                       ncols_dev, ncols_max, lg, log_stride, state, s);
+    hipLaunchKernelGGL(jacobi_lds_sweep_kernel<false>, dim3(batch), dim3(1024), tri_bytes, st, a, v, stride,
+                       ncols_dev, ncols_max, lg, log_stride, state, s, error);
     hipLaunchKernelGGL(jacobi_lds_rows_kernel, dim3(row_blocks, batch), dim3(1024), 0, st, v, stride,
                        ncols_dev, ncols_max, lg, log_stride, state, s);
   }
@@ -1672,7 +1721,12 @@ void launch_jacobi_lds(double2* a, double2* v, size_t stride, const int* ncols_d
 hipError_t jacobi_lds_setup(int ncols_max) {
   if (ncols_max > kJacobiLdsMax) return hipErrorInvalidValue;
   const size_t tri_bytes = sizeof(double2) * (size_t)kJacobiLdsMax * (kJacobiLdsMax + 1) / 2;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(jacobi_lds_sweep_kernel),
+  const size_t all_bytes = sizeof(double2) * ((size_t)kJacobiAllMax * (kJacobiAllMax + 1) / 2 +
+                                              (size_t)kJacobiAllMax * kJacobiAllMax);
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(jacobi_lds_sweep_kernel<true>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)all_bytes);
+  if (e != hipSuccess) return e;
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(jacobi_lds_sweep_kernel<false>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)tri_bytes);
 }
 
