@@ -28,7 +28,9 @@ pass (window_pass_kernel): per launch it reads T' and phi and writes both
 back, 32 B per complex64 amplitude per active state (24 B for the first
 window of a sweep, which reads the target and writes no T', 16 B for the
 last, whose results are not read again), so algorithmic bytes = state-sweeps
-x 2^N x (32 (W - 2) + 24 + 16) over the W windows of a sweep.  Divided by the
+x 2^N x (32 (W - 2) + 24 + 16) over the W windows of a sweep, less what the
+passes over the first circuit layer's gates leave out (see _live_fractions:
+the last windows visit only the amplitudes that are not exactly zero).  Divided by the
 summed launch durations, measured with HIP events recorded by the library
 on the stream the kernel is launched on, launch by launch, over the timed
 steps.  ``traffic`` comes from two rocprofv3 counter runs (FETCH_SIZE, then
@@ -151,9 +153,34 @@ def cpu_baseline(svs: np.ndarray, wl: dict, gpu_fid_trace=None, seeds: int = 3, 
     return out
 
 
+def _live_fractions(n: int, windows: int) -> list[float]:
+    """The part of the state that each of a sweep's window passes visits: in the
+    last n steps the bits below the removed gates are in |0>, and from five
+    such bits on the amplitudes where they are set are left out."""
+    for layers in range(1, windows + 1):
+        starts, s = [], 0
+        while s < layers * n:
+            starts.append(s)
+            bits: set[int] = set()
+            while s < layers * n and s - starts[-1] < 8:
+                r = s % n
+                more = bits | ({r, r - 1} if r else {r})
+                if len(more) > 4:
+                    break
+                bits, s = more, s + 1
+        if len(starts) >= windows:
+            break
+    dead = [(s0 - 1) % n if s0 > (layers - 1) * n else 0 for s0 in starts[:windows]]
+    return [2.0 ** -d if d >= 5 else 1.0 for d in dead]
+
+
 def _algorithmic_bytes(n: int, windows: int, state_sweeps: float) -> float:
-    amp_bytes = 16.0 if windows == 1 else (32.0 * (windows - 2) + 24.0 + 16.0)
-    return state_sweeps * (2 ** n) * amp_bytes
+    live = _live_fractions(n, windows)
+    amp_bytes = [32.0] * windows
+    amp_bytes[0] -= 8.0
+    amp_bytes[-1] -= 16.0
+    return state_sweeps * (2 ** n) * sum(a * f for a, f in zip(amp_bytes, live)) if windows > 1 \
+        else state_sweeps * (2 ** n) * 16.0
 
 
 def traffic_probe(args) -> int:
