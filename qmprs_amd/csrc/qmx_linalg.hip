@@ -943,7 +943,8 @@ __global__ __launch_bounds__(kOsjWide) void pchol_panel_kernel(const double2* a_
       return;
     }
     if (row == 0) diag[ld] = tr;
-    if (row < 16) wbest[row] = -inf;
+    // (only for waves that are not there: the others write theirs next)
+    if (row < 16 && row >= (int)(blockDim.x >> 6)) wbest[row] = -inf;
     if (row >= n) d = -inf;
   } else {
     if (rank_all[b] != k0) return;
