@@ -112,3 +112,34 @@ def _against_steps(gpu, sweep_mode, dtype, n, layers, used):
                 assert (gates[i] - after).abs().max() < 1e-14
     finally:
         _lib.set_sweep_mode("auto")
+
+
+@pytest.mark.parametrize("n,sweeps", [(4, 0), (10, 1), (14, 0), (14, 1)])
+def test_final_state_into_awkward_places(gpu, n, sweeps):
+    """The final circuit state over the fidelity reference and at an address
+    that is aligned to one amplitude only: as in a buffer of its own."""
+    from qmprs_amd import engine
+    b, layers = 2, 2
+    gates0, widths = _random_layers(n, b, layers, gpu, 5)
+    lu = torch.full((b,), layers, dtype=torch.int32, device=gpu)
+    for dtype, awkward in ((torch.complex128, "reference"), (torch.complex64, "address")):
+        target = _states(n, b, gpu, dtype, 6)
+        ref = target.to(torch.complex128).clone()
+        got = []
+        for place in ("own", awkward):
+            psi_ref = ref.clone()
+            if place == "reference":
+                out = psi_ref
+            elif place == "address":
+                out = torch.empty(b * 2 ** n + 1, dtype=dtype, device=gpu)[1:].view(b, 2 ** n)
+            else:
+                out = torch.empty_like(target)
+            fid = torch.zeros((b, sweeps + 1), dtype=torch.complex128, device=gpu)
+            ov = torch.zeros((b, max(sweeps, 1)), dtype=torch.float64, device=gpu)
+            gates = gates0.clone()
+            engine.sweep_noalloc(target, gates, widths, lu, sweeps, fid, ov if sweeps else None, psi_ref,
+                                 circuit_out=out)
+            torch.cuda.synchronize()
+            got.append((out.clone(), fid, gates))
+        for x, y in zip(*got):
+            assert torch.equal(x, y)
