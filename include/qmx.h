@@ -105,7 +105,10 @@ const char* qmx_last_error(const qmx_handle* h);
  * fourteen times faster and closer to an SVD), and the layers' 4 x 4
  * eigenproblems through one lane instead of a wave.  Both give the truncated
  * state to rounding; 1 keeps the exact rounding of the two-sided solver, which
- * the layers of a deep circuit amplify (see qmprs_amd/primitives/mps.py). */
+ * the layers of a deep circuit amplify (see qmprs_amd/primitives/mps.py).
+ * Whatever the option, a truncation whose cutoff is below 128 bond_dimension
+ * 2^-52 (the default 1e-10 never is) runs two-sided: the one-sided solver gives
+ * eigenvalues below 2^-52 of the trace as 0 and has no vectors for them. */
 #define QMX_OPT_TWO_SIDED_JACOBI 10
 int qmx_set_option(qmx_handle* h, int option, int value);
 

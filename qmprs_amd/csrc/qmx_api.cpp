@@ -576,6 +576,12 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
   const int nmax = L.nmax;
   const size_t nm2 = static_cast<size_t>(nmax) * nmax;
   const int kmax = std::min(chi, nmax);
+  // The one-sided solver has no vectors for what its factor leaves out, a
+  // weight of up to nmax eps (an amplitude of 1.5e-8 a column).  So it is taken
+  // where the cutoff leaves out 64 times that in any case (the default 1e-10
+  // does at every size); a smaller cutoff asks for directions that only the
+  // two-sided solver gives.
+  const bool one_sided = !h->two_sided && cutoff >= 64.0 * nmax * 2.220446049250313e-16;
   auto xbuf = [&](int i) { return ((i_first - i) % 2 == 0) ? L.xa : L.xb; };
   // forward chain: X_i = Y_i W_i
   for (int i = i_first; i >= 1; --i) {
@@ -587,7 +593,7 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
     launch_gram_reduce(L.part, nchunks, L.ncur, nmax, L.a, nm2, batch, st);
     // sweep limits of the eigensolvers; QMX_OPT_JACOBI_SWEEP_CAP lowers them
     auto cap = [&](int limit) { return h->jacobi_sweep_cap > 0 ? std::min(limit, h->jacobi_sweep_cap) : limit; };
-    if (!h->two_sided && L.jdiag) {   // above 128 columns
+    if (one_sided && L.jdiag) {   // above 128 columns
       std::vector<int> conv(batch);
       if (launch_osj_wide(L.a, L.v, nm2, L.ncur, nmax, rows, batch, spectra ? 0 : chi, L.jrank, L.jdiag, conv.data(),
                           cap(kJacobiBlockSweeps), L.error, st) != 0)
@@ -597,9 +603,9 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
       if (launch_jacobi_block(L.a, L.v, nm2, L.ncur, nmax, batch, L.jblock, conv.data(), cap(kJacobiBlockSweeps),
                               L.error, st) != 0)
         return fail(h, QMX_ERR_HIP, "block Jacobi");
-    } else if (h->two_sided && L.jlog && jacobi_lds_setup(nmax) == hipSuccess) {
+    } else if (!one_sided && L.jlog && jacobi_lds_setup(nmax) == hipSuccess) {
       launch_jacobi_lds(L.a, L.v, nm2, L.ncur, nmax, batch, L.jlog, L.jstate, cap(kJacobiSweeps), L.error, st);
-    } else if (!h->two_sided && L.jrank && !L.jdiag) {
+    } else if (one_sided && L.jrank && !L.jdiag) {
       // (the spectra of bonds that are not truncated are wanted too if any are)
       if (launch_osj(L.a, L.v, nm2, L.ncur, nmax, batch, spectra ? 0 : chi, L.jrank, cap(kJacobiSweeps), L.error,
                      st) != 0)
@@ -608,7 +614,7 @@ int run_chi(qmx_handle* h, int n, int batch, int chi, double cutoff, const void*
       launch_jacobi(L.a, L.v, nm2, L.ncur, nmax, batch, cap(kJacobiGlobalSweeps), L.error, st);
     }
     double2* wi = L.w + static_cast<size_t>(i) * batch * nm2;
-    launch_select(L.a, L.v, wi, nm2, L.ncur, nmax, chi, cutoff, L.kk + i, n + 1,
+    launch_select(L.a, L.v, wi, nm2, L.ncur, nmax, chi, one_sided, cutoff, L.kk + i, n + 1,
                   spectra ? spectra + static_cast<size_t>(i) * 2 * chi : nullptr,
                   static_cast<size_t>(n + 1) * 2 * chi, batch, st);
     GemmDims d{i, L.nn + i, L.kk + i, n + 1, nmax, kmax, nmax};

@@ -339,8 +339,8 @@ int launch_osj_wide(double2* a, double2* v, size_t stride, const int* ncols_dev,
 void launch_jacobi(double2* a, double2* v, size_t stride, const int* ncols_dev, int ncols_max,
                    int batch, int max_sweeps, int* error, hipStream_t);
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,
-                   const int* ncols_dev, int ncols_max, int chi, double cutoff, int* k_out,
-                   int kstride, double* spectra, size_t spec_stride, int batch, hipStream_t);
+                   const int* ncols_dev, int ncols_max, int chi, bool keep_as_is, double cutoff,
+                   int* k_out, int kstride, double* spectra, size_t spec_stride, int batch, hipStream_t);
 void launch_chain_dims(int* nn, int* ncur, const int* kk, int n, int step, int first_cols,
                        int batch, hipStream_t);
 void launch_goal_check(const double2* dot, int dot_stride, const double* goal, int* skip,

@@ -548,7 +548,9 @@ __global__ void jacobi_lds_check_kernel(const int* state, int batch, int* error)
 // the rotations converge (8 to 10 sweeps on the chain's matrices, the last of
 // them only checking), and the columns that a rank-deficient Gram matrix does
 // not have (fewer rows than columns left of the chain's centre) are never
-// touched.  Columns dropped at eps * trace get eigenvalue 0 and a zero vector.
+// touched.  Columns dropped at eps * trace get eigenvalue 0 and a zero vector:
+// the caller takes this solver where its cutoff drops them too, and the identity
+// in the place of the vectors of a matrix that is not truncated.
 constexpr double kEps = 2.220446049250313e-16;
 // columns p, q are orthogonal when |p^H q| <= kOsjTol |p| |q|: the rounding of
 // a 128-term product is about sqrt(128) eps
@@ -1455,12 +1457,14 @@ __global__ __launch_bounds__(256) void bj_store_kernel(const double2* cur_all, c
 // Sort eigenvalues (diag of A) in decreasing order, pick k (rsum2 cutoff and
 // max bond chi; k = n when n <= chi), and write the sorted eigenvectors into
 // the columns of w (same layout as v).  k_out[b] = k; spectra (optional).
+// keep_as_is: w is the identity when n <= chi (the one-sided solver's vectors
+// of such a matrix are not a basis where its factor has no columns).
 // Every block of a state sorts for itself and copies its rows of w; the first
 // one also picks k (600 columns: 36 us, in one block 192).
 constexpr int kSelectRows = 16;
 __global__ __launch_bounds__(512) void select_kernel(const double2* a_all, const double2* v_all,
                                                      double2* w_all, size_t stride,
-                                                     const int* ncols_dev, int ld, int chi,
+                                                     const int* ncols_dev, int ld, int chi, bool keep_as_is,
                                                      double cutoff, int* k_out, int kstride,
                                                      double* spectra, size_t spec_stride) {
   __shared__ double val[2 * kJacobiMaxPairs], lam[2 * kJacobiMaxPairs];
@@ -1516,7 +1520,8 @@ __global__ __launch_bounds__(512) void select_kernel(const double2* a_all, const
       for (int j = threadIdx.x; j < n; j += blockDim.x) spectra[(size_t)b * spec_stride + j] = lam[j];
   }
   for (int i = row0; i < min(row0 + kSelectRows, n); ++i)
-    for (int c = threadIdx.x; c < n; c += blockDim.x) w[(size_t)i * ld + c] = v[(size_t)i * ld + perm[c]];
+    for (int c = threadIdx.x; c < n; c += blockDim.x)
+      w[(size_t)i * ld + c] = keep_as_is && n <= chi ? make_double2(i == c ? 1.0 : 0.0, 0.0) : v[(size_t)i * ld + perm[c]];
 }
 
 // ------------------------------------------------------------------ gemm ----
@@ -1800,10 +1805,11 @@ int launch_osj_wide(double2* a, double2* v, size_t stride, const int* ncols_dev,
 }
 
 void launch_select(const double2* a, const double2* v, double2* w, size_t stride,
-                   const int* ncols_dev, int ncols_max, int chi, double cutoff, int* k_out,
-                   int kstride, double* spectra, size_t spec_stride, int batch, hipStream_t st) {
-  hipLaunchKernelGGL(select_kernel, dim3((ncols_max + kSelectRows - 1) / kSelectRows, batch), dim3(std::min(512, (ncols_max + 63) / 64 * 64)), 0, st, a, v, w, stride, ncols_dev,
-                     ncols_max, chi, cutoff, k_out, kstride, spectra, spec_stride);
+                   const int* ncols_dev, int ncols_max, int chi, bool keep_as_is, double cutoff,
+                   int* k_out, int kstride, double* spectra, size_t spec_stride, int batch, hipStream_t st) {
+  hipLaunchKernelGGL(select_kernel, dim3((ncols_max + kSelectRows - 1) / kSelectRows, batch),
+                     dim3(std::min(512, (ncols_max + 63) / 64 * 64)), 0, st, a, v, w, stride, ncols_dev, ncols_max, chi,
+                     keep_as_is, cutoff, k_out, kstride, spectra, spec_stride);
 }
 
 // nn[b][step] = ncur[b] = first_cols (> 0) or 2 * kk[b][step + 1]
