@@ -225,7 +225,8 @@ int qmx_extract_layers(qmx_handle* h, int num_qubits, int batch, int num_layers,
  *               one-block sweeps of small states it synchronises
  *               once per sweep); sweeps_done (device or NULL, B ints) then
  *               receives the number of sweeps each state ran.
- *   circuit_out device or NULL, B x 2^N of storage_dtype: final C|0..0> */
+ *   circuit_out device or NULL, B x 2^N of storage_dtype: final C|0..0>; may
+ *               lie over target or psi_ref (written when both have been read) */
 size_t qmx_sweep_workspace(int num_qubits, int batch, int storage_dtype);
 int qmx_sweep(qmx_handle* h, int num_qubits, int batch, int num_layers, const int* layers_used,
               int num_sweeps, const void* target, int storage_dtype, void* gates,

@@ -836,7 +836,7 @@ struct SweepJob {
   int* sweeps_done;
   S* circuit_out;
   // the final state is built in circuit_out itself: it is aligned as the kernels'
-  // own buffers are, and the reference, read afterwards, is somewhere else
+  // own buffers are, and what is still to be read is somewhere else
   bool out_direct = false;
   SweepLayout<S> L;
   hipStream_t st;
@@ -1096,12 +1096,16 @@ int run_sweep_jobs(qmx_handle* h, std::vector<SweepJob<S>>& jobs) {
     for (size_t j = 1; j < nj; ++j) QMX_CALL(stream_join(h, h->join_ev[j], jobs[j].st, s0));
     swt.stop(windowed ? (long long)wins.size() : (long long)kmax);
   }
-  // final circuit state and fidelity
-  for (auto& J : jobs) {
-    QMX_CALL(job_rebuild(h, J, nsweeps, true));
+  // final circuit state and fidelity; an output that may lie over the inputs is
+  // written when every job has read them
+  for (auto& J : jobs) QMX_CALL(job_rebuild(h, J, nsweeps, true));
+  if (nj > 1 && jobs[0].circuit_out && !(jobs[0].out_direct && jobs[1].out_direct)) {
+    QMX_CALL(stream_join(h, h->join_ev[0], jobs[0].st, jobs[1].st));
+    QMX_CALL(stream_join(h, h->join_ev[1], jobs[1].st, jobs[0].st));
+  }
+  for (auto& J : jobs)
     if (J.circuit_out && !J.out_direct)
       launch_scale_convert<S, S>(J.L.phi, J.circuit_out, n, J.batch, nullptr, J.st);
-  }
   QMX_LAUNCHED(h, "final circuit state");
   return QMX_OK;
 }
@@ -1116,6 +1120,16 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
                    double2* fidelity, double* overlap, const double* goal, int* sweeps_done,
                    S* circuit_out, Carver& c, hipStream_t st, int snap_first = -1,
                    double2* snapshots = nullptr) {
+  const size_t len = state_len(n);
+  // circuit_out over psi_ref or target (at target itself each state's output lies
+  // over its own input, which is read by then): to be written when all states'
+  // inputs have been read
+  const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+  const auto over = [&](const void* p, size_t amp) {
+    return p && circuit_out && at(circuit_out) < at(p) + batch * len * amp &&
+           at(p) < at(circuit_out) + batch * len * sizeof(S);
+  };
+  const bool shared = over(psi_ref, sizeof(double2)) || (circuit_out != target && over(target, sizeof(S)));
   // Small states are swept by one block each, in one launch: their sweeps are
   // chains of polar factors, and a launch per window or gate costs more than
   // its work (complex128, 4 layers, 4 sweeps: N=5 0.30 ms against 0.86 gate by
@@ -1150,7 +1164,7 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
     a.overlap = overlap;
     a.goal = goal;
     a.sweeps_done = sweeps_done;
-    a.circuit_out = circuit_out;
+    a.circuit_out = shared ? sweep_layout<S>(c, n, batch).phi : circuit_out;
     a.omega_m1 = (h->relax_milli - 1000) * 1e-3;
     if (snapshots && snap_first >= 0) {
       a.snap_first = snap_first;
@@ -1159,11 +1173,12 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
     }
     if (fidelity) launch_fill_int(reinterpret_cast<int*>(fidelity), 0, batch * (nsweeps + 1) * 4, st);
     QMX_HIP(h, launch_lds_sweep<S>(a, batch, st));
+    if (shared) launch_scale_convert<S, S>(a.circuit_out, circuit_out, n, batch, nullptr, st);
+    QMX_LAUNCHED(h, "one-block sweep");
     swt.stop(1);
     return QMX_OK;
   }
   const bool split = h->split_sweeps && batch >= 2 && sweep_windowed(h, n);
-  const size_t len = state_len(n);
   auto job = [&](int b0, int nb, hipStream_t js) {
     SweepJob<S> J{};
     J.n = n;
@@ -1180,10 +1195,7 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
     J.goal = goal ? goal + b0 : nullptr;
     J.sweeps_done = sweeps_done ? sweeps_done + b0 : nullptr;
     J.circuit_out = circuit_out ? circuit_out + (size_t)b0 * len : nullptr;
-    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
-    const bool apart = !psi_ref || at(circuit_out + (size_t)batch * len) <= at(psi_ref) ||
-                       at(psi_ref + (size_t)batch * len) <= at(circuit_out);
-    J.out_direct = circuit_out && apart && at(J.circuit_out) % 16 == 0;
+    J.out_direct = circuit_out && !shared && at(J.circuit_out) % 16 == 0;
     if (snapshots && snap_first >= 0) {
       J.snap_first = snap_first;
       J.snaps = snapshots + (size_t)b0 * lmax * n * 16;
