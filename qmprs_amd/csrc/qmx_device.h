@@ -357,13 +357,18 @@ struct Mat4 {
   double v, o;
 };
 QMX_DEV Mat4 mat4(double v) { return {v, dpp<kDppRow3>(v)}; }   // row_ror:4: the block before
-// M^T B, or M^H B with CONJ
+// C + M^T B, or C + M^H B with CONJ
 template <bool CONJ>
-QMX_DEV double mat4_tmul(Mat4 m, Mat4 b, bool even) {
+QMX_DEV double mat4_tmul(Mat4 m, Mat4 b, bool even, double c = 0.0) {
   const double re = even ? m.v : m.o;
   const double im = CONJ ? (even ? m.o : -m.v) : (even ? -m.o : m.v);
-  const double d = __builtin_amdgcn_mfma_f64_4x4x4f64(re, b.v, 0.0, 0, 0, 0);
+  const double d = __builtin_amdgcn_mfma_f64_4x4x4f64(re, b.v, c, 0, 0, 0);
   return __builtin_amdgcn_mfma_f64_4x4x4f64(im, b.o, d, 0, 0, 0);
+}
+// C + M^T B with the sums of mat4_tmul<false>(b, m): the same bits, transposed
+QMX_DEV double mat4_tmul_swapped(Mat4 m, Mat4 b, bool even, double c = 0.0) {
+  const double d = __builtin_amdgcn_mfma_f64_4x4x4f64(m.v, even ? b.v : b.o, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(even ? -m.o : m.o, even ? b.o : b.v, d, 0, 0, 0);
 }
 
 QMX_DEV bool polar4_rank2(double2& x, int l, const double2* es, int h, double fro, double* nuc);
@@ -379,13 +384,23 @@ QMX_DEV bool polar4_rank2(double2& x, int l, const double2* es, int h, double fr
 // quadratically: once |X^H X - 1| <= 3e-9 in every entry the next step is exact
 // to rounding.  On the sweeps' environments (condition numbers 5 to 90 at the
 // median, 1e3 to 1e4 at the 90th percentile) that takes 8 to 14 steps on
-// average.  The transpose of X is carried along as the left operand.
-// Bound by the latency of the two products, about 300 cycles per step: 3700
-// cycles for a Gaussian 4 x 4 matrix, 4900 at condition number 1000.  The scaled
-// Newton iteration took 24000 and 27000 with its pivoted inverse by ds_bpermute,
-// 6700 and 10500 with an inverse from cofactors by DPP moves.  Error against
-// 80-bit arithmetic: within 1.6 times that of the Newton iteration (both a few
-// 1e-16 times the condition number over 5).
+// average.  The transpose of X is carried along as the left operand, with the
+// same sums and so the same rounding.
+// The steps' roundings turn X away from E's factor, by eps over the singular
+// values of the time: the first step has the matrix as it is (its norm is in
+// the step's coefficients), and the last X is turned back, X <- X + X W: with
+// X^H E = (1 + W) H, H Hermitian, X^H E - E^H X is H W + W H, of which 0.9 over
+// E's norm is taken for W (all of it for equal singular values, less for the
+// small ones, whose share the early steps decide).
+// Bound by the latency of the two products, about 300 cycles per step: 4600
+// cycles for a Gaussian 4 x 4 matrix, 6400 at condition number 1000 (4100 and
+// 5800 without the exact start and the turn back).  The scaled Newton iteration
+// took 24000 and 27000 with its pivoted inverse by ds_bpermute.  Error against
+// 80-bit arithmetic, rms of the factor, and the Newton iteration's: Gaussian
+// 4.4e-16 and 5.3e-16, unitary 2.3e-16 and 2.5e-16, condition numbers up to 10
+// 3.4e-16 and 3.5e-16, up to 1000 2.5e-15 and 2.9e-15, up to 1e5 1.27e-13 and
+// 1.29e-13 (without the exact start and the turn back 6.5e-16, 4.4e-16, 5.5e-16,
+// 3.5e-15 and 1.7e-13).
 // u: this lane's part of the factor in the split layout.  False after 34
 // unscaled steps (a condition number above about 1e6).
 QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane, Mat4& u, double2& x2, double& nuc2,
@@ -394,22 +409,25 @@ QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane
   const bool even = !(lane & 4);
   const double r = rsqrt_newton(fro);
   const double2 e = es[4 * i + j], t = es[4 * j + i];
-  Mat4 x = mat4(ldexp(even ? e.x : e.y, h) * r), xt = mat4(ldexp(even ? t.x : t.y, h) * r);
+  const Mat4 x0 = mat4(ldexp(even ? e.x : e.y, h));   // r x0 is the matrix to start from
+  Mat4 x = x0, xt = mat4(ldexp(even ? t.x : t.y, h));
   const double one = even && i == j ? 1.0 : 0.0;
-  auto step = [&](double a, double b, double y) {
-    const Mat4 p = mat4(fma(-b, y, a * one));
-    const double xn = mat4_tmul<false>(xt, p, even);
-    const double tn = mat4_tmul<false>(p, xt, even);
+  // X <- X P, or X + X P; and its transpose, bit for bit
+  auto times = [&](double pv, bool add) {
+    const Mat4 p = mat4(pv);
+    const double xn = mat4_tmul<false>(xt, p, even, add ? x.v : 0.0);
+    const double tn = mat4_tmul_swapped(p, xt, even, add ? xt.v : 0.0);
     x = mat4(xn);
     xt = mat4(tn);
   };
   auto gram = [&]() { return mat4_tmul<true>(x, x, even); };
-  step(2.5324497354750872, 2.406128014703171, gram());   // l = 0.05
-  step(2.430892812235437, 2.128107957418897, gram());    // 0.1263
-  step(2.200129819325986, 1.5777607537549168, gram());   // 0.3028
-  step(1.832672820412407, 0.9119080391587333, gram());   // 0.6224
-  step(1.5614350757473685, 0.5639856062462636, gram());  // 0.9208
-  step(1.5019149323066294, 0.5019173779907503, gram());  // 0.9974
+  auto scaled = [&](double a, double b) { times(fma(-b, gram(), a * one), false); };
+  scaled(2.5324497354750872 * r, 2.406128014703171 * (r * r * r));   // l = 0.05
+  scaled(2.430892812235437, 2.128107957418897);    // 0.1263
+  scaled(2.200129819325986, 1.5777607537549168);   // 0.3028
+  scaled(1.832672820412407, 0.9119080391587333);   // 0.6224
+  scaled(1.5614350757473685, 0.5639856062462636);  // 0.9208
+  scaled(1.5019149323066294, 0.5019173779907503);  // 0.9974
   for (int it = 0; it < 34; ++it) {
     const double y = gram();
     if (it == 0) {
@@ -422,8 +440,9 @@ QMX_DEV bool polar4_newton_schulz(const double2* es, int h, double fro, int lane
       }
     }
     const bool last = __all(fabs(y - one) <= 3e-9);
-    step(1.5, 0.5, y);
+    times(0.5 * (one - y), true);
     if (last) {
+      times(0.9 * r * (mat4_tmul<true>(x, x0, even) - mat4_tmul<true>(x0, x, even)), true);
       u = x;
       return true;
     }

@@ -1,0 +1,100 @@
+"""Rounding of the gate update's polar factor, apart from everything before it.
+
+Four sites and two layers of gates with entries 0, 1 and 1/2, after which the
+environment of the first two-site gate of the sweep is the conjugate of the
+target over two, a 4 x 4 matrix, without rounding.  The one-site gate before it
+has the partial trace of that matrix as its environment; targets lie on a grid
+of 2^-20 and have a partial trace of one, so that this gate stays the identity."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+N, LAYERS = 4, 2
+COUNT = 3000
+
+
+def _circuit():
+    """sum_ab |a b b a> / 2, and identities on the last two sites."""
+    gates = np.zeros((LAYERS, N, 4, 4), dtype=np.complex128)
+    h = np.array([[1.0, 1.0], [1.0, -1.0]])
+    cnot = np.eye(4)[[0, 1, 3, 2]]
+    swap = np.eye(4)[[0, 2, 1, 3]]
+    gates[1, 0], gates[1, 1], gates[1, 2] = np.kron(h, h) / 2, cnot, swap      # acts first
+    gates[0, 0], gates[0, 1], gates[0, 2] = swap, cnot, np.eye(4)
+    gates[:, 3, :2, :2] = np.eye(2)
+    widths = np.full((LAYERS, N), 2, dtype=np.int32)
+    widths[:, 3] = 1
+    return gates, widths
+
+
+def _environments(kind):
+    """(COUNT, 4, 4): entry (o, i) over sites 2, 3, partial trace over site 2 one."""
+    rng = np.random.default_rng(5)
+    g = lambda: rng.standard_normal((COUNT, 4, 4)) + 1j * rng.standard_normal((COUNT, 4, 4))
+    if kind == "gauss":
+        e = g()
+    else:
+        u, v = np.linalg.qr(g())[0], np.linalg.qr(g())[0]
+        e = (u * (1 / kind) ** rng.random((COUNT, 1, 4))) @ v
+    t = np.trace(e.reshape(COUNT, 2, 2, 2, 2), axis1=1, axis2=3)
+    # a factor on the right that makes the partial trace the identity, near enough
+    # for the grid's correction to be small
+    e = e @ np.kron(np.eye(2), np.linalg.inv(t))
+    grid = lambda a: np.round(a * 2.0 ** 20) / 2.0 ** 20
+    e = grid(e)
+    t = np.trace(e.reshape(COUNT, 2, 2, 2, 2), axis1=1, axis2=3)
+    e[:, 2:, 2:] += np.eye(2) - t
+    return e
+
+
+def _polar_long(e):
+    """The unitary polar factors in extended precision (Newton's iteration)."""
+    x = e.astype(np.clongdouble)
+    for it in range(40):
+        a = np.concatenate([x, np.broadcast_to(np.eye(4, dtype=np.clongdouble), x.shape)], axis=2).copy()
+        rows = np.arange(len(x))
+        for k in range(4):
+            p = np.argmax(np.abs(a[:, k:, k]), axis=1) + k
+            a[rows, k], a[rows, p] = a[rows, p].copy(), a[rows, k].copy()
+            a[:, k] /= a[:, k, k][:, None]
+            for i in range(4):
+                if i != k:
+                    a[:, i] -= a[:, i, k][:, None] * a[:, k]
+        inv = np.conj(np.swapaxes(a[:, :, 4:], 1, 2))
+        z = np.sqrt(np.sqrt((np.abs(inv) ** 2).sum((1, 2)) / (np.abs(x) ** 2).sum((1, 2)))) if it < 20 else np.ones(len(x))
+        x = (z[:, None, None] * x + inv / z[:, None, None]) / 2
+    return x
+
+
+# Root mean square of |G' - conj(polar(E))|_F that a scaled Newton iteration with
+# pivoted inverses has on these matrices (measured), the rounding to keep to.
+NEWTON = {"gauss": 6.9e-16, 1.0: 4.4e-16, 10.0: 5.6e-16, 100.0: 2.33e-15, 1000.0: 6.1e-15}
+
+
+@pytest.mark.parametrize("mode", ["auto", "step"])
+@pytest.mark.parametrize("kind", NEWTON)
+def test_polar_factor_rounding(gpu, kind, mode):
+    from qmprs_amd import _lib, engine
+    e = _environments(kind)
+    e = e[np.linalg.cond(e) < 1e5]      # beyond it another path decides
+    g, w = _circuit()
+    b = len(e)
+    # amplitude of |s0 s1 s2 s3>: E[(s2 s3), (s1 s0)] = conj(T) / 2
+    target = 2 * np.conj(e).reshape(b, 2, 2, 2, 2).transpose(0, 4, 3, 1, 2).reshape(b, 16)
+    gates = torch.from_numpy(np.broadcast_to(g, (b,) + g.shape).copy()).to(gpu)
+    widths = torch.from_numpy(np.broadcast_to(w, (b,) + w.shape).copy()).to(gpu)
+    used = torch.full((b,), LAYERS, dtype=torch.int32, device=gpu)
+    _lib.set_sweep_mode(mode)
+    try:
+        engine.sweep(torch.from_numpy(np.ascontiguousarray(target)).to(gpu), gates, widths, used, 1)
+    finally:
+        _lib.set_sweep_mode("auto")
+    out = gates.cpu().numpy()
+    assert (out[:, 0, 3, :2, :2] == np.eye(2)).all()
+    err = np.sqrt((np.abs(out[:, 0, 2] - np.conj(_polar_long(e))) ** 2).sum((1, 2)).astype(float))
+    rms = float(np.sqrt((err ** 2).mean()))
+    print(f"{kind}: rms {rms:.2e}, largest {err.max():.2e}, Newton {NEWTON[kind]:.2e}")
+    assert rms <= NEWTON[kind]
