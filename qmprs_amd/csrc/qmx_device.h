@@ -481,6 +481,12 @@ QMX_DEV double row_total(double v) {
   v += dpp<kDppSwap>(v);
   return v + dpp<kDppCol2>(v);
 }
+// x - q (q^H x), x and q by the lanes' rows i: a second pass for an x that was
+// e_k - sum q conj(q_k), whose rounding grows with what was taken off
+QMX_DEV double2 without(double2 x, double2 q) {
+  const double2 t = cmulc(q, x);
+  return csub(x, cmul(q, make_double2(col_total(t.x), col_total(t.y))));
+}
 // Two unit vectors beside q_0, q_1 (rows in the lanes' i), as polar4_jacobi
 // completes: residuals of the first e_k, in order, whose squared norm is above 1/4
 QMX_DEV bool complete_two(int i, double2 q0, double2 q1, double2& q2, double2& q3) {
@@ -492,12 +498,14 @@ QMX_DEV bool complete_two(int i, double2 q0, double2 q1, double2& q2, double2& q
   auto row = [&](double2 v, int k) { return make_double2(lane_value(v.x, 4 * k), lane_value(v.y, 4 * k)); };
   double2 t = cadd(cmulc(row(q0, e2), q0), cmulc(row(q1, e2), q1));
   q2 = make_double2((i == e2 ? 1.0 : 0.0) - t.x, -t.y);
+  q2 = without(without(q2, q0), q1);
   q2 = cscale(q2, rsqrt_newton(col_total(cabs2(q2))));
   const unsigned m3 = (unsigned)__ballot(i > e2 && res - cabs2(q2) > 0.25) & 0x1111u;
   if (!m3) return false;
   const int e3 = __builtin_amdgcn_readfirstlane((__ffs(m3) - 1) >> 2);
   t = cadd(cadd(cmulc(row(q0, e3), q0), cmulc(row(q1, e3), q1)), cmulc(row(q2, e3), q2));
   q3 = make_double2((i == e3 ? 1.0 : 0.0) - t.x, -t.y);
+  q3 = without(without(without(q3, q0), q1), q2);
   q3 = cscale(q3, rsqrt_newton(col_total(cabs2(q3))));
   return true;
 }
@@ -507,11 +515,10 @@ QMX_DEV bool complete_two(int i, double2 q0, double2 q1, double2& q2, double2& q
 // 1e-13 of the largest).  With Q R = the two columns left (Gram-Schmidt, two
 // passes), their part of the factor is Q polar(R); the zero columns z_1 < z_2,
 // whose right singular vectors are e_{z_1}, e_{z_2}, take the rule's left
-// completion, the first unit vectors with a residual above 1/2 (which one
-// pass of Gram-Schmidt then gives to rounding).  Lane 4 i + j of 16 works on
+// completion, the first unit vectors with a residual above 1/2.  Lane 4 i + j of 16 works on
 // row i and on column j of (live, live, zero, zero).  zero: the zero columns
 // (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry (i, j) of
-// the factor.  False where the Jacobi path decides (30600 cycles); 2700
+// the factor.  False where the Jacobi path decides (30600 cycles); 2900
 // cycles, against 5300 to 7500 with the whole problem in every lane.
 QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, unsigned zero, double fro, double* nuc) {
   const unsigned live = ~zero & 15u;
@@ -569,7 +576,9 @@ QMX_DEV bool polar4_one_column(double2& x, int l, const double2* es, int h, unsi
 #pragma unroll
     for (int b = 0; b < k; ++b)
       t = cadd(t, cmulc(make_double2(lane_value(q[b].x, 4 * ek), lane_value(q[b].y, 4 * ek)), q[b]));
-    const double2 w = make_double2((i == ek ? 1.0 : 0.0) - t.x, -t.y);
+    double2 w = make_double2((i == ek ? 1.0 : 0.0) - t.x, -t.y);
+#pragma unroll
+    for (int b = 0; b < k; ++b) w = without(w, q[b]);
     q[k] = cscale(w, rsqrt_newton(col_total(cabs2(w))));
     res -= cabs2(q[k]);
     from = ek + 1;
@@ -591,7 +600,7 @@ QMX_DEV double2 pick4(int k, double2 a, double2 b, double2 c, double2 d) {
 // column-pivoted Gram-Schmidt and again on the rows, and the factor is
 // Q polar(L) W^H with both sides completed as polar4_jacobi completes them.
 // Taken when nothing above 3e-14 of the norm is left beside Q (the Jacobi path
-// drops singular values below 1e-13).  7900 cycles with the six steps that find
+// drops singular values below 1e-13).  9500 cycles with the six steps that find
 // it out; it is met once a sweep, and the Jacobi path took 64000 there.
 QMX_DEV bool polar4_rank2(double2& x, int l, const double2* es, int h, double fro, double* nuc) {
   const int i = l >> 2, j = l & 3;
@@ -698,6 +707,9 @@ QMX_DEV bool polar4_wave(int d, const double2* es, double2* out, double sgn, int
       const double2 t0 = cmulc(g, a), t1 = cmulc(g, c);
       b = make_double2((first ? 1.0 : 0.0) - t0.x, -t0.y);
       f = make_double2((first ? 0.0 : 1.0) - t1.x, -t1.y);
+      const double2 again = cadd(cmulc(a, b), cmulc(c, f));
+      b = csub(b, cmul(a, again));
+      f = csub(f, cmul(c, again));
       const double q = rsqrt_newton(cabs2(b) + cabs2(f));
       b = cscale(b, q);
       f = cscale(f, q);

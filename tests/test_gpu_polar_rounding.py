@@ -98,3 +98,82 @@ def test_polar_factor_rounding(gpu, kind, mode):
     rms = float(np.sqrt((err ** 2).mean()))
     print(f"{kind}: rms {rms:.2e}, largest {err.max():.2e}, Newton {NEWTON[kind]:.2e}")
     assert rms <= NEWTON[kind]
+
+
+def _column_case(kind):
+    """(gates, widths, targets, environments, their zero columns) of one layer
+    whose sites are still in |0>: the two-site gate of two sites, whose environment
+    has one column, and the second one of three sites, whose environment has two."""
+    rng = np.random.default_rng(6)
+    n = 2 if kind == "one column" else 3
+    gates = np.zeros((1, n, 4, 4), dtype=np.complex128)
+    gates[0, n - 2] = np.eye(4)
+    gates[0, n - 1, :2, :2] = np.eye(2)
+    h = np.ones((1, 1))                                   # the circuit: sum h[r][a] |r a 0>
+    if n == 3:
+        hadamard = np.array([[1.0, 1.0], [1.0, -1.0]])
+        gates[0, 0] = np.diag([1, 1, 1, -1]) @ np.kron(hadamard, hadamard) / 2
+        h = hadamard / 2
+    widths = np.full((1, n), 2, dtype=np.int32)
+    widths[0, n - 1] = 1
+    t = rng.standard_normal((COUNT, len(h), 2, 2)) + 1j * rng.standard_normal((COUNT, len(h), 2, 2))
+    t = np.round(t * 2.0 ** 20) / 2.0 ** 20
+    # the last site's environment is one column: (1, 0), so that its gate stays
+    t[:, 0, 0] += (np.array([1.0, 0.0]) - np.einsum("brac,ra->bc", t[:, :, :h.shape[1]], h)) / h[0, 0]
+    e = np.zeros((COUNT, 4, 4), dtype=np.complex128)
+    e[:, :, :2 * h.shape[1]:2] = np.einsum("brac,ri->baci", np.conj(t), h).reshape(COUNT, 4, h.shape[1])
+    return gates, widths, t.reshape(COUNT, -1), e, [1, 2, 3] if n == 2 else [1, 3]
+
+
+def _completed_long(e, zero):
+    """Polar factors whose zero columns are completed by the first unit vectors
+    with a residual above 1/2 against the columns so far, in extended precision."""
+    m, q = e.astype(np.clongdouble), []
+
+    def residual(v):
+        for _ in range(2):
+            for b in q:
+                v = v - b * (np.conj(b) * v).sum(1)[:, None]
+        return v, np.sqrt((np.abs(v) ** 2).sum(1))
+
+    for c in range(4):
+        if c not in zero:
+            v, size = residual(m[:, :, c])
+            q.append(v / size[:, None])
+    start = np.zeros(len(e), dtype=int)
+    for c in zero:
+        done = np.zeros(len(e), dtype=bool)
+        for k in range(4):
+            v, size = residual(np.tile(np.eye(4, dtype=np.clongdouble)[k], (len(e), 1)))
+            take = ~done & (k >= start) & (size > 0.5)
+            m[take, :, c] = v[take] / size[take, None]
+            start[take] = k + 1
+            done |= take
+        q.append(m[:, :, c].copy())
+    return _polar_long(m)
+
+
+# the same for the one-sided Jacobi with two passes of Gram-Schmidt for the completion
+TWO_PASSES = {"one column": 1.62e-16, "two columns": 2.82e-16}
+
+
+@pytest.mark.parametrize("mode", ["auto", "step"])
+@pytest.mark.parametrize("kind", TWO_PASSES)
+def test_completed_factor_rounding(gpu, kind, mode):
+    from qmprs_amd import _lib, engine
+    g, w, target, e, zero = _column_case(kind)
+    n, b = g.shape[1], len(target)
+    gates = torch.from_numpy(np.broadcast_to(g, (b,) + g.shape).copy()).to(gpu)
+    widths = torch.from_numpy(np.broadcast_to(w, (b,) + w.shape).copy()).to(gpu)
+    used = torch.ones(b, dtype=torch.int32, device=gpu)
+    _lib.set_sweep_mode(mode)
+    try:
+        engine.sweep(torch.from_numpy(target).to(gpu), gates, widths, used, 1)
+    finally:
+        _lib.set_sweep_mode("auto")
+    out = gates.cpu().numpy()
+    assert (out[:, 0, n - 1, :2, :2] == np.eye(2)).all()
+    err = np.sqrt((np.abs(out[:, 0, n - 2] - np.conj(_completed_long(e, zero))) ** 2).sum((1, 2)).astype(float))
+    rms = float(np.sqrt((err ** 2).mean()))
+    print(f"{kind}: rms {rms:.2e}, largest {err.max():.2e}, two passes {TWO_PASSES[kind]:.2e}")
+    assert rms <= TWO_PASSES[kind]
