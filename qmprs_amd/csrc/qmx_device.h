@@ -808,13 +808,20 @@ QMX_DEV void polar4_jacobi(int d, const double2* e, double2* out, double sgn, in
           const double dd = be - al, w = fma(4.0, ag2, dd * dd);
           double f = 2.0 * rcp_newton(fma(w, rsqrt_newton(w), fabs(dd)));
           f = dd >= 0.0 ? f : -f;
-          const double2 te = cscale(g, f), tm = make_double2(-te.x, te.y);   // te, -conj(te)
+          double2 te = cscale(g, f);
           const double c = rsqrt_newton(1.0 + cabs2(te));
+          te = cscale(te, c);
+          const double2 tm = make_double2(-te.x, te.y);   // c te, -c conj(te)
+          // (the larger term last: one rounding at its size)
+          auto turn = [&](double2 t, double2 y, double2 x) {
+            const double2 w = cmul(t, y);
+            return make_double2(fma(c, x.x, w.x), fma(c, x.y, w.y));
+          };
           const double2 x = a[p], y = a[q], vx = v[p], vy = v[q];
-          a[p] = cscale(cfma(tm, y, x), c);
-          a[q] = cscale(cfma(te, x, y), c);
-          v[p] = cscale(cfma(tm, vy, vx), c);
-          v[q] = cscale(cfma(te, vx, vy), c);
+          a[p] = turn(tm, y, x);
+          a[q] = turn(te, x, y);
+          v[p] = turn(tm, vy, vx);
+          v[q] = turn(te, vx, vy);
         }
       }
     if (!rotated) break;

@@ -34,8 +34,11 @@ def _environments(kind):
     """(COUNT, 4, 4): entry (o, i) over sites 2, 3, partial trace over site 2 one."""
     rng = np.random.default_rng(5)
     g = lambda: rng.standard_normal((COUNT, 4, 4)) + 1j * rng.standard_normal((COUNT, 4, 4))
+    bits = 20
     if kind == "gauss":
         e = g()
+    elif kind == "rank 3":      # but for the grid
+        e, bits = g()[:, :, :3] @ g()[:, :3], 32
     else:
         u, v = np.linalg.qr(g())[0], np.linalg.qr(g())[0]
         e = (u * (1 / kind) ** rng.random((COUNT, 1, 4))) @ v
@@ -43,8 +46,7 @@ def _environments(kind):
     # a factor on the right that makes the partial trace the identity, near enough
     # for the grid's correction to be small
     e = e @ np.kron(np.eye(2), np.linalg.inv(t))
-    grid = lambda a: np.round(a * 2.0 ** 20) / 2.0 ** 20
-    e = grid(e)
+    e = np.round(e * 2.0 ** bits) / 2.0 ** bits
     t = np.trace(e.reshape(COUNT, 2, 2, 2, 2), axis1=1, axis2=3)
     e[:, 2:, 2:] += np.eye(2) - t
     return e
@@ -74,29 +76,39 @@ def _polar_long(e):
 NEWTON = {"gauss": 6.9e-16, 1.0: 4.4e-16, 10.0: 5.6e-16, 100.0: 2.33e-15, 1000.0: 6.1e-15}
 
 
+def _updated(gpu, mode, gates, widths, target):
+    """The gates after one sweep of every target from the same circuit."""
+    from qmprs_amd import _lib, engine
+    b = len(target)
+    out = torch.from_numpy(np.broadcast_to(gates, (b,) + gates.shape).copy()).to(gpu)
+    w = torch.from_numpy(np.broadcast_to(widths, (b,) + widths.shape).copy()).to(gpu)
+    used = torch.full((b,), len(gates), dtype=torch.int32, device=gpu)
+    _lib.set_sweep_mode(mode)
+    try:
+        engine.sweep(torch.from_numpy(np.ascontiguousarray(target)).to(gpu), out, w, used, 1)
+    finally:
+        _lib.set_sweep_mode("auto")
+    out = out.cpu().numpy()
+    assert (out[:, 0, -1, :2, :2] == np.eye(2)).all()     # the one-site gate before
+    return out[:, 0, -2]
+
+
+def _target(e):
+    # amplitude of |s0 s1 s2 s3>: E[(s2 s3), (s1 s0)] = conj(T) / 2
+    return 2 * np.conj(e).reshape(-1, 2, 2, 2, 2).transpose(0, 4, 3, 1, 2).reshape(-1, 16)
+
+
+def _rms(a):
+    return float(np.sqrt((np.abs(a) ** 2).sum((1, 2)).mean()))
+
+
 @pytest.mark.parametrize("mode", ["auto", "step"])
 @pytest.mark.parametrize("kind", NEWTON)
 def test_polar_factor_rounding(gpu, kind, mode):
-    from qmprs_amd import _lib, engine
     e = _environments(kind)
     e = e[np.linalg.cond(e) < 1e5]      # beyond it another path decides
-    g, w = _circuit()
-    b = len(e)
-    # amplitude of |s0 s1 s2 s3>: E[(s2 s3), (s1 s0)] = conj(T) / 2
-    target = 2 * np.conj(e).reshape(b, 2, 2, 2, 2).transpose(0, 4, 3, 1, 2).reshape(b, 16)
-    gates = torch.from_numpy(np.broadcast_to(g, (b,) + g.shape).copy()).to(gpu)
-    widths = torch.from_numpy(np.broadcast_to(w, (b,) + w.shape).copy()).to(gpu)
-    used = torch.full((b,), LAYERS, dtype=torch.int32, device=gpu)
-    _lib.set_sweep_mode(mode)
-    try:
-        engine.sweep(torch.from_numpy(np.ascontiguousarray(target)).to(gpu), gates, widths, used, 1)
-    finally:
-        _lib.set_sweep_mode("auto")
-    out = gates.cpu().numpy()
-    assert (out[:, 0, 3, :2, :2] == np.eye(2)).all()
-    err = np.sqrt((np.abs(out[:, 0, 2] - np.conj(_polar_long(e))) ** 2).sum((1, 2)).astype(float))
-    rms = float(np.sqrt((err ** 2).mean()))
-    print(f"{kind}: rms {rms:.2e}, largest {err.max():.2e}, Newton {NEWTON[kind]:.2e}")
+    rms = _rms(_updated(gpu, mode, *_circuit(), _target(e)) - np.conj(_polar_long(e)))
+    print(f"{kind}: rms {rms:.2e}, Newton {NEWTON[kind]:.2e}")
     assert rms <= NEWTON[kind]
 
 
@@ -160,20 +172,23 @@ TWO_PASSES = {"one column": 1.62e-16, "two columns": 2.82e-16}
 @pytest.mark.parametrize("mode", ["auto", "step"])
 @pytest.mark.parametrize("kind", TWO_PASSES)
 def test_completed_factor_rounding(gpu, kind, mode):
-    from qmprs_amd import _lib, engine
     g, w, target, e, zero = _column_case(kind)
-    n, b = g.shape[1], len(target)
-    gates = torch.from_numpy(np.broadcast_to(g, (b,) + g.shape).copy()).to(gpu)
-    widths = torch.from_numpy(np.broadcast_to(w, (b,) + w.shape).copy()).to(gpu)
-    used = torch.ones(b, dtype=torch.int32, device=gpu)
-    _lib.set_sweep_mode(mode)
-    try:
-        engine.sweep(torch.from_numpy(target).to(gpu), gates, widths, used, 1)
-    finally:
-        _lib.set_sweep_mode("auto")
-    out = gates.cpu().numpy()
-    assert (out[:, 0, n - 1, :2, :2] == np.eye(2)).all()
-    err = np.sqrt((np.abs(out[:, 0, n - 2] - np.conj(_completed_long(e, zero))) ** 2).sum((1, 2)).astype(float))
-    rms = float(np.sqrt((err ** 2).mean()))
-    print(f"{kind}: rms {rms:.2e}, largest {err.max():.2e}, two passes {TWO_PASSES[kind]:.2e}")
+    rms = _rms(_updated(gpu, mode, g, w, target) - np.conj(_completed_long(e, zero)))
+    print(f"{kind}: rms {rms:.2e}, two passes {TWO_PASSES[kind]:.2e}")
     assert rms <= TWO_PASSES[kind]
+
+
+ONE_LANE = 3.45e-16
+
+
+@pytest.mark.parametrize("mode", ["auto", "step"])
+def test_jacobi_factor_rounding(gpu, mode):
+    """A smallest singular value near 1e-10, which the Jacobi path decides: what
+    U^H E lacks of being Hermitian, in units of E's norm, against that path in one
+    lane's registers (measured)."""
+    e = _environments("rank 3")
+    u = np.conj(_updated(gpu, mode, *_circuit(), _target(e))).astype(np.clongdouble)
+    h = np.conj(np.swapaxes(u, 1, 2)) @ e.astype(np.clongdouble)
+    rms = _rms((h - np.conj(np.swapaxes(h, 1, 2))) / np.linalg.norm(e, axis=(1, 2))[:, None, None])
+    print(f"rms {rms:.2e}")
+    assert rms <= ONE_LANE
