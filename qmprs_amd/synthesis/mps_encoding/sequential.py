@@ -77,7 +77,7 @@ class Sequential(MPSEncoder):
     # -- GPU phases ---------------------------------------------------------
     def _device_layers(self, mps: MPS, num_layers: int):
         work = (mps.state / mps.norm).contiguous()
-        with layer_rounding(mps.num_sites):
+        with layer_rounding(mps.num_sites, num_layers):
             gates, widths, used, amp0, _ = engine.extract_layers(
                 work, num_layers, self.fidelity_threshold)
         return gates, widths, used, amp0

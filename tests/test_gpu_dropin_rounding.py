@@ -1,0 +1,61 @@
+"""The drop-in calls keep one eigensolver's rounding wherever the layers amplify it."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import qmprs_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _gates(sv, chi, **kw):
+    from qmprs_amd.circuit import GateCircuit
+    from qmprs_amd.synthesis.mps_encoding import Sequential
+    circuit = Sequential(GateCircuit).prepare_state(sv, chi, **kw)
+    return np.concatenate([m.reshape(-1) for m, _ in circuit.gates])
+
+
+@pytest.mark.parametrize("n,layers,schedule", [(4, 4, "DallOall"), (6, 6, "DallOall"), (8, 5, "DallOall"),
+                                               (8, 12, "DallOall"), (10, 2, "DallOall")])
+def test_deep_layers_keep_the_one_lane_rounding(gpu, n, layers, schedule):
+    """Bit for bit the circuit of QMX_OPT_TWO_SIDED_JACOBI."""
+    from qmprs_amd import _lib
+    kw = dict(num_layers=layers, num_sweeps=0 if schedule == "DallOall" else 1, schedule=schedule)
+    for seed in range(4):
+        sv = O.random_uniform_state(n, seed)
+        got = _gates(sv, 2 ** n, **kw)
+        with _lib.two_sided_jacobi():
+            want = _gates(sv, 2 ** n, **kw)
+        assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n,layers", [(5, 3), (6, 4), (7, 4), (8, 4)])
+def test_shallow_layers_of_few_qubits(gpu, n, layers):
+    """These take the solver on a wave: within 1e-10, the suite's bar, of the other."""
+    from qmprs_amd import _lib
+    for seed in range(4):
+        sv = O.random_uniform_state(n, seed)
+        got = _gates(sv, 2 ** n, num_layers=layers)
+        with _lib.two_sided_jacobi():
+            want = _gates(sv, 2 ** n, num_layers=layers)
+        print(f"n={n} layers={layers} {np.abs(got - want).max():.1e}")
+        assert np.abs(got - want).max() < 1e-10
+
+
+def test_layer_after_layer(gpu):
+    """MPS.generate_bond_D_unitary_layer, peeled off and called again."""
+    from qmprs_amd import _lib, engine
+    from qmprs_amd.primitives import MPS
+    mps = MPS(O.random_uniform_state(7, 3), bond_dimension=2 ** 7)
+    for _ in range(6):
+        with _lib.two_sided_jacobi():
+            g, w, _ = engine.generate_layer((mps.state / mps.norm).contiguous())
+        want = engine.gates_to_layers(g.cpu().numpy(), w.cpu().numpy(), 1)[0]
+        layer = mps.generate_bond_D_unitary_layer()
+        assert len(layer) == len(want)
+        for (a, b, block), (c, d, other) in zip(layer, want):
+            assert (a, b) == (c, d)
+            assert all(np.array_equal(x.data, y.data) for x, y in zip(block, other))
+        mps.apply_unitary_layer(layer, inverse=True)
+    assert torch.isfinite(torch.view_as_real(mps.state)).all()
