@@ -121,9 +121,11 @@ class Sequential(MPSEncoder):
         """IterDiOi / IterDiOall on the GPU (engine.schedule_layers)."""
         psi = mps._psi.reshape(1, -1).to(torch.complex128).contiguous()
         target = mps.state.reshape(1, -1).to(torch.complex128).contiguous()
-        gates, widths, used, fid = engine.schedule_layers(
-            psi, target, num_layers, num_sweeps, schedule, self.fidelity_threshold,
-            sweep_dtype=sweep_dtype)
+        # (a layer's rounding goes through sweeps into the next layer)
+        with _lib.two_sided_jacobi():
+            gates, widths, used, fid = engine.schedule_layers(
+                psi, target, num_layers, num_sweeps, schedule, self.fidelity_threshold,
+                sweep_dtype=sweep_dtype)
         self.last_info = {"fidelity": float(fid[0].item()), "layers_used": int(used[0].item()),
                           "schedule": schedule}
         layers = engine.gates_to_layers(gates[0].cpu().numpy(), widths[0].cpu().numpy(),

@@ -17,7 +17,8 @@ def _gates(sv, chi, **kw):
 
 
 @pytest.mark.parametrize("n,layers,schedule", [(4, 4, "DallOall"), (6, 6, "DallOall"), (8, 5, "DallOall"),
-                                               (8, 12, "DallOall"), (10, 2, "DallOall")])
+                                               (8, 12, "DallOall"), (10, 2, "DallOall"), (5, 2, "IterDiOi"),
+                                               (9, 3, "IterDiOall")])
 def test_deep_layers_keep_the_one_lane_rounding(gpu, n, layers, schedule):
     """Bit for bit the circuit of QMX_OPT_TWO_SIDED_JACOBI."""
     from qmprs_amd import _lib
