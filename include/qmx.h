@@ -52,10 +52,12 @@ const char* qmx_last_error(const qmx_handle* h);
 /* Tuning options (no reference counterpart).
  * QMX_OPT_SWEEP_MODE: QMX_SWEEP_AUTO (small states, up to N = 12 in complex128
  * and 13 in complex64, each in one block that keeps the state on chip for all
- * sweeps; windowed passes above, else one pass per gate), QMX_SWEEP_STEP (one
- * pass per gate) or QMX_SWEEP_WINDOW (windowed passes; below N = 10, where a
- * tile holds too few rest indices for the pass kernel's four waves, it runs
- * one pass per gate). */
+ * sweeps, but at those two sizes a lone state and batches above two states per
+ * CU in windows, so there a state's rounding depends on its batch; windowed
+ * passes above and for a goal with snapshots), QMX_SWEEP_STEP (one pass per
+ * gate) or QMX_SWEEP_WINDOW (windowed passes).  Where windows are taken below N =
+ * 10, where a tile holds too few rest indices for the pass kernel's four waves,
+ * they are one pass per gate. */
 #define QMX_OPT_SWEEP_MODE 1
 #define QMX_SWEEP_AUTO 0
 #define QMX_SWEEP_STEP 1

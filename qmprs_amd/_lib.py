@@ -285,7 +285,8 @@ def set_sweep_relaxation(omega: float) -> None:
 
 
 def set_sweep_mode(mode: str) -> None:
-    """'auto' (small states in one block each, else windowed passes), 'step'
+    """'auto' (small states in one block each, else windowed passes; at the
+    largest of the small sizes the batch decides, see QMX_SWEEP_AUTO), 'step'
     (one pass per gate) or 'window' (windowed passes; below N = 10 it also
     runs one pass per gate)."""
     h = handle()

@@ -207,6 +207,8 @@ struct ChiLayout {
   int* error;
   int* jrank;        // one-sided Jacobi: Cholesky factors' column counts (nmax > 128: 3 per state)
   double* jdiag;     // and their remaining diagonals, then squared column norms (nmax > 128)
+  // (the two-sided solvers run by option or for a small cutoff, which a workspace
+  // query does not know: every layout holds both)
   double* jlog;      // two-sided LDS Jacobi: rotation log (nmax <= 128)
   int* jstate;
   char* jblock;      // block Jacobi state (nmax > 512)
@@ -265,7 +267,7 @@ struct LayerLayout {
   int* error;
 };
 constexpr int kChain2MaxBlocks = 256;
-constexpr int kJacobiSweeps = 30;   // sweeps for 2r <= 128 (at 2r = 128 one-sided 8 to 10 run, two-sided 16 to 17)
+constexpr int kJacobiSweeps = 30;   // sweeps for 2r <= 128 (at 2r = 128 one-sided 8 to 10 run, two-sided up to 17)
 // sweeps of the block Jacobi (2r > 512): 1 to 34 per bond (16 on average)
 // on the Gram matrices of an N=26 random-MPS state of bond 1024 at chi = 512
 constexpr int kJacobiBlockSweeps = 80;
@@ -1137,7 +1139,10 @@ int sweep_dispatch(qmx_handle* h, int n, int batch, int lmax, const int* layers_
   // At the largest N a block has a CU for itself and is bound by its one CU's
   // work, so a lone state (1.8 ms against 1.65 in windows at N=12) and batches
   // that run in more than two rounds over the CUs (600 complex64 states of
-  // N=13: 10 against 6.4) stay in windows.  Snapshots with a goal keep the
+  // N=13: 10 against 6.4) stay in windows.  (One size below, the crossing lies at
+  // thousands of states: 8 layers and 2 sweeps of 1024 complex128 states of N=11
+  // 4.5 ms against 5.8, of 4096 17.7 against 15.9; of 512 complex64 states of
+  // N=12 3.8 against 3.9, of 1024 7.6 against 5.5.)  Snapshots with a goal keep the
   // windows too: whether one is written depends on the whole batch there.  And
   // so does a goal on a capturing stream: the windows' host check ends such a
   // capture with an error at every size.

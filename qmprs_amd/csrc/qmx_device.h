@@ -515,10 +515,10 @@ QMX_DEV bool complete_two(int i, double2 q0, double2 q1, double2& q2, double2& q
 // 1e-13 of the largest).  With Q R = the two columns left (Gram-Schmidt, two
 // passes), their part of the factor is Q polar(R); the zero columns z_1 < z_2,
 // whose right singular vectors are e_{z_1}, e_{z_2}, take the rule's left
-// completion, the first unit vectors with a residual above 1/2.  Lane 4 i + j of 16 works on
-// row i and on column j of (live, live, zero, zero).  zero: the zero columns
-// (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry (i, j) of
-// the factor.  False where the Jacobi path decides (30600 cycles); 2900
+// completion, the first unit vectors with a residual above 1/2.  Lane 4 i + j of
+// 16 works on row i and on column j of (live, live, zero, zero).  zero: the zero
+// columns (bits), es 2^h: the matrix, fro: its squared norm, near 1; x: entry
+// (i, j) of the factor.  False where the Jacobi path decides (30600 cycles); 2900
 // cycles, against 5300 to 7500 with the whole problem in every lane.
 QMX_DEV bool polar4_two_columns(double2& x, int l, const double2* es, int h, unsigned zero, double fro, double* nuc) {
   const unsigned live = ~zero & 15u;

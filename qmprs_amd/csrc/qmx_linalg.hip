@@ -222,7 +222,8 @@ __global__ __launch_bounds__(512) void jacobi_kernel(double2* a_all, double2* v_
 }
 
 // ------------------------------------------------ LDS-resident Jacobi -------
-// QMX_OPT_TWO_SIDED_JACOBI (the one-sided solver below is the default).
+// QMX_OPT_TWO_SIDED_JACOBI and cutoffs near rounding (the one-sided solver below
+// is the default).
 // For n <= kJacobiLdsMax the upper triangle of A (n (n + 1) / 2 complex128,
 // 132 KiB at n = 128) lives in LDS for a whole sweep: one block per state,
 // the same parallel (circle) ordering and rotations as jacobi_kernel.  Each
@@ -649,7 +650,7 @@ QMX_DEV bool rotate4(Col<NR>& p0, Col<NR>& q0, Col<NR>& p1, Col<NR>& q1, Col<NR>
 // chi = 64: ten matrices of 128 columns and rank 96 to 8) spends 13.2 ms here
 // and 1.3 ms in the Cholesky factors; the two-sided Jacobi it replaces, which
 // kept A's triangle in LDS and logged its rotations for a second kernel that
-// accumulated V, spent 62.7 + 16.1 ms (14 sweeps per matrix).
+// accumulated V, spent 62.7 + 16.1 ms (up to 17 sweeps per matrix).
 constexpr int kOsjMax = 128;
 
 // Pivoted Cholesky factor of one state's Gram matrix (n <= 128): thread (row,

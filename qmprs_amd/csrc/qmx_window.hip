@@ -1006,8 +1006,8 @@ __global__ __launch_bounds__(256) void window_finalize_kernel(WinFinArgs a) {
 // After the gate of site i of the first circuit layer is removed, the sites
 // behind i are in |0>: phi is set to exactly zero where they are not.
 // Bound by the issue of the lead's chain and of the worker that shares its SIMD
-// up to 2^10 complex128 amplitudes (6.1k cycles a step at N = 6, environment
-// 1.7k and polar factor 3.9k, and 6.9k at N = 10), by the workers' updates and
+// up to 2^10 complex128 amplitudes (6.2k cycles a step at N = 6, environment
+// 1.7k and polar factor 4.2k, and 7.0k at N = 10), by the workers' updates and
 // products above (17k at N = 12).  The code of a step has to stay inside the 64
 // KiB instruction cache that two CUs share: paths that are cold cost more to
 // fetch than to run.  One state, 4 layers, 4 sweeps: 0.30 ms against 0.86 gate

@@ -76,7 +76,7 @@ def _truncate(states: torch.Tensor, bond_dimension: int):
     solvers' targets differ becomes 1e-10 to 1e-8 in the gates.  The drop-in
     path therefore keeps one solver's rounding, so that a statevector goes on
     giving the same circuit (24.5 ms for that call with the one-sided solver,
-    47 ms with this one); the batched entry points of ``engine`` take the
+    37 ms with this one); the batched entry points of ``engine`` take the
     faster one."""
     with _lib.two_sided_jacobi():
         psi, target, _ = engine.chi_truncate(states, bond_dimension)

@@ -1,9 +1,9 @@
 """The gate update's polar factor on environments that are hard for it.
 
 States close to a product state give environments whose singular values fall
-like (1, e^2, e^2, e^4): the cofactor inverse, the pivoted inverse and the
-Jacobi path each take some of them, and the layer next to |0..0> gives the
-rank-2 and rank-1 ones.
+like (1, e^2, e^2, e^4): the matrix iteration takes most of them, the Jacobi path
+those that it leaves, and the layer next to |0..0> gives the rank-2 and rank-1
+ones, which have closed forms.
 """
 
 import numpy as np
